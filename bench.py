@@ -242,8 +242,11 @@ def main():
                    (1 << (args.chunk_log2 or 23)))
     nchunks = -(-ncells // chunk_cells)
     tr = profiled_traffic(ncells)
+    # large launches in stiffness order give a cell a lane, the others a group of lanes
+    integrator = ("chem_bdf_lane_kernel" if effective_setup(args, tuning)["order"] == "stiffness"
+                  and min(ncells, chunk_cells) >= LANE_CELLS else "chem_bdf_kernel")
     roofline = {
-        "kernel": "rates_kernel + chem_bdf_kernel (one chemistry step)",
+        "kernel": "rates_kernel + %s (one chemistry step)" % integrator,
         "bound": "fp64_valu",
         "compute": "FP64 vector ALU (the 9x9 LU and mass-action work is per-lane vector code; "
                    "MI355X's FP64 vector and matrix peaks are both 78.6 TFLOP/s)",
@@ -257,11 +260,9 @@ def main():
         "dispatches_per_call": nchunks,
         "algorithmic_flops_per_launch": mean_flops,
         "hbm_boundary_GBs": round(flop_model.BYTES_BOUNDARY * ncells / (mean_ms * 1e-3) / 1e9, 2),
-        "lane_utilisation": profiled_lanes(),
+        "lane_utilisation": profiled_lanes(integrator),
         "lane_utilisation_source": os.path.relpath(SQ_PROFILE, ROOT),
-        "chem_bdf_kernel_resources": kernel_resources(
-            "chem_bdf_kernelILb1ELb0E" if effective_setup(args, tuning)["form"] == "persistent"
-            else "chem_bdf_kernelILb0ELb0E"),
+        "chem_bdf_kernel_resources": kernel_resources(integrator),
     }
 
     # ---- CPU baseline and audit on the sample ---------------------------------------------
@@ -426,7 +427,10 @@ TABLE_BYTES_INTEGRATED = 8 + 1 + 9 * 8 + (9 + 9) * 8 + 8 + 4
 TABLE_BYTES_GATED = 8 + 1 + 9 * 8 + 8 + 4
 HBM_PROFILE = os.path.join(ROOT, "profiles", "chem_step_256cube_hbm_bytes.txt")
 SQ_PROFILE = os.path.join(ROOT, "profiles", "chem_step_256cube_sq_counters.txt")
-RESOURCE_USAGE = os.path.join(ROOT, "nrg_amd", "csrc", "resource_usage.txt")
+RESOURCE_USAGE = {"chem_bdf_kernel": os.path.join(ROOT, "nrg_amd", "csrc", "resource_usage.txt"),
+                  "chem_bdf_lane_kernel": os.path.join(ROOT, "nrg_amd", "csrc",
+                                                       "resource_usage_lane_keromnes.txt")}
+LANE_CELLS = 5 << 17             # cells of a launch from which the one-cell-per-lane integrator runs
 
 
 def profiled_lanes(kernel="chem_bdf_kernel"):
@@ -442,15 +446,16 @@ def profiled_lanes(kernel="chem_bdf_kernel"):
     return None
 
 
-def kernel_resources(name="chem_bdf_kernelILb1ELb0E"):
-    """VGPRs, AGPRs, scratch bytes per lane and occupancy of a kernel, from the
-    compiler's resource report written when the library was built, or None."""
-    if not os.path.exists(RESOURCE_USAGE):
+def kernel_resources(name="chem_bdf_lane_kernel"):
+    """VGPRs, AGPRs, scratch bytes per lane and occupancy of an integrator kernel
+    (finite-difference Jacobian), from the compiler's resource report written
+    when the library was built, or None."""
+    if not os.path.exists(RESOURCE_USAGE[name]):
         return None
     out, cur = {}, False
-    for line in open(RESOURCE_USAGE):
+    for line in open(RESOURCE_USAGE[name]):
         if "Function Name:" in line:
-            cur = name in line
+            cur = name + "ILb0E" in line
             continue
         if cur:
             m = re.search(r"(VGPRs|AGPRs|ScratchSize \[bytes/lane\]|Occupancy \[waves/SIMD\]): (\d+)",
@@ -462,7 +467,7 @@ def kernel_resources(name="chem_bdf_kernelILb1ELb0E"):
     return out or None
 
 
-def profiled_traffic(cells_per_call, kernels=("chem_bdf_kernel", "rates_kernel")):
+def profiled_traffic(cells_per_call, kernels=("chem_bdf_kernel", "chem_bdf_lane_kernel", "rates_kernel")):
     """HBM bytes of one chemistry call from the committed rocprofv3 FETCH_SIZE /
     WRITE_SIZE summary: per-dispatch bytes (copy-calibrated) of the profiled
     run, whose dispatches covered 2^k cells (its command's --chunk-log2 k),
@@ -588,10 +593,9 @@ def uneven_leg(args, mech, tuning, dts=(1e-8, 1e-7, 1e-6), reps=2):
     """The uneven-stiffness workload: n^3 cells, 5 % of them fresh mixture in the
     1000-1300 K ignition window (tens to hundreds of steps each), the rest burnt
     or cold (a few steps).  For each dt, the chemistry step (rates_kernel +
-    chem_bdf_kernel, device time from HIP events) in two launch forms from the
-    same state: the persistent work queue in a HIP graph with stiffness order and
-    the main leg's autotuned queue set-up, and the plain one-cell-per-lane launch
-    in natural order.  Both give the same outputs bit for bit (checked here)."""
+    chem_bdf_kernel, device time from HIP events) in two set-ups from the
+    same state: stiffness order in a HIP graph with the main leg's autotuned queue
+    set-up (a cell to a lane), and natural order (a cell to a group of lanes).  Both give the same outputs bit for bit (checked here)."""
     import numpy as np
     import torch
 
@@ -615,8 +619,8 @@ def uneven_leg(args, mech, tuning, dts=(1e-8, 1e-7, 1e-6), reps=2):
     plain = capi.default_opts(form=capi.NRG_FORM_PLAIN, cell_order=capi.NRG_ORDER_NATURAL,
                               use_graph=0, chunk_log2=(n - 1).bit_length() if n > 1 else 16)
     res = {"cells": n, "window_frac": 0.05, "reps": reps, "per_dt": []}
-    engines = {"persistent_graph_queue": ChemistryStep(mech, queued),
-               "one_cell_per_lane": ChemistryStep(mech, plain)}
+    engines = {"stiffness_order_graph": ChemistryStep(mech, queued),
+               "natural_order": ChemistryStep(mech, plain)}
     try:
         for dt in dts:
             row = {"dt": dt}
@@ -639,8 +643,8 @@ def uneven_leg(args, mech, tuning, dts=(1e-8, 1e-7, 1e-6), reps=2):
                     "integrated_cells": int(r.cells_integrated),
                     "nfe_per_integrated_cell": round(r.nfe_sum / max(1, r.cells_integrated), 2),
                     "nstep_max": int(r.nstep_max)}
-            row["queue_speedup"] = round(row["one_cell_per_lane"]["kernel_ms"] /
-                                         row["persistent_graph_queue"]["kernel_ms"], 3)
+            row["queue_speedup"] = round(row["natural_order"]["kernel_ms"] /
+                                         row["stiffness_order_graph"]["kernel_ms"], 3)
             row["identical_outputs"] = bool(all(torch.equal(a, c) for a, c in zip(*outs)))
             res["per_dt"].append(row)
     finally:

@@ -79,10 +79,14 @@ enum {
   NRG_ORDER_STIFFNESS = 1
 };
 
-/* Launch form of the per-cell integrator (same arithmetic, same results). */
+/*
+ * Launch form of the per-cell integrator.  Both forms run the same resident
+ * grid over the work queue (same arithmetic, same results, same time): a cell to
+ * a group of lanes, or, in large grids in stiffness order, a cell to a lane.
+ */
 enum {
-  NRG_FORM_PLAIN = 0,          /* one cell per lane, one launch over all inner cells          */
-  NRG_FORM_PERSISTENT = 1      /* resident grid; lanes refill from a work queue as cells end  */
+  NRG_FORM_PLAIN = 0,
+  NRG_FORM_PERSISTENT = 1
 };
 
 /*
@@ -130,7 +134,7 @@ typedef struct nrg_chem_opts {
   int32_t form;                /* NRG_FORM_*                                                   */
   int32_t jac_batch_pct;       /* a wave runs a batched Jacobian when at least this percentage
                                   of its pending lanes wait for one (1..100; 0 = default 50)   */
-  int32_t waves_per_cu;        /* persistent form: resident waves per CU (0 = occupancy limit) */
+  int32_t waves_per_cu;        /* resident waves per CU (0 = occupancy limit)                  */
   int32_t cell_order;          /* NRG_ORDER_*: order in which the queue hands out cells        */
   int32_t use_graph;           /* 1: capture the step's launches in a HIP graph and replay it
                                   while the arguments stay the same (same results)             */
@@ -141,9 +145,10 @@ typedef struct nrg_chem_opts {
                                   error test until this percentage of the wave's lanes that
                                   are stepping is there (100: the wave's cells take their
                                   steps' error tests together; 0: no waiting).  Same results. */
-  int32_t refill_min_idle;     /* persistent form: a wave hands new cells to its idle lanes once
-                                  this many of its 64 lanes are idle, or all are (1..64; 0 =
-                                  default 63: the wave's cells start together).  Same results. */
+  int32_t refill_min_idle;     /* a wave hands new cells to its idle lanes once this many of its
+                                  64 lanes are idle, or all are (1..64; 0 = default: 63 in
+                                  stiffness order, where a wave's cells cost alike and start
+                                  together, 32 in natural order).  Same results.              */
 } nrg_chem_opts;
 
 /*
@@ -289,8 +294,8 @@ int nrg_energy_from_temperature_dev(nrg_chem_t *h, const nrg_grid *grid,
 
 /*
  * Autotuner of the batched form.  A cell is one lane and a workgroup one
- * wave (64 cells), so what is tuned is how the queue feeds the waves: launch
- * form, cell order, the error-test gathering, the batched-Jacobian threshold,
+ * wave (64 cells), so what is tuned is how the queue feeds the waves: cell
+ * order, the error-test gathering, the batched-Jacobian threshold,
  * the refill threshold, resident waves per CU and the queue chunk size.  Starting from the handle's current set-up it tries
  * one change at a time (greedy), each as a full chemistry step on the given
  * fields timed with HIP events, keeps the fastest and leaves it in the

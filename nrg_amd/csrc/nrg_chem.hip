@@ -13,12 +13,11 @@
 // (nrg_api.cpp) as a table (topo_api.h); nrg_chem_create picks the table whose
 // topology the mechanism has.
 //
-// NRG_PART splits a build into two objects: 1 = everything but the
-// integrator kernel's body, 2 = the integrator kernel alone (so that it can be
-// compiled with scheduling options of its own); 0 (default) = both in one.
-// With NRG_PART 2, NRG_BDF_JAC selects the kernel's instantiations: 1 = those
-// with the finite-difference Jacobian, 2 = those with the analytic one, unset
-// = all four.
+// NRG_PART splits a build into objects: 1 = everything but the integrator
+// kernels' bodies, 2 = the lane-group integrator alone, 3 = the one-cell-per-lane
+// integrator alone (so that they can be compiled with options of their own);
+// 0 (default) = all in one.  With NRG_PART 2, NRG_BDF_JAC selects the kernel's
+// instantiation: 1 = finite-difference Jacobian, 2 = analytic, unset = both.
 #ifndef NRG_PART
 #define NRG_PART 0
 #endif
@@ -43,6 +42,8 @@
 #include "../../include/nrg_chem.h"
 #include "../../include/nrg_low_mach.h"
 #include "../../include/nrg_surrogate.h"
+#include "bdf_group.h"
+#include "bdf_lane.h"
 #include "chem_device.h"
 #include "mlp_internal.h"
 #include "nrg_common.h"
@@ -148,6 +149,7 @@ struct StepArgs {
   long long base, nchunk;               // this launch covers queue positions [base, base+nchunk)
   const int32_t *list;                  // NULL: position t is inner cell t; else inner cell list[t]
   int32_t *hist;                        // optional: NSTEP of each inner cell (0 if gated), for ordering
+  int cpw;                              // cells a wave of the integrator holds at a time
 };
 
 // Inner cell (inner-loop order) at position base + t of the launch's queue.
@@ -187,30 +189,21 @@ NRG_DI void stage_mech(MechCoef &dst, const MechCoef *src)
   __syncthreads();
 }
 
-NRG_DI void stage_bdf(BdfCoef &dst, const MechCoef *src)
+NRG_DI void stage_bdf(BdfCoef &dst, const MechCoef *src, double sqrtn)
 {
   for (int i = threadIdx.x; i < MAXORD * (MAXORD + 1); i += blockDim.x)
     (&dst.el[0][0])[i] = (&src->el[0][0])[i];
-  for (int i = threadIdx.x; i < MAXORD * 3; i += blockDim.x) (&dst.tq[0][0])[i] = (&src->tq[0][0])[i];
+  for (int i = threadIdx.x; i < 3 * MAXORD; i += blockDim.x) {
+    const double d = src->tq[i % MAXORD][i / MAXORD] * sqrtn;
+    (&dst.den[0][0])[i] = d;
+    (&dst.rden[0][0])[i] = recip(d);
+  }
+  if (threadIdx.x < 8) dst.inv[threadIdx.x] = 1.0 / (double)(int)threadIdx.x;
   for (int i = threadIdx.x; i < S; i += blockDim.x) {
     dst.W[i] = src->W[i];
     dst.h_ref[i] = src->h_ref[i];
   }
   __syncthreads();
-}
-
-NRG_DI unsigned long long wave_sum_u64(unsigned long long v)
-{
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-NRG_DI int wave_max_i32(int v)
-{
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-  return v;
 }
 
 // accumulator slots
@@ -222,74 +215,66 @@ enum { ACC_INTEG = 0, ACC_NSTEP, ACC_NFE, ACC_NJE, ACC_NCORR, ACC_NATT, ACC_NSTE
 
 // Zero the work accumulators and the queue head (a kernel, so the launch
 // sequence can be captured in a graph without memset nodes).
-#if NRG_PART != 2
+#if NRG_PART < 2
 __global__ void reset_kernel(unsigned long long *acc, int n)
 {
   if ((int)threadIdx.x < n) acc[threadIdx.x] = 0ull;
 }
 #endif
 
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(3))) double lds_double;
-
-// The integrator keeps the whole cell record in LDS when four single-wave
-// blocks still fit a CU's 160 KiB (every mechanism up to ~37 record pairs);
-// a larger mechanism keeps the rate constants and [M] there and reads the
-// initial concentrations and the gate flag from HBM.
-constexpr size_t LDS_PER_CU = 160 * 1024;
-constexpr bool REC_C_IN_LDS = 4 * ((size_t)REC_PAIRS * 16 * WAVE + sizeof(BdfCoef)) <= LDS_PER_CU;
-constexpr int REC_LDS_PAIRS = REC_C_IN_LDS ? REC_PAIRS : REC_C;
-
-// Load one cell and set it up (chemical_kinetics_solver.f90:228-265).  The
-// cell record of position t (rates_kernel) goes from HBM straight into the
-// lane's LDS slots (recl: the block's record array, kl: this lane's view of
-// it): one round trip, no registers in between.  Returns false for a gated
-// cell, whose outputs are written here (:341-346).
-NRG_DI bool start_cell(const StepArgs &a, long long t, long long q, long long &off, Cell &c,
-                       lds_double *recl, const double *kl)
+// Load one cell and set it up (chemical_kinetics_solver.f90:228-265): the
+// group's lanes copy the cell record of position t (rates_kernel) from HBM to
+// the cell's slice of LDS, all loads in one round trip.  Returns false for a
+// gated cell, whose outputs are written here (:341-346).
+NRG_DI bool start_cell(const StepArgs &a, long long t, Cell &c, const Lane &ln)
 {
   const double *src = a.rates + 2 * t;
+  constexpr int K = (REC_PAIRS + G - 1) / G;
+  double2 v[K];
 #pragma unroll
-  for (int p = 0; p < REC_LDS_PAIRS; ++p)
-    __builtin_amdgcn_global_load_lds((const void *)(src + 2 * (long long)p * a.nchunk),
-                                     (lds_void *)(recl + 2 * p * WAVE), 16, 0, 0);   // M0: LDS address
-  double cs[S + 1];
-  if (!REC_C_IN_LDS) {
-#pragma unroll
-    for (int s = 0; s <= S; ++s) cs[s] = src[rec_slot(REC_C, s, a.nchunk)];
+  for (int k = 0; k < K; ++k) {
+    const int p = k * G + ln.sub;
+    if ((k + 1) * G <= REC_PAIRS || p < REC_PAIRS)
+      v[k] = *reinterpret_cast<const double2 *>(src + 2 * (long long)p * a.nchunk);
   }
-  off = cell_offset_wide(a.g, q);
-  // a direct load's data is in LDS once vmcnt has counted it
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if (REC_C_IN_LDS) {
+  const long long q = cell_of(a, t);
+  const long long off = cell_offset(a.g, q);
+  wave_sync();
 #pragma unroll
-    for (int s = 0; s <= S; ++s) cs[s] = rec_c(kl, s);
-  }
-  if (cs[REC_FLAG] == 0.0) {
-#pragma unroll
-    for (int s = 0; s < S; ++s) a.Yp[s][off] = 0.0;
-    a.Efp[off] = 0.0;
-    if (a.status) a.status[off] = NRG_CELL_GATED;
-    if (a.nstep) {
-      a.nstep[q] = 0;
-      a.nfe[q] = 0;
-      a.nje[q] = 0;
+  for (int k = 0; k < K; ++k) {
+    const int p = k * G + ln.sub;
+    if ((k + 1) * G <= REC_PAIRS || p < REC_PAIRS) {
+      *slot(ln, 2 * p) = v[k].x;
+      *slot(ln, 2 * p + 1) = v[k].y;
     }
-    if (a.hist) a.hist[q] = 0;
+  }
+  if (ln.sub == 0) {
+    *slot(ln, CCELL) = __longlong_as_double(q);
+    *slot(ln, CCELL + 1) = __longlong_as_double(off);
+  }
+  wave_sync();
+  if (*slot(ln, 2 * REC_C + REC_FLAG) == 0.0) {
+#pragma unroll
+    for (int s0 = 0; s0 < S; s0 += G)
+      if (s0 + ln.sub < S) a.Yp[s0 + ln.sub][off] = 0.0;
+    if (ln.sub == 0) {
+      a.Efp[off] = 0.0;
+      if (a.status) a.status[off] = NRG_CELL_GATED;
+      if (a.nstep) {
+        a.nstep[q] = 0;
+        a.nfe[q] = 0;
+        a.nje[q] = 0;
+      }
+      if (a.hist) a.hist[q] = 0;
+    }
     return false;
   }
-#pragma unroll
-  for (int s = 0; s < S; ++s) {
-    if (kSp.act[s] >= 0)
-      c.y[kSp.act[s]] = cs[s];
-    else
-      c.yi[kSp.islot[s]] = cs[s];
-  }
+  c.y = holds(ln) ? *slot(ln, 2 * REC_C + slot_species(ln.sub)) : 0.0;
   bdf_init(c, a.dt, a.k);
   return true;
 }
 
-#if NRG_PART != 2
+#if NRG_PART < 2
 // Cell records of the chunk's positions: the gate (:224-227), and for every
 // integrated cell its concentrations (:228-233), rate constants and [M]
 // (:235-252, 360-493), kept apart from the integrator so its ~80
@@ -347,28 +332,245 @@ __global__ void __launch_bounds__(256) rates_kernel(StepArgs a)
 
 #endif
 
-// Output assembly (:318-340) once the cell's DDRIV3 has returned; returns the
-// cell's NRG_CELL_* status.
-NRG_DI int finish_cell(const StepArgs &a, const BdfCoef &mc, long long q, long long off,
-                       const Cell &c, const double *kl)
+// Output assembly (:318-340) once the cell's DDRIV3 has returned, a species to
+// a lane, and the cell's work and status counts (tally, in LDS).
+NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, const Cell &c, const Lane &ln,
+                        unsigned long long *tally)
 {
-  const double rho = REC_C_IN_LDS ? 0.0 : a.rho[off];
+  wave_sync();
+  if (holds(ln)) *own(ln, CZ) = c.y;
+  wave_sync();
+  const long long q = __double_as_longlong(*slot(ln, CCELL));
+  const long long off = __double_as_longlong(*slot(ln, CCELL + 1));
+  const double rdt = recip(a.dt);
+#pragma unroll
+  for (int s0 = 0; s0 < S; s0 += G) {
+    const int s = s0 + ln.sub;
+    if (s < S) {
+      // the initial concentration as rates_kernel recorded it
+      const double cin = *slot(ln, 2 * REC_C + s);
+      const double ys = inert_species(s) ? cin : *slot(ln, CZ + active_slot(s));
+      const double dc = ys - cin;
+      a.Yp[s][off] = div_by(dc * mc.W[s], a.dt, rdt);
+      a.Yp2[s][off] = dc;
+      *slot(ln, CX + s) = div_by(mc.h_ref[s] * dc, a.dt, rdt);
+    }
+  }
+  wave_sync();
+  const int out = c.pc & 15;
+  const int status = (out == OUT_OK) ? NRG_CELL_OK
+                   : (out == OUT_MXSTEP || out == OUT_EPS) ? NRG_CELL_MXSTEP
+                   : (out == OUT_STEP_ZERO) ? NRG_CELL_STEP_ZERO
+                   : (out == OUT_REPEATED_FAIL) ? NRG_CELL_REPEATED_FAIL
+                   : NRG_CELL_SINGULAR;
+  if (ln.sub == 0) {
+    double ef = 0.0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) ef = ef - *slot(ln, CX + s);
+    a.Efp[off] = ef;
+    if (a.status) a.status[off] = status;
+    if (a.nstep) a.nstep[q] = c.nstep;
+    if (a.hist) a.hist[q] = c.nstep;
+    atomicAdd(&tally[ACC_STATUS0 + status], 1ull);
+  }
+  if (a.nstep && ln.sub == WORK_NFE) a.nfe[q] = c.work;
+  if (a.nstep && ln.sub == WORK_NJE) a.nje[q] = c.work;
+  // the work counters, each added by the lane that holds it, and the others
+  static_assert(ACC_NJE == ACC_NFE + WORK_NJE && ACC_NCORR == ACC_NFE + WORK_NCORR &&
+                ACC_NATT == ACC_NFE + WORK_NATT && WORK_NFE == 0 && G >= 4, "a counter to a lane");
+  const int nfe = __shfl(c.work, ln.gshift + WORK_NFE, WAVE);
+  if (ln.sub < 4) {
+    atomicAdd(&tally[ACC_NFE + ln.sub], (unsigned long long)c.work);
+    if (ln.sub < 2)
+      atomicAdd(&tally[ln.sub == 0 ? ACC_INTEG : ACC_NSTEP], ln.sub == 0 ? 1ull : (unsigned long long)c.nstep);
+    else
+      atomicMax(&tally[ln.sub == 2 ? ACC_NSTEP_MAX : ACC_NFE_MAX], (unsigned long long)(ln.sub == 2 ? c.nstep : nfe));
+  }
+  wave_sync();
+}
+
+// A wave's counts into the launch's: one atomic per counter.
+NRG_DI void flush_tally(unsigned long long *acc, const unsigned long long *tally, int lane)
+{
+  wave_sync();
+  if (lane < ACC_QUEUE0 && tally[lane]) {
+    if (lane == ACC_NSTEP_MAX || lane == ACC_NFE_MAX)
+      atomicMax(&acc[lane], tally[lane]);
+    else
+      atomicAdd(&acc[lane], tally[lane]);
+  }
+}
+
+// One chemistry step (solve_chemical_kinetics, :224-346), a cell to a group of
+// G lanes (bdf_group.h).  A resident grid of one-wave blocks; each wave holds up
+// to a.cpw cells and takes the next unclaimed ones of the chunk's queue (one
+// atomic per wave per refill) once k.refill_idle of its 64 lanes (in proportion
+// where it holds fewer cells) are idle, or all are.
+// Each pass evaluates f for the cells that asked for it and, when at least
+// jac_pct % of the pending cells wait for a Jacobian or nothing else is
+// pending, forms and factors the waiting cells' iteration matrices.
+//
+// Idle lanes that trigger a refill.  In stiffness order a wave's cells cost
+// alike and are best started together (256 x 4096 flame cells: 17.8 ms, 22.4
+// with 32, 26.0 with 8); in natural order a long cell would keep the others'
+// lanes idle (262,144 cells of an igniting mixture: 12.1 ms with 64, 9.0 with
+// 32, 8.0 with 8, but flame fronts and hot kernels want more: 22.0, 23.5, 24.2
+// and 6.7, 6.4, 9.1).
+constexpr int REFILL_IDLE_ORDERED = 63, REFILL_IDLE_NATURAL = 32;
+
+// Resident waves per SIMD the register budget is sized for (168 registers at
+// three, 256 at two): a group of 8 lanes needs 166, one of 16 up to 213 without
+// spills, and spilling costs more than the third wave gives.
+constexpr int BDF_WAVES = G == 8 ? 3 : 2;
+template <bool ANALYTIC>
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(BDF_WAVES)))
+chem_bdf_kernel(StepArgs a)
+#if NRG_PART == 1 || NRG_PART == 3
+;   // defined in the integrator part of this build
+extern template __global__ void chem_bdf_kernel<false>(StepArgs);
+extern template __global__ void chem_bdf_kernel<true>(StepArgs);
+#else
+{
+  __shared__ BdfCoef mc;
+  __shared__ __align__(16) double cells[CPW * CELL_DOUBLES];   // the cells' slices
+  __shared__ __align__(16) unsigned table[G * TABW];
+  __shared__ __align__(16) unsigned jtable[ANALYTIC ? G * JTABW : 4];
+  __shared__ unsigned long long tally[ACC_QUEUE0];             // the wave's share of acc
+  const int lane = threadIdx.x;
+  if (lane < ACC_QUEUE0) tally[lane] = 0ull;
+  stage_bdf(mc, a.mech, a.k.sqrtn);
+  const GroupConst gc = {a.k.sqrtn, uniform(recip(a.k.sqrtn)), a.k.eps, uniform(recip(a.k.eps))};
+  Lane ln;
+  group_init(ln, (lds_double *)cells, (lds_word *)table, ANALYTIC ? (lds_word *)jtable : nullptr, lane);
+  Cell c;
+  c.pc = PC_IDLE;
+  const int grp = lane / G;
+  bool exhausted = grp >= a.cpw;
+  for (;;) {
+    bool need = c.pc >= PC_DONE && !exhausted;
+    if (wave_any(c.pc < PC_DONE) && __popcll(__ballot(need ? 1 : 0)) * CPW < a.k.refill_idle * a.cpw)
+      need = false;
+    while (wave_any(need)) {
+      const unsigned long long mask = __ballot(need ? 1 : 0);
+      const int leader = __ffsll((long long)mask) - 1;
+      unsigned long long base = 0;
+      if (lane == leader) base = atomicAdd(a.queue, (unsigned long long)(__popcll(mask) / G));
+      base = __shfl(base, leader, WAVE);
+      if (need) {
+        const long long t =
+            (long long)(base + (unsigned long long)(__popcll(mask & ((1ull << ln.gshift) - 1ull)) / G));
+        if (t >= a.nchunk)
+          exhausted = true;
+        else if (!start_cell(a, t, c, ln) && ln.sub == 0)
+          atomicAdd(&tally[ACC_STATUS0 + NRG_CELL_GATED], 1ull);
+      }
+      need = need && c.pc >= PC_DONE && !exhausted;
+    }
+    if (!wave_any(c.pc < PC_DONE)) break;
+    const bool wantj = (c.pc & PC_WAIT_JAC) != 0, wantf = (c.pc & PC_WAIT_F) != 0;
+    const int nj = __popcll(__ballot(wantj ? 1 : 0));
+    const int nf = __popcll(__ballot(wantf ? 1 : 0));
+    const bool run_jac = nj > 0 && (nf == 0 || nj * 100 >= a.jac_pct * (nj + nf));
+    if (wantf) {
+      c.save2 = rhs_group(ln, c.y);
+      c.pc &= 15;
+    }
+    if (run_jac && wantj) {
+      if (ANALYTIC)
+        jac_exact(ln, c, mc);
+      else
+        jac_fd(ln, c, a.k, mc);
+      c.pc &= 15;
+    }
+    if (c.pc < PC_WAIT_F) advance(ln, c, a.dt, a.k, gc, mc);
+    if ((c.pc & PC_DONE) && c.pc != PC_IDLE) {
+      finish_cell(a, mc, c, ln, tally);
+      c.pc = PC_IDLE;
+    }
+  }
+  flush_tally(a.acc, tally, lane);
+}
+#endif
+
+// ---------------------------------------------------------------------------
+// The same step with one cell per lane (bdf_lane.h), for large grids of the
+// topologies whose state fits the register file.
+// ---------------------------------------------------------------------------
+constexpr bool LANE_KERNEL = SA <= 10;
+constexpr int LANE_WAVES_PER_CU = 4;   // one to a SIMD: it takes the whole register file
+#if NRG_PART == 0 || NRG_PART == 3
+typedef __attribute__((address_space(3))) void lds_void;
+
+// Load one cell and set it up (chemical_kinetics_solver.f90:228-265).  The
+// cell record of position t (rates_kernel) goes from HBM straight into the
+// lane's LDS slots (recl: the block's record array, kl: this lane's view of
+// it): one round trip, no registers in between.  Returns false for a gated
+// cell, whose outputs are written here (:341-346).
+NRG_DI bool start_cell(const StepArgs &a, long long t, long long q, long long &off, lane::Cell &c,
+                       lds_double *recl, const double *kl)
+{
+  const double *src = a.rates + 2 * t;
+#pragma unroll
+  for (int p = 0; p < REC_PAIRS; ++p)
+    __builtin_amdgcn_global_load_lds((const void *)(src + 2 * (long long)p * a.nchunk),
+                                     (lds_void *)(recl + 2 * p * WAVE), 16, 0, 0);   // M0: LDS address
+  off = cell_offset_wide(a.g, q);
+  // a direct load's data is in LDS once vmcnt has counted it
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (lane::rec_c(kl, REC_FLAG) == 0.0) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) a.Yp[s][off] = 0.0;
+    a.Efp[off] = 0.0;
+    if (a.status) a.status[off] = NRG_CELL_GATED;
+    if (a.nstep) {
+      a.nstep[q] = 0;
+      a.nfe[q] = 0;
+      a.nje[q] = 0;
+    }
+    if (a.hist) a.hist[q] = 0;
+    return false;
+  }
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    if (kSp.act[s] >= 0)
+      c.y[kSp.act[s]] = lane::rec_c(kl, s);
+    else
+      c.yi[kSp.islot[s]] = lane::rec_c(kl, s);
+  }
+  lane::bdf_init(c, a.dt, a.k);
+  return true;
+}
+
+// A lane's counts of its finished cells.  (In registers: cells of equal cost
+// finish together, and 64 atomics to one LDS word take as many turns; 2.1M
+// cells with hot kernels 5.44 ms so, 4.85 here.)
+struct LaneTally {
+  unsigned integrated = 0, gated = 0;
+  unsigned long long nstep = 0, nfe = 0, nje = 0, ncorr = 0, natt = 0;
+  int nstep_max = 0, nfe_max = 0;
+};
+
+// Output assembly (:318-340) once the cell's DDRIV3 has returned, and its
+// counts (a failure's straight into the wave's).
+NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, long long q, long long off,
+                        const lane::Cell &c, const double *kl, LaneTally &tl, unsigned long long *tally)
+{
+  const double rdt = recip(a.dt);
   double ef = 0.0;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
-    // the initial concentration as rates_kernel recorded it (the same expression)
-    const double cin = REC_C_IN_LDS ? rec_c(kl, s) : (a.Y[s][off] * rho) / mc.W[s];
+    const double cin = lane::rec_c(kl, s);   // the initial concentration as rates_kernel recorded it
     const double ys = (kSp.act[s] >= 0) ? c.y[kSp.act[s]] : c.yi[kSp.islot[s]];
     const double dc = ys - cin;
-    a.Yp[s][off] = (dc * mc.W[s]) / a.dt;
+    a.Yp[s][off] = div_by(dc * mc.W[s], a.dt, rdt);
     a.Yp2[s][off] = dc;
-    ef = ef - (mc.h_ref[s] * dc) / a.dt;
+    ef = ef - div_by(mc.h_ref[s] * dc, a.dt, rdt);
   }
   a.Efp[off] = ef;
-  const int status = (c.outcome == OUT_OK) ? NRG_CELL_OK
-                   : (c.outcome == OUT_MXSTEP || c.outcome == OUT_EPS) ? NRG_CELL_MXSTEP
-                   : (c.outcome == OUT_STEP_ZERO) ? NRG_CELL_STEP_ZERO
-                   : (c.outcome == OUT_REPEATED_FAIL) ? NRG_CELL_REPEATED_FAIL
+  const int status = (c.outcome == lane::OUT_OK) ? NRG_CELL_OK
+                   : (c.outcome == lane::OUT_MXSTEP || c.outcome == lane::OUT_EPS) ? NRG_CELL_MXSTEP
+                   : (c.outcome == lane::OUT_STEP_ZERO) ? NRG_CELL_STEP_ZERO
+                   : (c.outcome == lane::OUT_REPEATED_FAIL) ? NRG_CELL_REPEATED_FAIL
                    : NRG_CELL_SINGULAR;
   if (a.status) a.status[off] = status;
   if (a.nstep) {
@@ -377,169 +579,125 @@ NRG_DI int finish_cell(const StepArgs &a, const BdfCoef &mc, long long q, long l
     a.nje[q] = c.nje;
   }
   if (a.hist) a.hist[q] = c.nstep;
-  return status;
+  if (status != NRG_CELL_OK) atomicAdd(&tally[ACC_STATUS0 + status], 1ull);
+  tl.integrated += 1;
+  tl.nstep += c.nstep;
+  tl.nfe += c.nfe;
+  tl.nje += c.nje;
+  tl.ncorr += c.ncorr;
+  tl.natt += c.natt;
+  tl.nstep_max = max(tl.nstep_max, c.nstep);
+  tl.nfe_max = max(tl.nfe_max, c.nfe);
 }
-
-// Per-lane work and status counts, reduced once per wave at the end.
-struct Tally {
-  unsigned long long cnt[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  unsigned long long work[6] = {0, 0, 0, 0, 0, 0};
-  int mx_step = 0, mx_fe = 0;
-
-  NRG_DI void integrated(const Cell &c, int status)
-  {
-#pragma unroll
-    for (int st = 0; st < 8; ++st) cnt[st] += (status == st) ? 1ull : 0ull;
-    work[0] += 1;
-    work[1] += c.nstep;
-    work[2] += c.nfe;
-    work[3] += c.nje;
-    work[4] += c.ncorr;
-    work[5] += c.natt;
-    mx_step = max(mx_step, c.nstep);
-    mx_fe = max(mx_fe, c.nfe);
-  }
-
-  NRG_DI void flush(unsigned long long *acc, int lane)
-  {
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-      const unsigned long long w = wave_sum_u64(work[i]);
-      if (lane == 0 && w) atomicAdd(&acc[ACC_INTEG + i], w);
-    }
-    const int ms = wave_max_i32(mx_step);
-    const int mf = wave_max_i32(mx_fe);
-    if (lane == 0) {
-      atomicMax(&acc[ACC_NSTEP_MAX], (unsigned long long)ms);
-      atomicMax(&acc[ACC_NFE_MAX], (unsigned long long)mf);
-    }
-#pragma unroll
-    for (int st = 0; st < 6; ++st) {
-      const unsigned long long w = wave_sum_u64(cnt[st]);
-      if (lane == 0 && w) atomicAdd(&acc[ACC_STATUS0 + st], w);
-    }
-  }
-};
-
-// One chemistry step (solve_chemical_kinetics, :224-346), one cell per lane.
-// PERSISTENT = false: lane i of block b owns inner cell 64*b + i (the plain
-//   launch).  PERSISTENT = true: a resident grid; once k.refill_idle lanes
-//   of a wave have finished (or all have), they take the next unclaimed cells
-//   from a.queue (one atomic per wave per refill).
-// Each iteration either evaluates f for the lanes that asked, or -- when at
-// least jac_pct % of the pending lanes wait for a Jacobian, or nothing else is
-// pending -- runs one batched FD Jacobian + LU for the waiting lanes.
-constexpr int REFILL_MIN_IDLE_DEFAULT = 63;   // measured: 48 -> 41.9, 56 -> 40.5, 63 -> 40.0 ms per 256^3 step
-
-#ifndef NRG_BDF_WAVES_PER_EU
-#define NRG_BDF_WAVES_PER_EU 1   // resident waves per SIMD the register budget is sized for
 #endif
-template <bool PERSISTENT, bool ANALYTIC>
-__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(NRG_BDF_WAVES_PER_EU)))
-chem_bdf_kernel(StepArgs a)
-#if NRG_PART == 1
-;   // defined in the integrator part of this build
-extern template __global__ void chem_bdf_kernel<false, false>(StepArgs);
-extern template __global__ void chem_bdf_kernel<false, true>(StepArgs);
-extern template __global__ void chem_bdf_kernel<true, false>(StepArgs);
-extern template __global__ void chem_bdf_kernel<true, true>(StepArgs);
+
+// A resident grid of one-wave blocks; once k.refill_idle lanes of a wave have
+// finished (or all have), they take the next unclaimed cells from a.queue (one
+// atomic per wave per refill).  Each pass either evaluates f for the lanes that
+// asked, or -- when at least jac_pct % of the pending lanes wait for a Jacobian,
+// or nothing else is pending -- forms and factors the iteration matrices of the
+// waiting lanes.
+template <bool ANALYTIC>
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(1)))
+chem_bdf_lane_kernel(StepArgs a)
+#if NRG_PART == 1 || NRG_PART == 2
+;   // defined in a part of its own
+extern template __global__ void chem_bdf_lane_kernel<false>(StepArgs);
+extern template __global__ void chem_bdf_lane_kernel<true>(StepArgs);
 #else
 {
   __shared__ BdfCoef mc;
-  __shared__ __align__(16) double recl[2 * REC_LDS_PAIRS * WAVE];   // the lanes' cell records
-  stage_bdf(mc, a.mech);
+  __shared__ __align__(16) double recl[2 * REC_PAIRS * WAVE];   // the lanes' cell records
+  __shared__ unsigned long long tally[ACC_QUEUE0];              // the wave's share of acc
+  static_assert(4 * (sizeof(BdfCoef) + sizeof recl + sizeof tally) <= 160 * 1024, "four blocks to a CU");
   const int lane = threadIdx.x;
+  if (lane < ACC_QUEUE0) tally[lane] = 0ull;
+  stage_bdf(mc, a.mech, a.k.sqrtn);
+  const GroupConst gc = {a.k.sqrtn, uniform(recip(a.k.sqrtn)), a.k.eps, uniform(recip(a.k.eps))};
   const double *kl = recl + 2 * lane;
   lds_double *recl_lds = (lds_double *)recl;   // the array's LDS address (direct loads' M0)
-  Cell c;
-  c.req = REQ_DONE;
+  lane::Cell c;
+  c.req = lane::REQ_DONE;
   long long q = -1, off = 0;
+  LaneTally tl;
   bool have = false, exhausted = false;
-  // The persistent form tallies each finished cell as it goes; a lane of the
-  // plain form owns one cell, whose counts are read from its state at the end
-  // (keeping the tally out of the registers live across the loop).
-  Tally tl;
-  bool gated = false;
-  int status = 0;
-  if (!PERSISTENT) {
-    const long long t = (long long)blockIdx.x * WAVE + lane;
-    if (t < a.nchunk) {
-      q = cell_of(a, t);
-      have = start_cell(a, t, q, off, c, recl_lds, kl);
-      gated = !have;
-    }
-  }
   for (;;) {
-    if (PERSISTENT) {
-      // refill in batches: new cells start together, so the wave's lanes stay
-      // near the same stage (refilling every pass measured 30 % slower)
-      bool need = !have && !exhausted;
-      if (wave_any(have) && __popcll(__ballot(need ? 1 : 0)) < a.k.refill_idle) need = false;
-      while (wave_any(need)) {
-        const unsigned long long mask = __ballot(need ? 1 : 0);
-        const int leader = __ffsll((long long)mask) - 1;
-        unsigned long long base = 0;
-        if (lane == leader) base = atomicAdd(a.queue, (unsigned long long)__popcll(mask));
-        base = __shfl(base, leader, WAVE);
-        if (need) {
-          const long long t =
-              (long long)(base + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull)));
-          if (t >= a.nchunk) {
-            exhausted = true;
-          } else {
-            q = cell_of(a, t);
-            have = start_cell(a, t, q, off, c, recl_lds, kl);
-            if (!have) tl.cnt[NRG_CELL_GATED]++;
-          }
+    // refill in batches: new cells start together, so the wave's lanes stay
+    // near the same stage (refilling every pass measured 30 % slower)
+    bool need = !have && !exhausted;
+    if (wave_any(have) && __popcll(__ballot(need ? 1 : 0)) < a.k.refill_idle) need = false;
+    while (wave_any(need)) {
+      const unsigned long long mask = __ballot(need ? 1 : 0);
+      const int leader = __ffsll((long long)mask) - 1;
+      unsigned long long base = 0;
+      if (lane == leader) base = atomicAdd(a.queue, (unsigned long long)__popcll(mask));
+      base = __shfl(base, leader, WAVE);
+      if (need) {
+        const long long t = (long long)(base + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull)));
+        if (t >= a.nchunk) {
+          exhausted = true;
+        } else {
+          q = cell_of(a, t);
+          have = start_cell(a, t, q, off, c, recl_lds, kl);
+          tl.gated += have ? 0 : 1;
         }
-        need = !have && !exhausted;
       }
+      need = !have && !exhausted;
     }
     if (!wave_any(have)) break;
-    const bool wantj = have && c.req == REQ_JAC;
-    const bool wantf = have && c.req == REQ_F;
+    const bool wantj = have && c.req == lane::REQ_JAC;
+    const bool wantf = have && c.req == lane::REQ_F;
     const int nj = __popcll(__ballot(wantj ? 1 : 0));
     const int nf = __popcll(__ballot(wantf ? 1 : 0));
     const bool run_jac = nj > 0 && (nf == 0 || nj * 100 >= a.jac_pct * (nj + nf));
     if (run_jac) {
       if (ANALYTIC)
-        jac_analytic(c, wantj, mc, kl);
+        lane::jac_analytic(c, wantj, mc, kl);
       else
-        jac_batch(c, wantj, a.k, mc, kl);
+        lane::jac_batch(c, wantj, a.k, mc, kl);
     }
     else if (wantf)
-      rhs(kl, c.y, c.save2);
-    if (have && (c.req == REQ_NONE || (run_jac ? wantj : wantf))) {
-      c.req = REQ_NONE;
-      advance(c, a.dt, a.k, mc);
+      lane::rhs(kl, c.y, c.save2);
+    if (have && (c.req == lane::REQ_NONE || (run_jac ? wantj : wantf))) {
+      c.req = lane::REQ_NONE;
+      lane::advance(c, a.dt, a.k, gc, mc);
     }
-    if (have && c.req == REQ_DONE) {
-      status = finish_cell(a, mc, q, off, c, kl);
-      if (PERSISTENT) tl.integrated(c, status);
+    if (have && c.req == lane::REQ_DONE) {
+      finish_cell(a, mc, q, off, c, kl, tl, tally);
       have = false;
     }
-    if (!PERSISTENT && !wave_any(have)) break;
   }
-  if (!PERSISTENT) {
-    if (gated)
-      tl.cnt[NRG_CELL_GATED]++;
-    else if (q >= 0)
-      tl.integrated(c, status);
+  atomicAdd(&tally[ACC_STATUS0 + NRG_CELL_GATED], (unsigned long long)tl.gated);
+  atomicAdd(&tally[ACC_INTEG], (unsigned long long)tl.integrated);
+  atomicAdd(&tally[ACC_NSTEP], tl.nstep);
+  atomicAdd(&tally[ACC_NFE], tl.nfe);
+  atomicAdd(&tally[ACC_NJE], tl.nje);
+  atomicAdd(&tally[ACC_NCORR], tl.ncorr);
+  atomicAdd(&tally[ACC_NATT], tl.natt);
+  atomicMax(&tally[ACC_NSTEP_MAX], (unsigned long long)tl.nstep_max);
+  atomicMax(&tally[ACC_NFE_MAX], (unsigned long long)tl.nfe_max);
+  wave_sync();
+  if (lane == 0) {
+    unsigned long long failed = 0;
+    for (int s = 0; s < 6; ++s) failed += (s == NRG_CELL_OK || s == NRG_CELL_GATED) ? 0ull : tally[ACC_STATUS0 + s];
+    tally[ACC_STATUS0 + NRG_CELL_OK] = tally[ACC_INTEG] - failed;
   }
-  tl.flush(a.acc, lane);   // one atomic per wave and slot
+  flush_tally(a.acc, tally, lane);
 }
 #endif
 
-#if NRG_PART == 2
-// The integrator part ends here: its kernels, compiled with their own
-// scheduling options (the Makefile), and nothing else.
-#if !defined(NRG_BDF_JAC) || NRG_BDF_JAC == 1
-template __global__ void chem_bdf_kernel<false, false>(StepArgs);
-template __global__ void chem_bdf_kernel<true, false>(StepArgs);
+#if NRG_PART == 2 || NRG_PART == 3
+// The integrator parts end here: their kernels, compiled with their own
+// options (the Makefile), and nothing else.
+#if NRG_PART == 3
+template __global__ void chem_bdf_lane_kernel<false>(StepArgs);
+template __global__ void chem_bdf_lane_kernel<true>(StepArgs);
 #endif
-#if !defined(NRG_BDF_JAC) || NRG_BDF_JAC == 2
-template __global__ void chem_bdf_kernel<false, true>(StepArgs);
-template __global__ void chem_bdf_kernel<true, true>(StepArgs);
+#if NRG_PART == 2 && (!defined(NRG_BDF_JAC) || NRG_BDF_JAC == 1)
+template __global__ void chem_bdf_kernel<false>(StepArgs);
+#endif
+#if NRG_PART == 2 && (!defined(NRG_BDF_JAC) || NRG_BDF_JAC == 2)
+template __global__ void chem_bdf_kernel<true>(StepArgs);
 #endif
 }  // namespace kern
 }  // namespace NRG_TOPO_NS
@@ -1862,7 +2020,7 @@ struct StepKey {
   const double *rates;         // buffer the graph's kernels write (reallocated when it grows)
   int use_hist, form;
   long long chunk_max;
-  long long persistent_blocks; // grid of the persistent form (the autotuner may change it alone)
+  long long persistent_blocks; // the integrator's grid (the autotuner may change it alone)
   int jacobian;                // NRG_JAC_*: which integrator kernel the graph launches
 };
 
@@ -1877,7 +2035,8 @@ struct nrg_chem_handle {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int form = NRG_FORM_PLAIN;
   int jac_pct = 50;
-  int persistent_blocks = 0;               // resident one-wave blocks of the persistent form
+  int persistent_blocks = 0;               // resident one-wave blocks of the integrator
+  int lane_blocks = 0;                     // and of its one-cell-per-lane form
   // staging buffers for the host-pointer entry point
   std::vector<void *> stage;
   // cell records of one chunk: REC_PAIRS pairs of doubles per position
@@ -2029,7 +2188,9 @@ BdfConst make_const(const nrg_chem_opts &o)
   k.mxstep = o.mxstep;
   k.maxord = std::min(o.mxord, MAXORD);
   k.gather_pct = o.errtest_gather_pct;
-  k.refill_idle = o.refill_min_idle > 0 ? o.refill_min_idle : REFILL_MIN_IDLE_DEFAULT;
+  k.refill_idle = o.refill_min_idle > 0                ? o.refill_min_idle
+                  : o.cell_order == NRG_ORDER_STIFFNESS ? REFILL_IDLE_ORDERED
+                                                        : REFILL_IDLE_NATURAL;
   return k;
 }
 
@@ -2191,12 +2352,13 @@ int nrg_chem_create(const nrg_chem_mech *mech, const nrg_chem_opts *opts, nrg_ch
     hipDeviceProp_t prop;
     int per_cu = 0;
     if (hipGetDeviceProperties(&prop, h->device) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (chem_bdf_kernel<true, false>), WAVE, 0) !=
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, chem_bdf_kernel<false>, WAVE, 0) !=
             hipSuccess)
       return fail(set_error(NRG_CHEM_E_HIP, "occupancy query"));
     if (o.waves_per_cu > 0) per_cu = o.waves_per_cu;
     if (per_cu < 1) per_cu = 1;
     h->persistent_blocks = per_cu * prop.multiProcessorCount;
+    h->lane_blocks = (o.waves_per_cu > 0 ? o.waves_per_cu : LANE_WAVES_PER_CU) * prop.multiProcessorCount;
     h->num_cu = std::max(prop.multiProcessorCount, 1);
   }
   if (hipMemcpy(h->dev_mech, &h->host_mech, sizeof(MechCoef), hipMemcpyHostToDevice) != hipSuccess)
@@ -2306,10 +2468,33 @@ static int prepare_rates(nrg_chem_t *h, long long npos)
   return NRG_CHEM_OK;
 }
 
-// Launch rates_kernel + chem_bdf_kernel per chunk of `chunk` positions, with
+// Cells of a launch in stiffness order from which they go one to a lane
+// instead of one to a lane group: from there they fill the chip often enough
+// (65,536 once) that a lane's shorter way through a step counts more than the
+// group's shorter way through a cell.  Kernel ms, group against lane, KEROMNES:
+//   finite differences: 262,144 flame cells 4.62 / 4.49, 589,824 9.9 / 8.7,
+//   1M 17.4 / 14.6; igniting 262,144 5.2 / 4.6 in 100 ns and 11.8 / 13.3 in 1 us,
+//   545,400 in 1 us 23 / 25; with most cells cold (hot kernels) 884,736 2.6 / 3.6,
+//   1.4M 3.4 / 3.6, 2.1M 5.5 / 4.9.
+//   analytic Jacobian (few right-hand sides, so the vector work that a group
+//   shares counts less): 65,536 flame cells 0.91 / 1.11, 262,144 2.55 / 1.96;
+//   igniting 131,072 1.52 / 1.49, 196,608 2.14 / 1.80.  The learned step's
+//   fallback list holds no idle cells, which moves the line: 83,905 of 2.4M
+//   cells 1.67 / 1.51.
+// With nine or ten species a group has 16 lanes, and a lane's state spills:
+//   TEREZA flame cells 1M 33.0 / 31.1, 2.4M 72 / 64; hot kernels 2.1M 10.6 /
+//   15.1, 7.1M 42 / 30; analytic igniting 131,072 3.1 / 2.0.
+// In natural order a group is ahead at every size (1M flame cells: 23.5 ms, a
+// lane 39).
+static long long lane_cells(bool analytic, bool fallback)
+{
+  return analytic ? (fallback ? 1 : 3) << 16 : SA <= 8 ? 5 << 17 : 1 << 22;
+}
+
+// Launch rates_kernel + the integrator kernel per chunk of `chunk` positions, with
 // the chunk's rate constants in `rates` and its queue head in acc[ACC_QUEUE0 + ci].
 static void enqueue_chunks(nrg_chem_t *h, StepArgs &a, long long npos, long long chunk,
-                           double *rates, unsigned long long *acc)
+                           double *rates, unsigned long long *acc, bool fallback)
 {
   const long long nchunks = npos > 0 ? (npos + chunk - 1) / chunk : 0;
   a.rates = rates;
@@ -2320,28 +2505,35 @@ static void enqueue_chunks(nrg_chem_t *h, StepArgs &a, long long npos, long long
     a.queue = acc + ACC_QUEUE0 + ci;
     hipLaunchKernelGGL(rates_kernel, dim3((unsigned)((a.nchunk + RATES_CELLS - 1) / RATES_CELLS)),
                        dim3(256), 0, h->stream, a);
-    const long long need = (a.nchunk + WAVE - 1) / WAVE;
-    const bool an = h->opts.jacobian == NRG_JAC_ANALYTIC;
-    if (h->form == NRG_FORM_PERSISTENT) {
-      const long long nb = std::min<long long>(h->persistent_blocks, need);
-      if (an)
-        hipLaunchKernelGGL((chem_bdf_kernel<true, true>), dim3((unsigned)nb), dim3(WAVE), 0, h->stream, a);
-      else
-        hipLaunchKernelGGL((chem_bdf_kernel<true, false>), dim3((unsigned)nb), dim3(WAVE), 0, h->stream, a);
-    } else {
-      if (an)
-        hipLaunchKernelGGL((chem_bdf_kernel<false, true>), dim3((unsigned)need), dim3(WAVE), 0, h->stream, a);
-      else
-        hipLaunchKernelGGL((chem_bdf_kernel<false, false>), dim3((unsigned)need), dim3(WAVE), 0, h->stream, a);
-    }
+    // A wave holds fewer cells than it could where the grid gives the SIMDs less
+    // than a full wave each: cells that share a wave wait for each other's
+    // stages (420 flame cells: one to a wave 0.60 ms, eight 0.75; 16,384: the same).
+    a.cpw = (int)std::min<long long>(CPW, std::max<long long>(1, (a.nchunk + 4 * h->num_cu - 1) / (4 * h->num_cu)));
+    const bool analytic = h->opts.jacobian == NRG_JAC_ANALYTIC;
+    const bool ordered = a.list && a.list == h->order_list;
+    const long long need = (a.nchunk + a.cpw - 1) / a.cpw;
+    const dim3 grid((unsigned)std::min<long long>(need, h->persistent_blocks));
+    if constexpr (LANE_KERNEL)
+      if (ordered && a.nchunk >= lane_cells(analytic, fallback)) {
+        const dim3 lanes((unsigned)std::min<long long>((a.nchunk + WAVE - 1) / WAVE, h->lane_blocks));
+        if (analytic)
+          hipLaunchKernelGGL(chem_bdf_lane_kernel<true>, lanes, dim3(WAVE), 0, h->stream, a);
+        else
+          hipLaunchKernelGGL(chem_bdf_lane_kernel<false>, lanes, dim3(WAVE), 0, h->stream, a);
+        continue;
+      }
+    if (analytic)
+      hipLaunchKernelGGL(chem_bdf_kernel<true>, grid, dim3(WAVE), 0, h->stream, a);
+    else
+      hipLaunchKernelGGL(chem_bdf_kernel<false>, grid, dim3(WAVE), 0, h->stream, a);
   }
 }
 
-static int enqueue_integrator(nrg_chem_t *h, StepArgs &a, long long npos)
+static int enqueue_integrator(nrg_chem_t *h, StepArgs &a, long long npos, bool fallback = false)
 {
   int st = prepare_rates(h, npos);
   if (st) return st;
-  enqueue_chunks(h, a, npos, chunk_for(h, npos), h->rates, h->dev_acc);
+  enqueue_chunks(h, a, npos, chunk_for(h, npos), h->rates, h->dev_acc, fallback);
   HIP_TRY(hipGetLastError());
   return NRG_CHEM_OK;
 }
@@ -2560,7 +2752,7 @@ int nrg_chem_step_dev_noalloc(nrg_chem_t *h, const nrg_grid *grid, double dt, co
   float ms = 0.f;
   HIP_TRY(hipEventRecord(h->ev0, h->stream));
   hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(ACC_SLOTS), 0, h->stream, acc_dev, ACC_SLOTS);
-  if (a.g.ninner > 0) enqueue_chunks(h, a, a.g.ninner, NRG_NOALLOC_CHUNK_CELLS, rates, acc_dev);
+  if (a.g.ninner > 0) enqueue_chunks(h, a, a.g.ninner, NRG_NOALLOC_CHUNK_CELLS, rates, acc_dev, false);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(h->ev1, h->stream));
   HIP_TRY(hipMemcpyAsync(acc, acc_dev, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
@@ -2963,7 +3155,7 @@ int nrg_chem_autotune_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, const 
   hipDeviceProp_t prop;
   HIP_TRY(hipGetDeviceProperties(&prop, h->device));
   int occ = 0;
-  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (chem_bdf_kernel<true, false>), WAVE, 0));
+  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, chem_bdf_kernel<false>, WAVE, 0));
   occ = std::max(occ, 1);
   struct Cfg {
     int form, order, jac, wpc;
@@ -2977,6 +3169,7 @@ int nrg_chem_autotune_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, const 
     h->order = c.order;
     h->jac_pct = c.jac;
     h->persistent_blocks = (c.wpc > 0 ? c.wpc : occ) * prop.multiProcessorCount;
+    h->lane_blocks = (c.wpc > 0 ? c.wpc : LANE_WAVES_PER_CU) * prop.multiProcessorCount;
     h->chunk_max = c.chunk;
   };
   auto trial = [&](const Cfg &c, double &ms) -> int {
@@ -3026,12 +3219,6 @@ int nrg_chem_autotune_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, const 
       c.order = order;
       if ((st = consider(c))) return st;
     }
-  for (int form : {NRG_FORM_PLAIN, NRG_FORM_PERSISTENT})
-    if (form != best.form) {
-      Cfg c = best;
-      c.form = form;
-      if ((st = consider(c))) return st;
-    }
   for (int gather : {0, 100})
     if (gather != best.gather) {
       Cfg c = best;
@@ -3044,19 +3231,17 @@ int nrg_chem_autotune_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, const 
       c.jac = jac;
       if ((st = consider(c))) return st;
     }
-  if (best.form == NRG_FORM_PERSISTENT)
-    for (int refill : {48, REFILL_MIN_IDLE_DEFAULT})
-      if (refill != best.refill) {
-        Cfg c = best;
-        c.refill = refill;
-        if ((st = consider(c))) return st;
-      }
-  if (best.form == NRG_FORM_PERSISTENT)
-    for (int w : {2 * occ, 4 * occ}) {
+  for (int refill : {REFILL_IDLE_NATURAL, REFILL_IDLE_ORDERED})
+    if (refill != best.refill) {
       Cfg c = best;
-      c.wpc = w;
+      c.refill = refill;
       if ((st = consider(c))) return st;
     }
+  for (int w : {2 * occ, 4 * occ}) {
+    Cfg c = best;
+    c.wpc = w;
+    if ((st = consider(c))) return st;
+  }
   for (long long ch : {1ll << 21, 1ll << 22, 1ll << 23, 1ll << 24})
     if (ch != best.chunk) {
       Cfg c = best;
@@ -3253,7 +3438,7 @@ int nrg_chem_surrogate_step_dev(nrg_chem_t *h, nrg_mlp_t *mlp, const nrg_surroga
         h->hist_valid = true;
         h->hist_grid = a.g;
       }
-      if ((st = enqueue_integrator(h, a, nfb))) return st;
+      if ((st = enqueue_integrator(h, a, nfb, true))) return st;
     }
     HIP_TRY(hipEventRecord(h->ev1, h->stream));
     HIP_TRY(hipMemcpyAsync(acc, h->dev_acc, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
@@ -3326,4 +3511,4 @@ __attribute__((visibility("hidden"))) const nrg_topo_ops *NRG_TOPO_OPS_FN()
 #undef NRG_TOPO_OP_INIT
   return &table;
 }
-#endif  // NRG_PART != 2
+#endif  // NRG_PART < 2
