@@ -1,5 +1,5 @@
-// mlp.hip -- BF16 MFMA perceptron for the chemistry surrogate: training GEMMs
-// with fused epilogues, a fused all-layer inference kernel, loss and Adam.
+// mlp.hip -- BF16 MFMA perceptron for the chemistry surrogate: training (a pass
+// over the rows, a pass over the weights, Adam) and fused all-layer inference.
 //
 // MFMA: v_mfma_f32_32x32x16_bf16 (gfx950).  Lane l of a wave holds
 //   A fragment: A[row = l%32][k = 8*(l/32) + v], v = 0..7
@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <new>
 #include <vector>
 
@@ -53,68 +54,277 @@ __device__ __forceinline__ float gelu_grad(float z)
   return sg + 2.0f * z * sg * (1.0f - sg) * dudz;
 }
 
-// ---- training GEMM: one wave per 32x32 tile of C, optional split over K ----------
-enum { EPI_STORE = 0, EPI_BIAS_GELU = 1, EPI_BIAS = 2, EPI_GELU_BACK = 3 };
-
-struct GemmArgs {
-  const bf16 *A;
-  long long sAm, sAk;          // A(m, k) = A[m*sAm + k*sAk]
-  const bf16 *B;
-  long long sBk, sBn;          // B(k, n) = B[k*sBk + n*sBn]
-  int M, N, K;
-  int mode;                    // EPI_*
-  int ksplit;                  // EPI_STORE only: K ranges per tile, atomically added
-  long long ldc;
-  float *C;                    // EPI_STORE / EPI_BIAS out (EPI_STORE with ksplit > 1: pre-zeroed)
-  const float *bias;           // EPI_BIAS_GELU / EPI_BIAS
-  float *Z;                    // EPI_BIAS_GELU: pre-activation
-  bf16 *H;                     // EPI_BIAS_GELU: gelu(z); EPI_GELU_BACK: acc * gelu'(Zin)
-  const float *Zin;            // EPI_GELU_BACK
+// ---- training: one pass over the rows, one over the weights ----------------------
+// A step was ~20 launches of a GEMM that loaded its operands by single strided
+// bf16 values (689 us for 4096 rows of 256 x 4).  Two kernels do the work now:
+//   train_rows_kernel  forward, loss and the chain of dZ for a block's rows, whose
+//                      activations stay in LDS (one wave per 32 columns);
+//   train_weights_kernel  all dW = H^T dZ and db, split over the rows.
+// Between them H and dZ are kept as the second one's MFMA fragments: a lane's
+// accumulator holds 16 rows of its column, and since the order of the rows inside
+// a reduction over them is free, elements 0..7 and 8..15 are its 8 k-values of two
+// k-blocks as they stand (rows 16 kb + 8 (v/4) + 4 hi + v%4), so that every operand
+// of the reduction is one coalesced 16-byte load and nothing is transposed.
+// What bounds the first is a block's way through the layers (9 products of 16
+// dependent MFMAs, each with its GELUs and a barrier), the second the latency of
+// its loads and the atomics that add up the ranges.  4096 rows of 256 x 4: 27 + 13
+// us (before: 20 launches, 420 us).
+struct TrainArgs {
+  const float *x, *t, *w;      // n x n_in, n x n_out, n_out weights or NULL
+  long long n;
+  int n_in, n_out, layers;     // layers: hidden layers
+  const bf16 *Wf[MLP_MAX_LAYERS];    // forward fragments of the weights (Wsw)
+  const bf16 *Wb[MLP_MAX_LAYERS];    // backward fragments (frag_kernel)
+  const float *bias[MLP_MAX_LAYERS];
+  bf16 *Xf, *dYf;              // fragments of the input and of dL/dy
+  bf16 *Hf[MLP_MAX_LAYERS], *dZf[MLP_MAX_LAYERS];   // of each hidden layer
+  float *gz[MLP_MAX_LAYERS];   // gelu'(z), each lane's 16 values together
+  float *y;                    // n x n_out, or NULL
+  float *loss_part;            // a value per tile
+  float *grad;                 // gradients, cleared here for train_weights_kernel
+  long long n_grad;
 };
 
-__global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g)
+// Barrier for what went through LDS.  (__syncthreads also waits for every global
+// load and store under way, here the next product's weights and the fragments.)
+__device__ __forceinline__ void lds_barrier()
 {
-  const int l = threadIdx.x & (WAVE - 1);
-  const int tiles_n = g.N / 32;
-  const int ntiles = (g.M / 32) * tiles_n;
-  const long long wid = (long long)blockIdx.x * 4 + threadIdx.x / WAVE;
-  if (wid >= (long long)ntiles * g.ksplit) return;
-  const int tile = (int)(wid % ntiles), part = (int)(wid / ntiles);
-  const int m0 = (tile / tiles_n) * 32, n0 = (tile % tiles_n) * 32;
-  const int r32 = l & 31, hi = l >> 5;
-  const int kchunk = ((g.K / 16 + g.ksplit - 1) / g.ksplit) * 16;
-  const int kbeg = part * kchunk, kend = min(g.K, kbeg + kchunk);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
 
-  f32x16 acc = {};
-  const bf16 *Ap = g.A + (long long)(m0 + r32) * g.sAm;
-  const bf16 *Bp = g.B + (long long)(n0 + r32) * g.sBn;
-  for (int k0 = kbeg; k0 < kend; k0 += 16) {
-    bf16x8 a, b;
+// row of its 32-row tile that element r of a lane's accumulator holds
+__device__ __forceinline__ int acc_row(int r, int hi) { return 8 * (r / 4) + 4 * hi + r % 4; }
+
+// A lane's first EL elements of an accumulator as bf16: its share of the fragments
+// of EL / 8 k-blocks.
+template <int EL>
+__device__ __forceinline__ void store_frags(bf16 *f, const bf16 (&v)[EL], int l)
+{
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      const long long k = k0 + 8 * hi + v;
-      a[v] = Ap[k * g.sAk];
-      b[v] = Bp[k * g.sBk];
+  for (int k = 0; k < EL / 8; ++k) {
+    bf16x8 x;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) x[r] = v[8 * k + r];
+    reinterpret_cast<bf16x8 *>(f)[k * WAVE + l] = x;
+  }
+}
+
+// Hidden width 32 NT (one wave per 32 columns), 2 EL rows per block (EL: the
+// accumulator elements in use; with 8 the MFMAs see the 16 rows twice, but the
+// epilogues, which cost more, are halved and twice the CUs work).
+template <int NT, int EL>
+__global__ void __launch_bounds__(NT * 64) train_rows_kernel(TrainArgs a)
+{
+  constexpr int HID = 32 * NT, KB = 2 * NT, LD = HID + 8, ROWS = 2 * EL, NTHR = NT * WAVE;
+  constexpr int INLD = MLP_IN_PAD + 8;
+  static_assert(EL == 8 || EL == 16, "one or two k-blocks of rows");
+  __shared__ __align__(16) bf16 act[2][ROWS][LD];
+  __shared__ __align__(16) bf16 io[ROWS][INLD];  // the input, later dL/dy
+  const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
+  const int r32 = l & 31, hi = l >> 5, col = 32 * w + r32;
+  const int arow = r32 % ROWS;
+  const long long row0 = (long long)blockIdx.x * ROWS;
+  // the rows' fragments of columns 32 c.. of a matrix nt tiles wide
+  auto frag = [&](bf16 *f, int nt, int c) {
+    const long long kb = (long long)blockIdx.x * (ROWS / 16);   // first k-block
+    return f + (((kb / 2) * nt + c) * 2 + kb % 2) * (WAVE * 8);
+  };
+  auto slope = [&](int layer) {                  // the lane's EL values of gelu'(z)
+    return a.gz[layer] + (((long long)blockIdx.x * NT + w) * WAVE + l) * EL;
+  };
+
+  for (long long i = (long long)blockIdx.x * NTHR + threadIdx.x; i < a.n_grad; i += (long long)gridDim.x * NTHR)
+    a.grad[i] = 0.0f;
+  for (int i = threadIdx.x; i < ROWS * MLP_IN_PAD; i += NTHR) {
+    const int row = i / MLP_IN_PAD, c = i % MLP_IN_PAD;
+    io[row][c] = (bf16)(row0 + row < a.n && c < a.n_in ? a.x[(row0 + row) * a.n_in + c] : 0.0f);
+  }
+  bf16x8 b[KB];                                  // this wave's weights of a layer
+  auto weights = [&](const bf16 *W, int kbs) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      if (kb < kbs) b[kb] = reinterpret_cast<const bf16x8 *>(W)[(kb * NT + w) * WAVE + l];
+  };
+  f32x16 acc;
+  auto product = [&](const bf16 *in, int ld, int kbs) {
+    acc = f32x16{};
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      if (kb < kbs) acc = mfma(*reinterpret_cast<const bf16x8 *>(in + arow * ld + 16 * kb + 8 * hi), b[kb], acc);
+  };
+  weights(a.Wf[0], 2);
+  lds_barrier();
+  if (w == 0) {                                  // fragments of the input
+    bf16 v[EL];
+#pragma unroll
+    for (int r = 0; r < EL; ++r) v[r] = io[acc_row(r, hi)][r32];
+    store_frags<EL>(frag(a.Xf, 1, 0), v, l);
+  }
+
+  // forward through the hidden layers
+  for (int layer = 0; layer < a.layers; ++layer) {
+    if (layer == 0)
+      product(&io[0][0], INLD, 2);
+    else
+      product(&act[(layer - 1) & 1][0][0], LD, KB);
+    if (layer + 1 < a.layers) weights(a.Wf[layer + 1], KB);   // on their way during the epilogue
+    const float bias = a.bias[layer][col];
+    bf16 v[EL];
+    float *gz = slope(layer);
+#pragma unroll
+    for (int r = 0; r < EL; ++r) {
+      const float z = acc[r] + bias;
+      gz[r] = gelu_grad(z);
+      v[r] = (bf16)gelu(z);
+      act[layer & 1][acc_row(r, hi)][col] = v[r];
     }
-    acc = mfma(a, b, acc);
+    store_frags<EL>(frag(a.Hf[layer], NT, w), v, l);
+    lds_barrier();
+  }
+
+  // output, loss = sum_rows sum_c w_c (y - t)^2 / n and dY = 2 w_c (y - t) / n
+  weights(a.Wb[a.layers], 2);
+  if (w == 0) {
+    const bf16 *in = &act[(a.layers - 1) & 1][arow][8 * hi];
+    f32x16 o = {};
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      o = mfma(*reinterpret_cast<const bf16x8 *>(in + 16 * kb),
+               reinterpret_cast<const bf16x8 *>(a.Wf[a.layers])[kb * WAVE + l], o);
+    const float bias = a.bias[a.layers][r32], inv_n = 1.0f / (float)a.n;
+    const float wc = a.w && r32 < a.n_out ? a.w[r32] : 1.0f;
+    float s = 0.0f;
+    bf16 v[EL];
+#pragma unroll
+    for (int r = 0; r < EL; ++r) {
+      const long long row = row0 + acc_row(r, hi);
+      float g = 0.0f;
+      if (row < a.n && r32 < a.n_out) {
+        const float y = o[r] + bias, d = y - a.t[row * a.n_out + r32];
+        s += wc * d * d;
+        g = 2.0f * wc * d * inv_n;
+        if (a.y) a.y[row * a.n_out + r32] = y;
+      }
+      v[r] = (bf16)g;
+      io[acc_row(r, hi)][r32] = v[r];
+    }
+    store_frags<EL>(frag(a.dYf, 1, 0), v, l);
+    s *= inv_n;
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if (l == 0) a.loss_part[blockIdx.x] = s;
+  }
+  lds_barrier();
+
+  // dZ of the hidden layers, last first: (dZ of the next W^T) * gelu'(z)
+  for (int layer = a.layers - 1; layer >= 0; --layer) {
+    float gz[EL];
+#pragma unroll
+    for (int r = 0; r < EL; ++r) gz[r] = slope(layer)[r];
+    if (layer == a.layers - 1)
+      product(&io[0][0], INLD, 2);
+    else
+      product(&act[layer & 1][0][0], LD, KB);
+    if (layer > 0) weights(a.Wb[layer], KB);
+    bf16 v[EL];
+#pragma unroll
+    for (int r = 0; r < EL; ++r) {
+      v[r] = (bf16)(acc[r] * gz[r]);
+      if (layer > 0) act[(layer - 1) & 1][acc_row(r, hi)][col] = v[r];
+    }
+    store_frags<EL>(frag(a.dZf[layer], NT, w), v, l);
+    lds_barrier();
+  }
+}
+
+// dW = H^T dZ and db = sum of dZ of every layer: a block takes 2 x 2 tiles of one
+// layer's weights (a fragment then serves two products) and a range of the rows,
+// which its four waves share; their sums meet in LDS and the ranges' in G.
+struct WeightLayer {
+  const bf16 *A, *B;           // fragments of H (the layer's input) and of dZ
+  int MT, NT;                  // tiles of the weights
+  int block0;                  // first block (x) of the layer
+  int K, N;                    // extents kept of them, and the row pitch
+  float *dW, *db;
+};
+struct WeightArgs {
+  WeightLayer L[MLP_MAX_LAYERS];
+  int layers;                  // weight matrices
+  long long kblocks, kper;     // 16-row blocks, and those of one y-range
+  const float *loss_part;
+  long long n_part;
+  float *loss;                 // or NULL
+};
+
+__global__ void __launch_bounds__(256) train_weights_kernel(WeightArgs a)
+{
+  __shared__ float red[4][4][16][WAVE];
+  __shared__ float redb[4][2][32];
+  const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
+  const int r32 = l & 31, hi = l >> 5;
+  int i = 0;
+  while (i + 1 < a.layers && (int)blockIdx.x >= a.L[i + 1].block0) ++i;
+  const WeightLayer &L = a.L[i];
+  const int bn = (L.NT + 1) / 2, bid = (int)blockIdx.x - L.block0;
+  const int mt = bid / bn * 2, nt = bid % bn * 2;
+  const int m1 = mt + 1 < L.MT ? mt + 1 : mt, n1 = nt + 1 < L.NT ? nt + 1 : nt;   // a missing tile: twice the first
+  const bf16x8 *A = reinterpret_cast<const bf16x8 *>(L.A) + l, *B = reinterpret_cast<const bf16x8 *>(L.B) + l;
+  const long long k1 = min(a.kblocks, ((long long)blockIdx.y + 1) * a.kper);
+  f32x16 c[2][2] = {};
+  float s[2] = {0.0f, 0.0f};
+  constexpr int AHEAD = 4;       // k-blocks loaded together
+  for (long long k0 = (long long)blockIdx.y * a.kper + w; k0 < k1; k0 += 4 * AHEAD) {
+    bf16x8 fa[AHEAD][2] = {}, fb[AHEAD][2] = {};
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) {
+      const long long k = k0 + 4 * q;
+      if (k < k1) {
+        const long long ta = (k / 2) * L.MT, tb = (k / 2) * L.NT;
+        const int h = (int)(k & 1);
+        fa[q][0] = A[((ta + mt) * 2 + h) * WAVE];
+        fa[q][1] = A[((ta + m1) * 2 + h) * WAVE];
+        fb[q][0] = B[((tb + nt) * 2 + h) * WAVE];
+        fb[q][1] = B[((tb + n1) * 2 + h) * WAVE];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c[i / 2][i % 2] = mfma(fa[q][i / 2], fb[q][i % 2], c[i / 2][i % 2]);
+      if (mt == 0) {
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+          s[0] += (float)fb[q][0][v];
+          s[1] += (float)fb[q][1][v];
+        }
+      }
+    }
   }
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const long long row = m0 + 8 * (r / 4) + 4 * hi + (r % 4);
-    const int col = n0 + r32;
-    const long long o = row * g.ldc + col;
-    if (g.mode == EPI_STORE) {
-      if (g.ksplit > 1) atomicAdd(&g.C[o], acc[r]);
-      else g.C[o] = acc[r];
-    } else if (g.mode == EPI_BIAS_GELU) {
-      const float z = acc[r] + g.bias[col];
-      g.Z[o] = z;
-      g.H[o] = (bf16)gelu(z);
-    } else if (g.mode == EPI_BIAS) {
-      g.C[o] = acc[r] + g.bias[col];
-    } else {
-      g.H[o] = (bf16)(acc[r] * gelu_grad(g.Zin[o]));
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[w][q][r][l] = c[q / 2][q % 2][r];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    s[j] += __shfl_xor(s[j], 32);
+    if (hi == 0) redb[w][j][r32] = s[j];
+  }
+  __syncthreads();
+  const int tm = mt + w / 2, tn = nt + w % 2;        // wave w adds up tile w
+  if (tm < L.MT && tn < L.NT) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float v = ((red[0][w][r][l] + red[1][w][r][l]) + red[2][w][r][l]) + red[3][w][r][l];
+      const int row = 32 * tm + acc_row(r, hi), col = 32 * tn + r32;
+      if (row < L.K && col < L.N) atomicAdd(&L.dW[(long long)row * L.N + col], v);
     }
+    if (mt == 0 && w < 2 && hi == 0 && 32 * tn + r32 < L.N)
+      atomicAdd(&L.db[32 * tn + r32], ((redb[0][w][r32] + redb[1][w][r32]) + redb[2][w][r32]) + redb[3][w][r32]);
+  }
+  if (a.loss && blockIdx.x == 0 && blockIdx.y == 0 && w == 0) {
+    float p = 0.0f;
+    for (long long k = l; k < a.n_part; k += WAVE) p += a.loss_part[k];
+    for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off);
+    if (l == 0) *a.loss = p;
   }
 }
 
@@ -134,42 +344,6 @@ __global__ void pack_input_kernel(const float *x, long long n, int n_in, bf16 *X
   const long long row = i / MLP_IN_PAD;
   const int c = (int)(i % MLP_IN_PAD);
   X[i] = (bf16)(c < n_in ? x[row * n_in + c] : 0.0f);
-}
-
-// loss = sum_rows sum_c w_c (y - t)^2 / n and dY = 2 w_c (y - t) / n (bf16, padded)
-__global__ void loss_kernel(const float *Y, const float *T, const float *w, long long n, int n_out,
-                            bf16 *dY, float *loss)
-{
-  const long long row = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  float s = 0.0f;
-  if (row < n) {
-    const float inv_n = 1.0f / (float)n;
-    for (int c = 0; c < MLP_OUT_PAD; ++c) {
-      float g = 0.0f;
-      if (c < n_out) {
-        const float d = Y[row * MLP_OUT_PAD + c] - T[row * n_out + c];
-        const float wc = w ? w[c] : 1.0f;
-        s += wc * d * d;
-        g = 2.0f * wc * d * inv_n;
-      }
-      dY[row * MLP_OUT_PAD + c] = (bf16)g;
-    }
-    s *= inv_n;
-  }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if (loss && (threadIdx.x & (WAVE - 1)) == 0) atomicAdd(loss, s);
-}
-
-// db[c] += sum over a 256-row slab of dZ[row][c]
-__global__ void bias_grad_kernel(const bf16 *dZ, long long n, int N, float *db)
-{
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  const long long r0 = (long long)blockIdx.y * 256;
-  const long long r1 = r0 + 256 < n ? r0 + 256 : n;
-  float s = 0.0f;
-  for (long long r = r0; r < r1; ++r) s += (float)dZ[r * N + c];
-  atomicAdd(&db[c], s);
 }
 
 __global__ void adam_kernel(float *P, bf16 *Pbf, const float *G, float *M1, float *M2, long long n,
@@ -192,28 +366,6 @@ __global__ void to_bf16_kernel(const float *P, bf16 *Pbf, long long n)
 {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) Pbf[i] = (bf16)P[i];
-}
-
-__global__ void gather_kernel(const float *src, const int *idx, float *dst, long long n)
-{
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[idx[i]];
-}
-
-// Inference layout of layer weights: Wsw[((kb*NT + nt)*64 + lane)*8 + v] =
-// W[k = 16 kb + 8 (lane/32) + v][n = 32 nt + lane%32], so a lane's B fragment
-// is one 16-byte load.
-__global__ void swizzle_kernel(const bf16 *W, int K, int N, bf16 *Wsw)
-{
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)K * N) return;
-  const int v = (int)(i % 8);
-  const int lane = (int)((i / 8) % WAVE);
-  const long long f = i / (8 * WAVE);
-  const int NT = N / 32;
-  const int nt = (int)(f % NT), kb = (int)(f / NT);
-  const int k = 16 * kb + 8 * (lane / 32) + v, n = 32 * nt + lane % 32;
-  Wsw[i] = W[(long long)k * N + n];
 }
 
 // ---- fused inference: all layers, 32 rows per wave, 128 rows per block -----------
@@ -419,20 +571,42 @@ __host__ __device__ inline int t_phys(int kl)
   return 32 * (kb / 2) + 8 * (r / 4) + 4 * hi + r % 4;
 }
 
-// WswT[((mt*KB + kb)*64 + lane)*8 + v] = W[k][n], n = 32 mt + lane%32,
-// k = (permuted ? t_phys : identity)(16 kb + 8 (lane/32) + v).
-__global__ void swizzle_t_kernel(const bf16 *W, int K, int N, int permuted, bf16 *WswT)
+// MFMA fragments of every layer's weights W (K x N, row-major), 8 values a thread,
+// so that a lane's fragment is one 16-byte load:
+//   Wsw[((kb*N/32 + nt)*64 + lane)*8 + v] = W[16 kb + 8 (lane/32) + v][32 nt + lane%32]
+//     (forward: kernels with the weights as B operand)
+//   Wb[((kb*K/32 + nt)*64 + lane)*8 + v] = W[32 nt + lane%32][16 kb + 8 (lane/32) + v]
+//     (backward: W^T as B operand)
+//   WswT[((mt*K/16 + kb)*64 + lane)*8 + v] = W[k][32 mt + lane%32],
+//     k = (layer > 0 ? t_phys : identity)(16 kb + 8 (lane/32) + v)
+struct FragArgs {
+  int K[MLP_MAX_LAYERS], N[MLP_MAX_LAYERS], layers;
+  long long w_off[MLP_MAX_LAYERS], sw_off[MLP_MAX_LAYERS + 1];
+  const bf16 *W;
+  bf16 *Wsw, *Wb, *WswT;
+};
+__global__ void __launch_bounds__(256) frag_kernel(FragArgs a)
 {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)K * N) return;
-  const int v = (int)(i % 8);
-  const int lane = (int)((i / 8) % WAVE);
-  const long long f = i / (8 * WAVE);
-  const int KB = K / 16;
-  const int kb = (int)(f % KB), mt = (int)(f / KB);
-  const int kl = 16 * kb + 8 * (lane / 32) + v;
-  const int k = permuted ? t_phys(kl) : kl;
-  WswT[i] = W[(long long)k * N + 32 * mt + lane % 32];
+  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= a.sw_off[a.layers]) return;
+  int ly = 0;
+  while (i >= a.sw_off[ly + 1]) ++ly;
+  const int K = a.K[ly], N = a.N[ly];
+  const bf16 *W = a.W + a.w_off[ly];
+  const long long f = (i - a.sw_off[ly]) / 8;
+  const int lane = (int)(f % WAVE), r32 = lane & 31, k8 = 8 * (lane >> 5);
+  const int q = (int)(f / WAVE);
+  bf16x8 fw, bw, tr;
+#pragma unroll
+  for (int v = 0; v < 8; ++v) {
+    fw[v] = W[(long long)(16 * (q / (N / 32)) + k8 + v) * N + 32 * (q % (N / 32)) + r32];
+    bw[v] = W[(long long)(32 * (q % (K / 32)) + r32) * N + 16 * (q / (K / 32)) + k8 + v];
+    const int kl = 16 * (q % (K / 16)) + k8 + v;
+    tr[v] = W[(long long)(ly > 0 ? t_phys(kl) : kl) * N + 32 * (q / (K / 16)) + r32];
+  }
+  *reinterpret_cast<bf16x8 *>(a.Wsw + i) = fw;
+  *reinterpret_cast<bf16x8 *>(a.Wb + i) = bw;
+  *reinterpret_cast<bf16x8 *>(a.WswT + i) = tr;
 }
 
 // Accumulator start value: the bias of the lane's 16 output features of tile mt
@@ -570,160 +744,171 @@ struct MlpLayer {
 }  // namespace nrg
 
 struct nrg_mlp {
-  int device = 0;
+  int device = 0, num_cu = 0;
   hipStream_t stream = nullptr;
   int n_in = 0, hidden = 0, layers = 0, n_out = 0;
   std::vector<nrg::MlpLayer> L;            // layers + 1 entries
   long long n_pad = 0, n_packed = 0, n_sw = 0;
   float *P = nullptr, *G = nullptr, *M1 = nullptr, *M2 = nullptr;
-  nrg::bf16 *Pbf = nullptr, *Wsw = nullptr, *WswT = nullptr;   // WswT: transposed-kernel layout
-  int *gidx = nullptr;                      // packed index -> padded index
+  nrg::bf16 *Pbf = nullptr, *Wsw = nullptr, *Wb = nullptr, *WswT = nullptr;   // weights, and as fragments
   long long adam_t = 0;
-  bool sw_dirty = true;
+  bool sw_dirty = true;                     // the fragments are older than the weights
+  bool sw_synced = true;                    // written and waited for (other streams read them)
   // batch workspace
   long long cap = 0;
-  nrg::bf16 *X = nullptr, *dY = nullptr;
-  float *Yb = nullptr, *loss_tmp = nullptr;
-  std::vector<nrg::bf16 *> H;               // per hidden layer, n x hidden
-  std::vector<float *> Z;
-  nrg::bf16 *dZ[2] = {nullptr, nullptr};
+  nrg::bf16 *X = nullptr;                   // inference: n x 32
+  long long train_cap = 0;
+  nrg::bf16 *Xf = nullptr, *dYf = nullptr;  // training (TrainArgs)
+  float *loss_part = nullptr;
+  std::vector<nrg::bf16 *> Hf, dZf;         // per hidden layer
+  std::vector<float *> gz;
 };
 
 namespace nrg {
 namespace {
 
-int launch_gemm(nrg_mlp_t *h, const GemmArgs &g0)
+void free_all(std::initializer_list<void *> ps)
 {
-  GemmArgs g = g0;
-  if (g.M % 32 || g.N % 32 || g.K % 16 || g.M <= 0 || g.N <= 0 || g.K <= 0 || g.ksplit < 1)
-    return set_error(NRG_CHEM_E_ARG, "gemm shape %dx%dx%d not supported", g.M, g.N, g.K);
-  const long long waves = (long long)(g.M / 32) * (g.N / 32) * g.ksplit;
-  hipLaunchKernelGGL(gemm_kernel, dim3(blocks_for(waves, 4)), dim3(256), 0, h->stream, g);
-  HIP_TRY(hipGetLastError());
-  return NRG_CHEM_OK;
+  for (void *p : ps)
+    if (p) (void)hipFree(p);
 }
 
 int ensure_batch(nrg_mlp_t *h, long long n)
 {
   if (n <= h->cap) return NRG_CHEM_OK;
-  auto fr = [](void *p) { if (p) (void)hipFree(p); };
-  fr(h->X); fr(h->dY); fr(h->Yb); fr(h->dZ[0]); fr(h->dZ[1]);
-  for (auto p : h->H) fr(p);
-  for (auto p : h->Z) fr(p);
-  h->H.assign(h->layers, nullptr);
-  h->Z.assign(h->layers, nullptr);
-  h->X = h->dY = h->dZ[0] = h->dZ[1] = nullptr;
-  h->Yb = nullptr;
+  free_all({h->X});
+  h->X = nullptr;
   h->cap = 0;
   const long long m = ((n + 127) / 128) * 128;
   HIP_TRY(hipMalloc(&h->X, m * MLP_IN_PAD * sizeof(bf16)));
-  HIP_TRY(hipMalloc(&h->dY, m * MLP_OUT_PAD * sizeof(bf16)));
-  HIP_TRY(hipMalloc(&h->Yb, m * MLP_OUT_PAD * sizeof(float)));
-  for (int i = 0; i < 2; ++i) HIP_TRY(hipMalloc(&h->dZ[i], m * h->hidden * sizeof(bf16)));
-  for (int i = 0; i < h->layers; ++i) {
-    HIP_TRY(hipMalloc(&h->H[i], m * h->hidden * sizeof(bf16)));
-    HIP_TRY(hipMalloc(&h->Z[i], m * h->hidden * sizeof(float)));
-  }
   h->cap = m;
   return NRG_CHEM_OK;
 }
 
-int refresh_swizzle(nrg_mlp_t *h)
+void free_train(nrg_mlp_t *h)
 {
-  if (!h->sw_dirty) return NRG_CHEM_OK;
-  for (size_t i = 0; i < h->L.size(); ++i) {
-    const MlpLayer &ly = h->L[i];
-    const long long n = (long long)ly.K * ly.N;
-    hipLaunchKernelGGL(swizzle_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream,
-                       h->Pbf + ly.w_off, ly.K, ly.N, h->Wsw + ly.sw_off);
-    hipLaunchKernelGGL(swizzle_t_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream,
-                       h->Pbf + ly.w_off, ly.K, ly.N, i > 0 ? 1 : 0, h->WswT + ly.sw_off);
+  free_all({h->Xf, h->dYf, h->loss_part});
+  for (auto p : h->Hf) free_all({p});
+  for (auto p : h->dZf) free_all({p});
+  for (auto p : h->gz) free_all({p});
+  h->Xf = h->dYf = nullptr;
+  h->loss_part = nullptr;
+  h->Hf.assign(h->layers, nullptr);
+  h->dZf.assign(h->layers, nullptr);
+  h->gz.assign(h->layers, nullptr);
+  h->train_cap = 0;
+}
+
+int ensure_train(nrg_mlp_t *h, long long n)
+{
+  if (n <= h->train_cap) return NRG_CHEM_OK;
+  free_train(h);
+  const long long m = ((n + 127) / 128) * 128;
+  HIP_TRY(hipMalloc(&h->Xf, m * MLP_IN_PAD * sizeof(bf16)));
+  HIP_TRY(hipMalloc(&h->dYf, m * MLP_OUT_PAD * sizeof(bf16)));
+  HIP_TRY(hipMalloc(&h->loss_part, m / 16 * sizeof(float)));
+  for (int i = 0; i < h->layers; ++i) {
+    HIP_TRY(hipMalloc(&h->Hf[i], m * h->hidden * sizeof(bf16)));
+    HIP_TRY(hipMalloc(&h->dZf[i], m * h->hidden * sizeof(bf16)));
+    HIP_TRY(hipMalloc(&h->gz[i], m * h->hidden * sizeof(float)));
   }
-  HIP_TRY(hipGetLastError());
-  // inference may run on another stream (the chemistry handle's)
-  HIP_TRY(hipStreamSynchronize(h->stream));
-  h->sw_dirty = false;
+  h->train_cap = m;
   return NRG_CHEM_OK;
 }
 
-// Forward of the training path (rows padded to a multiple of 32 inside the workspace).
-int forward_train(nrg_mlp_t *h, long long n, const float *x)
+// Bring the fragments up to date on the handle's stream; with `wait`, for other
+// streams too (inference may run on the chemistry handle's).
+int refresh_frags(nrg_mlp_t *h, bool wait)
 {
-  int rc = ensure_batch(h, n);
+  if (h->sw_dirty) {
+    FragArgs f{};
+    f.layers = (int)h->L.size();
+    for (int i = 0; i < f.layers; ++i) {
+      f.K[i] = h->L[i].K; f.N[i] = h->L[i].N;
+      f.w_off[i] = h->L[i].w_off; f.sw_off[i] = h->L[i].sw_off;
+    }
+    f.sw_off[f.layers] = h->n_sw;
+    f.W = h->Pbf; f.Wsw = h->Wsw; f.Wb = h->Wb; f.WswT = h->WswT;
+    hipLaunchKernelGGL(frag_kernel, dim3(blocks_for(h->n_sw / 8, 256)), dim3(256), 0, h->stream, f);
+    HIP_TRY(hipGetLastError());
+    h->sw_dirty = false;
+    h->sw_synced = false;
+  }
+  if (wait && !h->sw_synced) {
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    h->sw_synced = true;
+  }
+  return NRG_CHEM_OK;
+}
+
+template <int NT>
+void launch_rows(nrg_mlp_t *h, const TrainArgs &a, long long blocks, int rows)
+{
+  if (rows == 16)
+    hipLaunchKernelGGL((train_rows_kernel<NT, 8>), dim3((unsigned)blocks), dim3(64 * NT), 0, h->stream, a);
+  else
+    hipLaunchKernelGGL((train_rows_kernel<NT, 16>), dim3((unsigned)blocks), dim3(64 * NT), 0, h->stream, a);
+}
+
+// Loss, predictions and the gradient: packed into `grad`, or padded into h->G.
+int loss_and_grad(nrg_mlp_t *h, long long n, const float *x, const float *t, const float *w,
+                  float *loss, float *y, float *grad)
+{
+  int rc = ensure_train(h, n);
   if (rc) return rc;
-  const long long m = ((n + 31) / 32) * 32;
-  if (m > n) HIP_TRY(hipMemsetAsync(h->X + n * MLP_IN_PAD, 0, (m - n) * MLP_IN_PAD * sizeof(bf16), h->stream));
-  hipLaunchKernelGGL(pack_input_kernel, dim3(blocks_for(n * MLP_IN_PAD, 256)), dim3(256), 0,
-                     h->stream, x, n, h->n_in, h->X);
-  const bf16 *in = h->X;
-  int K = MLP_IN_PAD;
+  if ((rc = refresh_frags(h, false))) return rc;
+  // 16 rows to a block up to two blocks per CU, where a block's latency counts
+  // (256 x 4: 4096 rows 73 us, 77 with 32; 128 x 4: 8192 rows 64, 68); above, the
+  // MFMAs' second half is worth having (256 x 4: 16384 rows 134, 141; 65536 378, 412).
+  // (64 rows, two tiles sharing each weight fragment: within 2 % of 32.)
+  const int rows = n <= 32ll * h->num_cu ? 16 : 32;
+  const long long row_blocks = (n + rows - 1) / rows;
+  TrainArgs a{};
+  a.x = x; a.t = t; a.w = w; a.n = n;
+  a.n_in = h->n_in; a.n_out = h->n_out; a.layers = h->layers;
+  a.Xf = h->Xf; a.dYf = h->dYf; a.y = y; a.loss_part = h->loss_part;
+  a.grad = grad ? grad : h->G;
+  a.n_grad = grad ? h->n_packed : h->n_pad;
+  WeightArgs g{};
+  int blocks = 0;
+  long long packed = 0;
   for (int i = 0; i <= h->layers; ++i) {
     const MlpLayer &ly = h->L[i];
-    GemmArgs g{};
-    g.A = in; g.sAm = K; g.sAk = 1;
-    g.B = h->Pbf + ly.w_off; g.sBk = ly.N; g.sBn = 1;
-    g.M = (int)m; g.N = ly.N; g.K = ly.K; g.ksplit = 1; g.ldc = ly.N;
-    g.bias = h->P + ly.b_off;
+    a.Wf[i] = h->Wsw + ly.sw_off;
+    a.Wb[i] = h->Wb + ly.sw_off;
+    a.bias[i] = h->P + ly.b_off;
     if (i < h->layers) {
-      g.mode = EPI_BIAS_GELU; g.Z = h->Z[i]; g.H = h->H[i];
-    } else {
-      g.mode = EPI_BIAS; g.C = h->Yb;
+      a.Hf[i] = h->Hf[i]; a.dZf[i] = h->dZf[i]; a.gz[i] = h->gz[i];
     }
-    if ((rc = launch_gemm(h, g))) return rc;
-    in = h->H[i < h->layers ? i : 0];
-    K = ly.N;
+    WeightLayer &q = g.L[i];
+    q.A = i > 0 ? h->Hf[i - 1] : h->Xf;
+    q.B = i < h->layers ? h->dZf[i] : h->dYf;
+    q.MT = ly.K / 32; q.NT = ly.N / 32;
+    q.block0 = blocks;
+    blocks += ((q.MT + 1) / 2) * ((q.NT + 1) / 2);
+    q.K = grad ? ly.Kr : ly.K; q.N = grad ? ly.Nr : ly.N;
+    q.dW = a.grad + packed;
+    q.db = q.dW + (long long)q.K * q.N;
+    packed += (long long)q.K * q.N + q.N;
   }
-  return NRG_CHEM_OK;
-}
-
-// Backward into h->G (padded layout); dY already in h->dY.
-int backward(nrg_mlp_t *h, long long n)
-{
-  const long long m = ((n + 31) / 32) * 32;
-  if (m > n) HIP_TRY(hipMemsetAsync(h->dY + n * MLP_OUT_PAD, 0, (m - n) * MLP_OUT_PAD * sizeof(bf16), h->stream));
-  hipLaunchKernelGGL(fill_f32_kernel, dim3(blocks_for(h->n_pad, 256)), dim3(256), 0, h->stream,
-                     h->G, h->n_pad, 0.0f);
-  const bf16 *dZ = h->dY;
-  int cur = 0;
-  int rc;
-  const int ksplit = (int)std::max<long long>(1, std::min<long long>(64, m / 512));
-  for (int i = h->layers; i >= 0; --i) {
-    const MlpLayer &ly = h->L[i];
-    const bf16 *Hin = i > 0 ? h->H[i - 1] : h->X;
-    const int Kin = ly.K;
-    // dW = Hin^T dZ   (Kin x N, reduction over the batch)
-    GemmArgs g{};
-    g.A = Hin; g.sAm = 1; g.sAk = Kin;
-    g.B = dZ; g.sBk = ly.N; g.sBn = 1;
-    g.M = Kin; g.N = ly.N; g.K = (int)m; g.mode = EPI_STORE; g.ksplit = ksplit; g.ldc = ly.N;
-    g.C = h->G + ly.w_off;
-    if ((rc = launch_gemm(h, g))) return rc;
-    hipLaunchKernelGGL(bias_grad_kernel, dim3(blocks_for(ly.N, 256), (unsigned)blocks_for(m, 256)),
-                       dim3(256), 0, h->stream, dZ, m, ly.N, h->G + ly.b_off);
-    if (i == 0) break;
-    // dZ_{i-1} = (dZ W^T) * gelu'(Z_{i-1})
-    GemmArgs b{};
-    b.A = dZ; b.sAm = ly.N; b.sAk = 1;
-    b.B = h->Pbf + ly.w_off; b.sBk = 1; b.sBn = ly.N;
-    b.M = (int)m; b.N = Kin; b.K = ly.N; b.mode = EPI_GELU_BACK; b.ksplit = 1; b.ldc = Kin;
-    b.Zin = h->Z[i - 1]; b.H = h->dZ[cur];
-    if ((rc = launch_gemm(h, b))) return rc;
-    dZ = h->dZ[cur];
-    cur ^= 1;
+  switch (h->hidden) {
+    case 64: launch_rows<2>(h, a, row_blocks, rows); break;
+    case 128: launch_rows<4>(h, a, row_blocks, rows); break;
+    case 256: launch_rows<8>(h, a, row_blocks, rows); break;
+    default: return set_error(NRG_CHEM_E_ARG, "hidden width %d has no training kernel", h->hidden);
   }
+  g.layers = h->layers + 1;
+  g.kblocks = row_blocks * (rows / 16);
+  // Ranges of the rows: at least 512 rows each, and no more than fill the chip,
+  // since every range adds its sums to G (256 x 4, 16384 rows: 32 ranges 134 us, 8
+  // of them 122).
+  const long long ksplit = std::max<long long>(1, std::min<long long>(n / 512, 2 * h->num_cu / blocks));
+  g.kper = (g.kblocks + ksplit - 1) / ksplit;
+  g.loss_part = h->loss_part; g.n_part = row_blocks; g.loss = loss;
+  hipLaunchKernelGGL(train_weights_kernel, dim3((unsigned)blocks, (unsigned)((g.kblocks + g.kper - 1) / g.kper)),
+                     dim3(256), 0, h->stream, g);
   HIP_TRY(hipGetLastError());
   return NRG_CHEM_OK;
-}
-
-int loss_and_grad(nrg_mlp_t *h, long long n, const float *x, const float *t, const float *w,
-                  float *loss)
-{
-  int rc = forward_train(h, n, x);
-  if (rc) return rc;
-  if (loss) hipLaunchKernelGGL(fill_f32_kernel, dim3(1), dim3(64), 0, h->stream, loss, 1, 0.0f);
-  hipLaunchKernelGGL(loss_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, h->stream, h->Yb, t, w,
-                     n, h->n_out, h->dY, loss);
-  return backward(h, n);
 }
 
 }  // namespace
@@ -731,7 +916,7 @@ int loss_and_grad(nrg_mlp_t *h, long long n, const float *x, const float *t, con
 int mlp_infer_bf16(nrg_mlp_t *h, long long n, const bf16 *X, float *Y, hipStream_t stream)
 {
   if (n <= 0) return NRG_CHEM_OK;
-  int rc = refresh_swizzle(h);
+  int rc = refresh_frags(h, true);
   if (rc) return rc;
   InferArgs a{};
   a.X = X; a.n = n; a.n_out = h->n_out; a.hidden = h->hidden; a.layers = h->layers; a.Y = Y;
@@ -785,6 +970,7 @@ int nrg_mlp_create(int32_t n_in, int32_t n_hidden, int32_t n_layers, int32_t n_o
   nrg_mlp_t *h = new (std::nothrow) nrg_mlp();
   if (!h) return set_error(NRG_CHEM_E_ARG, "out of host memory");
   h->device = device;
+  h->num_cu = prop.multiProcessorCount;
   h->n_in = n_in; h->hidden = n_hidden; h->layers = n_layers; h->n_out = n_out;
   long long off = 0, sw = 0, packed = 0;
   for (int i = 0; i <= n_layers; ++i) {
@@ -806,18 +992,8 @@ int nrg_mlp_create(int32_t n_in, int32_t n_hidden, int32_t n_layers, int32_t n_o
   const size_t fb = h->n_pad * sizeof(float);
   if (hipMalloc(&h->P, fb) || hipMalloc(&h->G, fb) || hipMalloc(&h->M1, fb) || hipMalloc(&h->M2, fb) ||
       hipMalloc(&h->Pbf, h->n_pad * sizeof(bf16)) || hipMalloc(&h->Wsw, h->n_sw * sizeof(bf16)) ||
-      hipMalloc(&h->WswT, h->n_sw * sizeof(bf16)) ||
-      hipMalloc(&h->gidx, h->n_packed * sizeof(int)) || hipMalloc(&h->loss_tmp, sizeof(float)))
+      hipMalloc(&h->Wb, h->n_sw * sizeof(bf16)) || hipMalloc(&h->WswT, h->n_sw * sizeof(bf16)))
     return fail(set_error(NRG_CHEM_E_HIP, "hipMalloc parameters"));
-  std::vector<int> gi;
-  gi.reserve(h->n_packed);
-  for (const MlpLayer &ly : h->L) {
-    for (int k = 0; k < ly.Kr; ++k)
-      for (int n = 0; n < ly.Nr; ++n) gi.push_back((int)(ly.w_off + (long long)k * ly.N + n));
-    for (int n = 0; n < ly.Nr; ++n) gi.push_back((int)(ly.b_off + n));
-  }
-  if (hipMemcpy(h->gidx, gi.data(), gi.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
-    return fail(set_error(NRG_CHEM_E_HIP, "hipMemcpy index map"));
   std::vector<float> zero(h->n_packed, 0.0f);
   int rc = nrg_mlp_set_params(h, zero.data());
   if (rc) return fail(rc);
@@ -830,12 +1006,8 @@ void nrg_mlp_destroy(nrg_mlp_t *h)
   if (!h) return;
   (void)hipSetDevice(h->device);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  for (void *p : {(void *)h->P, (void *)h->G, (void *)h->M1, (void *)h->M2, (void *)h->Pbf,
-                  (void *)h->Wsw, (void *)h->WswT, (void *)h->gidx, (void *)h->loss_tmp, (void *)h->X, (void *)h->dY,
-                  (void *)h->Yb, (void *)h->dZ[0], (void *)h->dZ[1]})
-    if (p) (void)hipFree(p);
-  for (auto p : h->H) if (p) (void)hipFree(p);
-  for (auto p : h->Z) if (p) (void)hipFree(p);
+  free_all({h->P, h->G, h->M1, h->M2, h->Pbf, h->Wsw, h->Wb, h->WswT, h->X});
+  free_train(h);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
@@ -902,13 +1074,8 @@ int nrg_mlp_grad_dev(nrg_mlp_t *h, int64_t n, const float *x, const float *t, co
 {
   if (!h || n <= 0 || !x || !t || !grad) return set_error(NRG_CHEM_E_ARG, "bad argument");
   HIP_TRY(hipSetDevice(h->device));
-  int rc = loss_and_grad(h, n, x, t, w, loss);
+  int rc = loss_and_grad(h, n, x, t, w, loss, y_out, grad);
   if (rc) return rc;
-  hipLaunchKernelGGL(gather_kernel, dim3(blocks_for(h->n_packed, 256)), dim3(256), 0, h->stream,
-                     h->G, h->gidx, grad, h->n_packed);
-  if (y_out)
-    HIP_TRY(hipMemcpy2DAsync(y_out, h->n_out * sizeof(float), h->Yb, MLP_OUT_PAD * sizeof(float),
-                             h->n_out * sizeof(float), n, hipMemcpyDeviceToDevice, h->stream));
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(h->stream));
   return NRG_CHEM_OK;
@@ -919,7 +1086,7 @@ int nrg_mlp_train_step_dev(nrg_mlp_t *h, int64_t n, const float *x, const float 
 {
   if (!h || n <= 0 || !x || !t) return set_error(NRG_CHEM_E_ARG, "bad argument");
   HIP_TRY(hipSetDevice(h->device));
-  int rc = loss_and_grad(h, n, x, t, w, loss);
+  int rc = loss_and_grad(h, n, x, t, w, loss, nullptr, nullptr);
   if (rc) return rc;
   h->adam_t += 1;
   const float bc1 = 1.0f - std::pow(0.9f, (float)h->adam_t);
@@ -927,8 +1094,8 @@ int nrg_mlp_train_step_dev(nrg_mlp_t *h, int64_t n, const float *x, const float 
   hipLaunchKernelGGL(adam_kernel, dim3(blocks_for(h->n_pad, 256)), dim3(256), 0, h->stream, h->P,
                      h->Pbf, h->G, h->M1, h->M2, h->n_pad, lr, bc1, bc2);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipStreamSynchronize(h->stream));
   h->sw_dirty = true;
+  HIP_TRY(hipStreamSynchronize(h->stream));
   return NRG_CHEM_OK;
 }
 

@@ -91,6 +91,44 @@ def test_gradients_match_reference():
     net.close()
 
 
+@pytest.mark.parametrize("n,dims", [(1, (12, 64, 1, 10)), (17, (1, 128, 2, 1)), (33, (32, 256, 7, 32)),
+                                    (64, (12, 64, 3, 10)), (4095, (12, 256, 2, 10)), (8192, (5, 128, 1, 32)),
+                                    (8193, (12, 64, 2, 10)), (8240, (32, 256, 1, 3))])
+def test_gradients_at_the_edges_of_the_row_tiles(n, dims):
+    """Row counts around the blocks' 16 rows (32 above 8192) and the split of the
+    rows; every hidden width; narrowest and widest input and output; without
+    weights, too.  The bars of the tests above, and two calls agree to the order
+    of the row sums (1e-4)."""
+    import torch
+    from nrg_amd.surrogate import MLP, init_params
+    net = MLP(dims[0], dims[3], dims[1], dims[2])
+    rng = np.random.default_rng(n)
+    p = init_params(dims[0], dims[3], dims[1], dims[2], seed=n)
+    p = p + rng.normal(0, 0.05, p.size).astype(np.float32) * (p == 0)
+    net.set_params(p)
+    x = rng.normal(size=(n, dims[0])).astype(np.float32)
+    t = rng.normal(size=(n, dims[3])).astype(np.float32)
+    w = rng.uniform(0.5, 2.0, dims[3]).astype(np.float32)
+    cu = lambda v: torch.as_tensor(v, device="cuda:0")  # noqa: E731
+    rel = lambda a, b: float(np.linalg.norm(a - b) / np.linalg.norm(b))  # noqa: E731
+    for weights in (w, None):
+        g, loss, y = net.grad(cu(x), cu(t), None if weights is None else cu(weights))
+        l_ref, g_ref, _ = M.loss_and_grad(p.astype(np.float64), dims, x.astype(np.float64), t.astype(np.float64),
+                                          np.ones(dims[3]) if weights is None else weights.astype(np.float64),
+                                          bf16=True)
+        y_ref, _ = M.forward(p.astype(np.float64), dims, x.astype(np.float64), bf16=True)
+        g = g.cpu().numpy().astype(np.float64)
+        _report("edges", n=n, dims=dims, loss=float(loss.item()) / l_ref - 1.0, grad=rel(g, g_ref),
+                y=rel(y.cpu().numpy(), y_ref))
+        assert float(loss.item()) == pytest.approx(l_ref, rel=5e-3)
+        assert rel(y.cpu().numpy(), y_ref) <= 5e-3
+        assert rel(g, g_ref) <= 2e-2 and float(g @ g_ref / (np.linalg.norm(g) * np.linalg.norm(g_ref))) >= 0.999
+        again = net.grad(cu(x), cu(t), None if weights is None else cu(weights))
+        assert rel(again[0].cpu().numpy().astype(np.float64), g) <= 1e-4
+        assert torch.equal(again[2], y)
+    net.close()
+
+
 def test_adam_training_reduces_loss():
     """Fit a smooth 12 -> 10 map; 400 Adam steps on the GPU kernels."""
     import torch
