@@ -25,6 +25,7 @@ namespace nrg {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int WAVE = 64;
@@ -336,16 +337,6 @@ __global__ void fill_f32_kernel(float *p, long long n, float v)
   if (i < n) p[i] = v;
 }
 
-// x (n x n_in FP32) -> X (n x 32 bf16, zero padded)
-__global__ void pack_input_kernel(const float *x, long long n, int n_in, bf16 *X)
-{
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * MLP_IN_PAD) return;
-  const long long row = i / MLP_IN_PAD;
-  const int c = (int)(i % MLP_IN_PAD);
-  X[i] = (bf16)(c < n_in ? x[row * n_in + c] : 0.0f);
-}
-
 __global__ void adam_kernel(float *P, bf16 *Pbf, const float *G, float *M1, float *M2, long long n,
                             float lr, float bc1, float bc2)
 {
@@ -368,200 +359,34 @@ __global__ void to_bf16_kernel(const float *P, bf16 *Pbf, long long n)
   if (i < n) Pbf[i] = (bf16)P[i];
 }
 
-// ---- fused inference: all layers, 32 rows per wave, 128 rows per block -----------
-// Hidden activations of a wave's rows stay in LDS as bf16 between layers;
-// weights stream from L2 as pre-swizzled B fragments.
-constexpr int ACT_LD = MLP_HIDDEN_MAX + 8;   // row pitch (bf16): 16 B skew against bank conflicts
-
+// ---- fused inference -------------------------------------------------------------
+// All layers in one kernel, computed transposed, Z^T = W^T H^T: the weights are the
+// MFMA A operand (32 output features x 16 inputs) and the activations the B operand
+// (16 inputs x 32 cells).  A wave owns 32 features of every hidden layer; its
+// weights of a layer (up to 16 KB) come from L2 into registers and serve the two
+// 32-cell tiles that a block works on, whose activations pass through LDS.  A
+// lane's accumulator holds, for its cell, features 32 w + 8 q + 4 hi + i (q, i =
+// 0..3, hi = lane/32): four stores of four.  Width 256 keeps a k-block's inputs in
+// the order (8 hi + 4 (q%2) + i of block q/2) that its K rows have in WswT, and the
+// bias as the accumulators' start; the others take the natural order and add it.
+//
+// What bounds it is the GELUs' VALU time (two of their seven operations are
+// quarter-rate), which several waves per SIMD overlap with each other's MFMAs and
+// loads.  The blocks share the tiles evenly.  Before, a wave took its cells through
+// all features with the weights staged in LDS (at the narrower widths the
+// activations): few cells left most of the chip idle for a long chain, and 70,001
+// cells were a second, nearly empty round.  Call times, width 256 x 4: 256 cells 56
+// -> 29 us, 16,384 58 -> 35, 70,001 91 -> 61, 262,144 197 -> 187; 128 x 4: 4096 39 ->
+// 26, 262,144 130 -> 99; 64 x 3: 4096 31 -> 25, 262,144 72 -> 50.
 struct InferArgs {
-  const bf16 *X;               // n x 32
+  const bf16 *X;               // n x 32, or NULL:
+  const float *x;              // n x n_in
   long long n;
-  int n_out;
-  int hidden, layers;          // hidden width (multiple of 32, <= MLP_HIDDEN_MAX), hidden layers
-  const bf16 *Wsw[MLP_MAX_LAYERS];
+  int n_in, n_out, layers;     // layers: hidden layers
+  const bf16 *W[MLP_MAX_LAYERS];     // WswT (width 256) or Wsw
   const float *bias[MLP_MAX_LAYERS];
   float *Y;                    // n x n_out
 };
-
-template <int NT>
-__device__ __forceinline__ void act_store(bf16 (*act)[ACT_LD], const f32x16 (&acc)[NT],
-                                          const float *bias, int lane)
-{
-  const int r32 = lane & 31, hi = lane >> 5;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = 8 * (r / 4) + 4 * hi + (r % 4), col = 32 * nt + r32;
-      act[row][col] = (bf16)gelu(acc[nt][r] + bias[col]);
-    }
-}
-
-template <int NT>
-__global__ void __launch_bounds__(256) mlp_infer_kernel(InferArgs a)
-{
-  __shared__ bf16 act_all[4][32][ACT_LD];
-  const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
-  const int r32 = l & 31, hi = l >> 5;
-  bf16 (*act)[ACT_LD] = act_all[w];
-  const long long row0 = (long long)blockIdx.x * 128 + w * 32;
-  const long long myrow = row0 + r32 < a.n ? row0 + r32 : a.n - 1;
-
-  f32x16 acc[NT];
-  // layer 0: K = 32 (two k-blocks) from the packed input
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x16{};
-#pragma unroll
-  for (int kb = 0; kb < MLP_IN_PAD / 16; ++kb) {
-    const bf16x8 av = *reinterpret_cast<const bf16x8 *>(a.X + myrow * MLP_IN_PAD + 16 * kb + 8 * hi);
-    const bf16x8 *Wb = reinterpret_cast<const bf16x8 *>(a.Wsw[0]) + (kb * NT) * WAVE + l;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma(av, Wb[nt * WAVE], acc[nt]);
-  }
-  act_store<NT>(act, acc, a.bias[0], l);
-  __syncthreads();
-
-  // hidden layers: K = N = hidden
-  for (int layer = 1; layer < a.layers; ++layer) {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x16{};
-    const bf16x8 *W = reinterpret_cast<const bf16x8 *>(a.Wsw[layer]);
-    for (int kb = 0; kb < NT * 2; ++kb) {
-      const bf16x8 av = *reinterpret_cast<const bf16x8 *>(&act[r32][16 * kb + 8 * hi]);
-      const bf16x8 *Wb = W + (kb * NT) * WAVE + l;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma(av, Wb[nt * WAVE], acc[nt]);
-    }
-    __syncthreads();
-    act_store<NT>(act, acc, a.bias[layer], l);
-    __syncthreads();
-  }
-
-  // output layer: K = hidden, N = 32 (padded)
-  f32x16 o = {};
-  const bf16x8 *Wo = reinterpret_cast<const bf16x8 *>(a.Wsw[a.layers]);
-  for (int kb = 0; kb < NT * 2; ++kb) {
-    const bf16x8 av = *reinterpret_cast<const bf16x8 *>(&act[r32][16 * kb + 8 * hi]);
-    o = mfma(av, Wo[kb * WAVE + l], o);
-  }
-  const float *bo = a.bias[a.layers];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const long long row = row0 + 8 * (r / 4) + 4 * hi + (r % 4);
-    if (r32 < a.n_out && row < a.n) a.Y[row * a.n_out + r32] = o[r] + bo[r32];
-  }
-}
-
-// Inference, hidden width 32*NT with staged weights: 64 rows per wave (two
-// 32-row MFMA tiles share every B fragment), 256 rows per block, and each
-// 16-row k-block of a hidden layer's weights copied once per block into a
-// double-buffered LDS slot that the four waves read.  The per-tile
-// accumulation order equals mlp_infer_kernel's, so the results are identical.
-constexpr int ROWS2 = 64;
-
-template <int NT>
-__global__ void __launch_bounds__(256) mlp_infer2_kernel(InferArgs a)
-{
-  __shared__ bf16 act_all[4][ROWS2][ACT_LD];
-  __shared__ bf16x8 wbuf[2][NT * WAVE];
-  const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
-  const int r32 = l & 31, hi = l >> 5;
-  bf16 (*act)[ACT_LD] = act_all[w];
-  const long long row0 = (long long)blockIdx.x * (4 * ROWS2) + w * ROWS2;
-  const long long ra = row0 + r32 < a.n ? row0 + r32 : a.n - 1;
-  const long long rb = row0 + 32 + r32 < a.n ? row0 + 32 + r32 : a.n - 1;
-
-  f32x16 acc[2][NT];
-  // layer 0: K = 32 from the packed input; its B fragments (16 KB) from L2
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) acc[0][nt] = acc[1][nt] = f32x16{};
-#pragma unroll
-  for (int kb = 0; kb < MLP_IN_PAD / 16; ++kb) {
-    const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(a.X + ra * MLP_IN_PAD + 16 * kb + 8 * hi);
-    const bf16x8 a1 = *reinterpret_cast<const bf16x8 *>(a.X + rb * MLP_IN_PAD + 16 * kb + 8 * hi);
-    const bf16x8 *Wb = reinterpret_cast<const bf16x8 *>(a.Wsw[0]) + (kb * NT) * WAVE + l;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const bf16x8 b = Wb[nt * WAVE];
-      acc[0][nt] = mfma(a0, b, acc[0][nt]);
-      acc[1][nt] = mfma(a1, b, acc[1][nt]);
-    }
-  }
-  act_store<NT>(act, acc[0], a.bias[0], l);
-  act_store<NT>(act + 32, acc[1], a.bias[0], l);
-  __syncthreads();
-
-  constexpr int NV = NT * WAVE;            // bf16x8 vectors per k-block
-  static_assert(NV % 256 == 0, "k-block staging assumes whole vectors per thread");
-  for (int layer = 1; layer < a.layers; ++layer) {
-    const bf16x8 *W = reinterpret_cast<const bf16x8 *>(a.Wsw[layer]);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[0][nt] = acc[1][nt] = f32x16{};
-#pragma unroll
-    for (int v = 0; v < NV / 256; ++v) wbuf[0][v * 256 + threadIdx.x] = W[v * 256 + threadIdx.x];
-    __syncthreads();
-    for (int kb = 0; kb < NT * 2; ++kb) {
-      bf16x8 nxt[NV / 256];
-      const bool more = kb + 1 < NT * 2;
-      if (more) {
-#pragma unroll
-        for (int v = 0; v < NV / 256; ++v) nxt[v] = W[(kb + 1) * NV + v * 256 + threadIdx.x];
-      }
-      const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(&act[r32][16 * kb + 8 * hi]);
-      const bf16x8 a1 = *reinterpret_cast<const bf16x8 *>(&act[32 + r32][16 * kb + 8 * hi]);
-      const bf16x8 *Wb = wbuf[kb & 1] + l;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const bf16x8 b = Wb[nt * WAVE];
-        acc[0][nt] = mfma(a0, b, acc[0][nt]);
-        acc[1][nt] = mfma(a1, b, acc[1][nt]);
-      }
-      if (more) {
-#pragma unroll
-        for (int v = 0; v < NV / 256; ++v) wbuf[(kb + 1) & 1][v * 256 + threadIdx.x] = nxt[v];
-      }
-      __syncthreads();
-    }
-    act_store<NT>(act, acc[0], a.bias[layer], l);
-    act_store<NT>(act + 32, acc[1], a.bias[layer], l);
-    __syncthreads();
-  }
-
-  // output layer: K = hidden, N = 32 (padded); its fragments (16 KB) from L2
-  f32x16 o0 = {}, o1 = {};
-  const bf16x8 *Wo = reinterpret_cast<const bf16x8 *>(a.Wsw[a.layers]);
-  for (int kb = 0; kb < NT * 2; ++kb) {
-    const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(&act[r32][16 * kb + 8 * hi]);
-    const bf16x8 a1 = *reinterpret_cast<const bf16x8 *>(&act[32 + r32][16 * kb + 8 * hi]);
-    const bf16x8 b = Wo[kb * WAVE + l];
-    o0 = mfma(a0, b, o0);
-    o1 = mfma(a1, b, o1);
-  }
-  const float *bo = a.bias[a.layers];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const long long row = row0 + 8 * (r / 4) + 4 * hi + (r % 4);
-    if (r32 < a.n_out && row < a.n) a.Y[row * a.n_out + r32] = o0[r] + bo[r32];
-    if (r32 < a.n_out && row + 32 < a.n) a.Y[(row + 32) * a.n_out + r32] = o1[r] + bo[r32];
-  }
-}
-
-// ---- inference with the activations in registers ---------------------------------
-// Each layer is computed transposed, Z^T = W^T H^T: the weights are the MFMA A
-// operand (32 output features x 16 inputs) and the activations the B operand
-// (16 inputs x 32 cells).  A lane's accumulator then holds, for its cell, the
-// output features 32 mt + 8 (r/4) + 4 hi + r%4 (r = 0..15, hi = lane/32): after
-// bias and GELU, elements r = 0..7 and 8..15 are exactly the lane's B fragments
-// of k-blocks 2 mt and 2 mt + 1 of the next layer, provided that layer's
-// weights are stored with their K rows in that order (swizzle_t_kernel).  So
-// hidden activations never leave the registers; the hidden layers' weights
-// (H x H bf16, 128 KB at H = 256) are staged in LDS once per layer and block.
-#ifndef T_NC
-#define T_NC 1                      // 32-cell tiles per wave (they share each A fragment)
-#endif
-#ifndef T_WPB
-#define T_WPB 8                     // waves per block: two per SIMD, so one wave's GELUs
-#endif                              // overlap the other's MFMAs
 
 // physical feature (output column of the previous layer) of logical K row kl
 __host__ __device__ inline int t_phys(int kl)
@@ -609,122 +434,126 @@ __global__ void __launch_bounds__(256) frag_kernel(FragArgs a)
   *reinterpret_cast<bf16x8 *>(a.WswT + i) = tr;
 }
 
-// Accumulator start value: the bias of the lane's 16 output features of tile mt
-// (so the epilogue needs no separate add).
-__device__ __forceinline__ f32x16 t_bias(const float *bias, int mt, int hi)
-{
-  f32x16 b;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) b[r] = bias[32 * mt + 8 * (r / 4) + 4 * hi + r % 4];
-  return b;
-}
+// Resident waves per SIMD, and the 32-cell tiles a block takes through the layers
+// together: two waves with up to 256 registers (a tile's fragments and a layer's
+// weights in flight at once; 262,144 cells at width 256 186 us, 298 with four waves,
+// which spill; at 128 99 and 104), but four at width 64 (50 us, 57 with two).
+constexpr int infer_waves(int nt) { return nt >= 4 ? 2 : 4; }
+constexpr int infer_tiles(int nt) { return nt >= 4 ? 4 : 2; }
 
-// GELU of one 32-feature tile, packed as the next layer's two B fragments
-__device__ __forceinline__ void t_epilogue(const f32x16 &acc, bf16x8 &lo, bf16x8 &up)
+template <int NT>
+__global__ void __launch_bounds__(NT * 64) __attribute__((amdgpu_waves_per_eu(infer_waves(NT), infer_waves(NT))))
+mlp_infer_kernel(InferArgs a)
 {
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const bf16 g = (bf16)gelu(acc[r]);
-    if (r < 8)
-      lo[r] = g;
-    else
-      up[r - 8] = g;
-  }
-}
-
-// NC 32-cell tiles per wave, WPB waves per block.
-template <int NT, int NC, int WPB>
-__global__ void __launch_bounds__(WPB * 64) mlp_infer_t_kernel(InferArgs a)
-{
-  constexpr int KB = 2 * NT;                      // k-blocks of a hidden layer
-  constexpr int NTHR = WPB * WAVE;
-  __shared__ bf16x8 wl[NT * KB * WAVE];           // one hidden layer's A fragments
-  __shared__ float bl[32 * NT];                   // its bias
+  constexpr bool PERM = NT == 8;
+  constexpr int KB = 2 * NT, LD = 32 * NT + 8, TILES = infer_tiles(NT);
+  __shared__ __align__(16) bf16 act[2][32 * TILES][LD];
   const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
   const int r32 = l & 31, hi = l >> 5;
-  const long long cell0 = ((long long)blockIdx.x * WPB + w) * (32 * NC);
-
-  bf16x8 h[KB][NC];
-  // layer 0 (K = 32): input B fragments straight from X, weights from L2
-  {
-    bf16x8 x[2][NC];
+  const long long T = (a.n + 31) / 32;
+  const long long t0 = T * blockIdx.x / gridDim.x, t1 = T * (blockIdx.x + 1) / gridDim.x;
+  const int groups = (int)((t1 - t0 + TILES - 1) / TILES);
+  // fragment kb of feature tile mt of a layer with nt feature tiles and kbs k-blocks
+  auto weight = [&](int layer, int mt, int nt, int kb, int kbs) {
+    return reinterpret_cast<const bf16x8 *>(a.W[layer])[(PERM ? mt * kbs + kb : kb * nt + mt) * WAVE + l];
+  };
+  bf16x8 W[KB];
+  auto weights = [&](int layer) {
 #pragma unroll
-    for (int ct = 0; ct < NC; ++ct) {
-      const long long c = cell0 + 32 * ct + r32 < a.n ? cell0 + 32 * ct + r32 : a.n - 1;
+    for (int kb = 0; kb < KB; ++kb) W[kb] = weight(layer, w, NT, kb, KB);
+  };
+  auto biases = [&](int layer, int mt) {
+    f32x16 b;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) b[r] = a.bias[layer][32 * mt + acc_row(r, hi)];
+    return b;
+  };
+  auto store = [&](int buf, int tile, const f32x16 &acc, const f32x16 &bias) {
+    bf16 *d = &act[buf][32 * tile + r32][32 * w];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bf16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (bf16)gelu(PERM ? acc[4 * q + i] : acc[4 * q + i] + bias[4 * q + i]);
+      *reinterpret_cast<bf16x4 *>(d + (PERM ? 16 * (q / 2) + 8 * hi + 4 * (q % 2) : 8 * q + 4 * hi)) = v;
+    }
+  };
+  for (int g = 0; g < groups; ++g) {
+    const long long tile = t0 + (t1 - t0) * g / groups;
+    const int nt = (int)(t0 + (t1 - t0) * (g + 1) / groups - tile);
+    // the input: packed in memory, or converted into the second buffer
+    if (!a.X) {
+      for (int i = threadIdx.x; i < 32 * nt * MLP_IN_PAD; i += NT * WAVE) {
+        const int row = i / MLP_IN_PAD, c = i % MLP_IN_PAD;
+        const long long cell = 32 * tile + row < a.n ? 32 * tile + row : a.n - 1;
+        act[1][row][c] = (bf16)(c < a.n_in ? a.x[cell * a.n_in + c] : 0.0f);
+      }
+    }
+    f32x16 bias = biases(0, w);
+    const bf16x8 W0[2] = {weight(0, w, NT, 0, 2), weight(0, w, NT, 1, 2)};
+    if (!a.X) lds_barrier();
+    for (int t = 0; t < nt; ++t) {
+      const long long cell = 32 * (tile + t) + r32 < a.n ? 32 * (tile + t) + r32 : a.n - 1;
+      bf16x8 x[2];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
-        x[kb][ct] = *reinterpret_cast<const bf16x8 *>(a.X + c * MLP_IN_PAD + 16 * kb + 8 * hi);
+        if (a.X)
+          x[kb] = *reinterpret_cast<const bf16x8 *>(a.X + cell * MLP_IN_PAD + 16 * kb + 8 * hi);
+        else
+          x[kb] = *reinterpret_cast<const bf16x8 *>(&act[1][32 * t + r32][16 * kb + 8 * hi]);
+      f32x16 acc = PERM ? bias : f32x16{};
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) acc = mfma(W0[kb], x[kb], acc);
+      if (t == nt - 1 && a.layers > 1) weights(1);
+      store(0, t, acc, bias);
     }
-    const bf16x8 *W0 = reinterpret_cast<const bf16x8 *>(a.Wsw[0]);
+    for (int layer = 1; layer < a.layers; ++layer) {
+      bias = biases(layer, w);
+      lds_barrier();
+      auto product = [&](int t) {
+        const bf16 *in = &act[(layer - 1) & 1][32 * t + r32][8 * hi];
+        f32x16 acc = PERM ? bias : f32x16{};
+        if (NT >= 4) {                           // all loads ahead
+          bf16x8 f[KB];
 #pragma unroll
-    for (int mt = 0; mt < NT; ++mt) {
-      const f32x16 b = t_bias(a.bias[0], mt, hi);
-      f32x16 acc[NC];
+          for (int kb = 0; kb < KB; ++kb) f[kb] = *reinterpret_cast<const bf16x8 *>(in + 16 * kb);
 #pragma unroll
-      for (int ct = 0; ct < NC; ++ct) acc[ct] = b;
+          for (int kb = 0; kb < KB; ++kb) acc = mfma(W[kb], f[kb], acc);
+        } else {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        const bf16x8 A = W0[(mt * 2 + kb) * WAVE + l];
-#pragma unroll
-        for (int ct = 0; ct < NC; ++ct) acc[ct] = mfma(A, x[kb][ct], acc[ct]);
+          for (int kb = 0; kb < KB; ++kb) acc = mfma(W[kb], *reinterpret_cast<const bf16x8 *>(in + 16 * kb), acc);
+        }
+        return acc;
+      };
+      // a tile's product runs beside the GELUs of the one before, the next layer's
+      // weights come during the last one's
+      f32x16 cur = product(0);
+#pragma unroll 1
+      for (int t = 1; t < nt; ++t) {
+        const f32x16 next = product(t);
+        store(layer & 1, t - 1, cur, bias);
+        cur = next;
       }
-#pragma unroll
-      for (int ct = 0; ct < NC; ++ct) t_epilogue(acc[ct], h[2 * mt][ct], h[2 * mt + 1][ct]);
+      if (layer + 1 < a.layers) weights(layer + 1);
+      store(layer & 1, nt - 1, cur, bias);
     }
-  }
-  // hidden layers
-  for (int layer = 1; layer < a.layers; ++layer) {
-    __syncthreads();                               // previous layer's weights no longer read
-    const bf16x8 *W = reinterpret_cast<const bf16x8 *>(a.Wsw[layer]);
-#pragma unroll 4
-    for (int i = threadIdx.x; i < NT * KB * WAVE; i += NTHR) wl[i] = W[i];
-    for (int i = threadIdx.x; i < 32 * NT; i += NTHR) bl[i] = a.bias[layer][i];
-    __syncthreads();
-    bf16x8 hn[KB][NC];
+    lds_barrier();
+#pragma unroll 1
+    for (int t = w; t < nt; t += NT) {           // output layer: a tile to a wave
+      const bf16 *in = &act[(a.layers - 1) & 1][32 * t + r32][8 * hi];
+      bias = biases(a.layers, 0);
+      f32x16 o = PERM ? bias : f32x16{};
 #pragma unroll
-    for (int mt = 0; mt < NT; ++mt) {
-      const f32x16 b = t_bias(bl, mt, hi);
-      f32x16 acc[NC];
+      for (int kb = 0; kb < KB; ++kb)
+        o = mfma(weight(a.layers, 0, 1, kb, KB), *reinterpret_cast<const bf16x8 *>(in + 16 * kb), o);
+      const long long cell = 32 * (tile + t) + r32;
 #pragma unroll
-      for (int ct = 0; ct < NC; ++ct) acc[ct] = b;
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const bf16x8 A = wl[(mt * KB + kb) * WAVE + l];
-#pragma unroll
-        for (int ct = 0; ct < NC; ++ct) acc[ct] = mfma(A, h[kb][ct], acc[ct]);
+      for (int r = 0; r < 16; ++r) {
+        const int f = acc_row(r, hi);
+        if (cell < a.n && f < a.n_out) a.Y[cell * a.n_out + f] = PERM ? o[r] : o[r] + bias[r];
       }
-#pragma unroll
-      for (int ct = 0; ct < NC; ++ct) t_epilogue(acc[ct], hn[2 * mt][ct], hn[2 * mt + 1][ct]);
     }
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int ct = 0; ct < NC; ++ct) h[kb][ct] = hn[kb][ct];
-  }
-  // output layer: one 32-feature tile, weights from L2
-  const bf16x8 *Wo = reinterpret_cast<const bf16x8 *>(a.Wsw[a.layers]);
-  const float *bo = a.bias[a.layers];
-  f32x16 o[NC];
-  {
-    const f32x16 b = t_bias(bo, 0, hi);
-#pragma unroll
-    for (int ct = 0; ct < NC; ++ct) o[ct] = b;
-  }
-#pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
-    const bf16x8 A = Wo[kb * WAVE + l];
-#pragma unroll
-    for (int ct = 0; ct < NC; ++ct) o[ct] = mfma(A, h[kb][ct], o[ct]);
-  }
-#pragma unroll
-  for (int ct = 0; ct < NC; ++ct) {
-    const long long c = cell0 + 32 * ct + r32;
-    if (c >= a.n) continue;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int f = 8 * (r / 4) + 4 * hi + r % 4;
-      if (f < a.n_out) a.Y[c * a.n_out + f] = o[ct][r];
-    }
+    lds_barrier();                               // the next tiles take the activations' place
   }
 }
 
@@ -755,8 +584,6 @@ struct nrg_mlp {
   bool sw_dirty = true;                     // the fragments are older than the weights
   bool sw_synced = true;                    // written and waited for (other streams read them)
   // batch workspace
-  long long cap = 0;
-  nrg::bf16 *X = nullptr;                   // inference: n x 32
   long long train_cap = 0;
   nrg::bf16 *Xf = nullptr, *dYf = nullptr;  // training (TrainArgs)
   float *loss_part = nullptr;
@@ -771,18 +598,6 @@ void free_all(std::initializer_list<void *> ps)
 {
   for (void *p : ps)
     if (p) (void)hipFree(p);
-}
-
-int ensure_batch(nrg_mlp_t *h, long long n)
-{
-  if (n <= h->cap) return NRG_CHEM_OK;
-  free_all({h->X});
-  h->X = nullptr;
-  h->cap = 0;
-  const long long m = ((n + 127) / 128) * 128;
-  HIP_TRY(hipMalloc(&h->X, m * MLP_IN_PAD * sizeof(bf16)));
-  h->cap = m;
-  return NRG_CHEM_OK;
 }
 
 void free_train(nrg_mlp_t *h)
@@ -913,30 +728,34 @@ int loss_and_grad(nrg_mlp_t *h, long long n, const float *x, const float *t, con
 
 }  // namespace
 
-int mlp_infer_bf16(nrg_mlp_t *h, long long n, const bf16 *X, float *Y, hipStream_t stream)
+// X: n x 32 bf16, or NULL with x: n x n_in
+static int launch_infer(nrg_mlp_t *h, long long n, const bf16 *X, const float *x, float *Y, hipStream_t stream)
 {
   if (n <= 0) return NRG_CHEM_OK;
-  int rc = refresh_frags(h, true);
+  int rc = refresh_frags(h, stream != h->stream);
   if (rc) return rc;
   InferArgs a{};
-  a.X = X; a.n = n; a.n_out = h->n_out; a.hidden = h->hidden; a.layers = h->layers; a.Y = Y;
-  const bool transposed = h->hidden == 256;
+  a.X = X; a.x = x; a.n = n; a.n_in = h->n_in; a.n_out = h->n_out; a.layers = h->layers; a.Y = Y;
   for (int i = 0; i <= h->layers; ++i) {
-    a.Wsw[i] = (transposed ? h->WswT : h->Wsw) + h->L[i].sw_off;
+    a.W[i] = (h->hidden == 256 ? h->WswT : h->Wsw) + h->L[i].sw_off;
     a.bias[i] = h->P + h->L[i].b_off;
   }
-  const dim3 grid(blocks_for(n, 128)), block(256);
+  const int nt = h->hidden / 32;
+  const long long resident = (long long)h->num_cu * (4 * infer_waves(nt) / nt);
+  const dim3 grid((unsigned)std::min<long long>((n + 31) / 32, resident)), block(2 * h->hidden);
   switch (h->hidden) {
     case 64: hipLaunchKernelGGL(mlp_infer_kernel<2>, grid, block, 0, stream, a); break;
     case 128: hipLaunchKernelGGL(mlp_infer_kernel<4>, grid, block, 0, stream, a); break;
-    case 256:
-      hipLaunchKernelGGL((mlp_infer_t_kernel<8, T_NC, T_WPB>), dim3(blocks_for(n, 32 * T_NC * T_WPB)),
-                         dim3(64 * T_WPB), 0, stream, a);
-      break;
+    case 256: hipLaunchKernelGGL(mlp_infer_kernel<8>, grid, block, 0, stream, a); break;
     default: return set_error(NRG_CHEM_E_ARG, "hidden width %d has no inference kernel", h->hidden);
   }
   HIP_TRY(hipGetLastError());
   return NRG_CHEM_OK;
+}
+
+int mlp_infer_bf16(nrg_mlp_t *h, long long n, const bf16 *X, float *Y, hipStream_t stream)
+{
+  return launch_infer(h, n, X, nullptr, Y, stream);
 }
 
 hipStream_t mlp_stream(nrg_mlp_t *h) { return h->stream; }
@@ -1006,7 +825,7 @@ void nrg_mlp_destroy(nrg_mlp_t *h)
   if (!h) return;
   (void)hipSetDevice(h->device);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  free_all({h->P, h->G, h->M1, h->M2, h->Pbf, h->Wsw, h->Wb, h->WswT, h->X});
+  free_all({h->P, h->G, h->M1, h->M2, h->Pbf, h->Wsw, h->Wb, h->WswT});
   free_train(h);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
@@ -1060,11 +879,8 @@ int nrg_mlp_forward_dev(nrg_mlp_t *h, int64_t n, const float *x, float *y)
   if (!h || (n > 0 && (!x || !y)) || n < 0) return set_error(NRG_CHEM_E_ARG, "bad argument");
   if (n == 0) return NRG_CHEM_OK;
   HIP_TRY(hipSetDevice(h->device));
-  int rc = ensure_batch(h, n);
+  const int rc = launch_infer(h, n, nullptr, x, y, h->stream);
   if (rc) return rc;
-  hipLaunchKernelGGL(pack_input_kernel, dim3(blocks_for(n * MLP_IN_PAD, 256)), dim3(256), 0,
-                     h->stream, x, n, h->n_in, h->X);
-  if ((rc = mlp_infer_bf16(h, n, h->X, y, h->stream))) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
   return NRG_CHEM_OK;
 }

@@ -63,6 +63,29 @@ def test_forward_matches_reference(n):
     net.close()
 
 
+@pytest.mark.parametrize("n,dims", [(1, (1, 64, 1, 1)), (33, (32, 128, 7, 32)), (8191, (12, 256, 2, 10)),
+                                    (8193, (12, 128, 4, 10)), (32769, (12, 256, 3, 10)), (65537, (5, 64, 3, 3))])
+def test_forward_at_the_edges_of_the_tiles(n, dims):
+    """Cell counts around a tile, a tile and a group of tiles to every block, at
+    every width: against the reference (the bar of the test above), and bit for
+    bit what the last cells give alone."""
+    import torch
+    from nrg_amd.surrogate import MLP, init_params
+    net = MLP(dims[0], dims[3], dims[1], dims[2])
+    rng = np.random.default_rng(n)
+    p = init_params(dims[0], dims[3], dims[1], dims[2], seed=n)
+    p = p + rng.normal(0, 0.05, p.size).astype(np.float32) * (p == 0)
+    net.set_params(p)
+    x = rng.normal(size=(n, dims[0])).astype(np.float32)
+    xt = torch.as_tensor(x, device="cuda:0")
+    y = net.forward(xt)
+    y_ref, _ = M.forward(p.astype(np.float64), dims, x.astype(np.float64), bf16=True)
+    assert np.linalg.norm(y.cpu().numpy() - y_ref) <= 5e-3 * np.linalg.norm(y_ref)
+    for k in (1, 35):
+        assert torch.equal(net.forward(xt[-k:].contiguous()), y[-k:])
+    net.close()
+
+
 def test_gradients_match_reference():
     import torch
     net, p = _net(7)
