@@ -1102,13 +1102,14 @@ __global__ void __launch_bounds__(LM_THREADS) low_mach_div_kernel(LowMachDivArgs
 
 // ---------------------------------------------------------------------------
 // Stiffness-ordered queue: bin the inner cells by expected cost, most
-// expensive bin first.  A block bins a contiguous run of BIN_RUN cells (one
+// expensive bin first.  A block bins a contiguous run of cells (one
 // global atomic per bin and block); within a bin, the cells of a run come in
 // roughly increasing index order.
 // ---------------------------------------------------------------------------
 constexpr int NBIN = 64;
+static_assert(NBIN == WAVE, "a bin to a lane");
 constexpr int BIN_THREADS = 256;
-constexpr int BIN_RUN = 32 * BIN_THREADS;
+constexpr int BIN_RUN_MAX = 32;       // cells a thread takes, at most
 
 struct BinArgs {
   GridIdx g;
@@ -1117,10 +1118,11 @@ struct BinArgs {
   double t_gate;
   const int32_t *hist;              // NSTEP of the previous call, or NULL (use T)
   unsigned long long *count;        // [NBIN]
-  unsigned long long *cursor;       // [NBIN] first queue position of each bin
+  unsigned long long *cursor;       // [NBIN] cells of each bin placed
   const int32_t *in_list;           // cells to order (NULL: all inner cells 0..npos-1)
   long long npos;                   // number of cells to order
   int32_t *list;                    // [npos] the ordered cells
+  int run;                          // cells a thread takes
 };
 
 // 0 = gated (no integration); otherwise grows with the expected cost.
@@ -1144,8 +1146,8 @@ NRG_DI void bin_histogram(const BinArgs &a, unsigned int *h)
 {
   if (threadIdx.x < NBIN) h[threadIdx.x] = 0u;
   __syncthreads();
-  const long long p0 = (long long)blockIdx.x * BIN_RUN + threadIdx.x;
-  for (int k = 0; k < BIN_RUN / BIN_THREADS; ++k) {
+  const long long p0 = (long long)blockIdx.x * a.run * BIN_THREADS + threadIdx.x;
+  for (int k = 0; k < a.run; ++k) {
     const long long p = p0 + (long long)k * BIN_THREADS;
     if (p < a.npos) atomicAdd(&h[cost_bin(a, a.in_list ? (long long)a.in_list[p] : p)], 1u);
   }
@@ -1159,32 +1161,27 @@ __global__ void __launch_bounds__(BIN_THREADS) bin_count_kernel(BinArgs a)
   if (threadIdx.x < NBIN && h[threadIdx.x]) atomicAdd(&a.count[threadIdx.x], (unsigned long long)h[threadIdx.x]);
 }
 
-// cursor[b] = number of cells in the bins more expensive than b (one wave).
-__global__ void bin_offsets_kernel(BinArgs a)
-{
-  if (threadIdx.x == 0) {
-    unsigned long long pos = 0;
-    for (int k = NBIN - 1; k >= 0; --k) {
-      a.cursor[k] = pos;
-      pos += a.count[k];
-    }
-  }
-}
-
-// Each block claims its bins' slots with one atomic per bin, then places its
-// run's cells (same run as bin_count_kernel, binned again).
+// Each block claims its bins' slots with one atomic per bin, behind the cells of
+// the more expensive bins, then places its run's cells (same run as
+// bin_count_kernel, binned again).
 __global__ void __launch_bounds__(BIN_THREADS) bin_scatter_kernel(BinArgs a)
 {
   __shared__ unsigned int h[NBIN];
   __shared__ unsigned long long base[NBIN];
   bin_histogram(a, h);
   if (threadIdx.x < NBIN) {
-    base[threadIdx.x] = h[threadIdx.x] ? atomicAdd(&a.cursor[threadIdx.x], (unsigned long long)h[threadIdx.x]) : 0ull;
+    unsigned long long after = a.count[threadIdx.x];   // ... of this bin and the more expensive ones
+    for (int d = 1; d < NBIN; d <<= 1) {
+      const unsigned long long v = __shfl_down(after, d, WAVE);
+      after += (int)threadIdx.x + d < NBIN ? v : 0ull;
+    }
+    base[threadIdx.x] = after - a.count[threadIdx.x] +
+                        (h[threadIdx.x] ? atomicAdd(&a.cursor[threadIdx.x], (unsigned long long)h[threadIdx.x]) : 0ull);
     h[threadIdx.x] = 0u;
   }
   __syncthreads();
-  const long long p0 = (long long)blockIdx.x * BIN_RUN + threadIdx.x;
-  for (int k = 0; k < BIN_RUN / BIN_THREADS; ++k) {
+  const long long p0 = (long long)blockIdx.x * a.run * BIN_THREADS + threadIdx.x;
+  for (int k = 0; k < a.run; ++k) {
     const long long p = p0 + (long long)k * BIN_THREADS;
     if (p < a.npos) {
       const long long q = a.in_list ? (long long)a.in_list[p] : p;
@@ -2438,10 +2435,12 @@ static void enqueue_order(nrg_chem_t *h, StepArgs &a, bool use_hist, const int32
   b.list = h->order_list;
   b.in_list = in_list;
   b.npos = n;
-  const unsigned nb = (unsigned)((n + BIN_RUN - 1) / BIN_RUN);
+  // runs as long as still give every CU four blocks (84,000 listed cells: 55 + 50 us
+  // with 32 cells a thread, and an offsets kernel of 8, 9 + 9 with one)
+  b.run = (int)std::min<long long>(BIN_RUN_MAX, std::max<long long>(1, n / (4ll * h->num_cu * BIN_THREADS)));
+  const unsigned nb = (unsigned)((n + b.run * BIN_THREADS - 1) / (b.run * BIN_THREADS));
   hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(2 * NBIN), 0, h->stream, h->bins, 2 * NBIN);
   hipLaunchKernelGGL(bin_count_kernel, dim3(nb), dim3(BIN_THREADS), 0, h->stream, b);
-  hipLaunchKernelGGL(bin_offsets_kernel, dim3(1), dim3(64), 0, h->stream, b);
   hipLaunchKernelGGL(bin_scatter_kernel, dim3(nb), dim3(BIN_THREADS), 0, h->stream, b);
 }
 
