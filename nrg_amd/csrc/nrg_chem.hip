@@ -163,6 +163,20 @@ NRG_DI long long cell_offset_wide(const GridIdx &g, long long q)
   return (i - g.lo0) + (long long)g.nx * ((j - g.lo1) + (long long)g.ny * (kk - g.lo2));
 }
 
+// A store of the passes over all fields that HBM bounds; with STREAM, past the
+// caches, which pays where such a pass touches more than the 256 MB memory-side
+// cache holds before anything is read again (streams()).  Waves write whole
+// 64-cell slices (a line written in parts costs more so: the table step with its
+// gated cells' stores apart 142 us, together 127).
+template <bool STREAM, class V, class W>
+NRG_DI void put(V *p, W v)
+{
+  if (STREAM)
+    __builtin_nontemporal_store((V)v, p);
+  else
+    *p = (V)v;
+}
+
 NRG_DI long long cell_of(const StepArgs &a, long long t)
 {
   return a.list ? (long long)a.list[a.base + t] : a.base + t;
@@ -746,6 +760,7 @@ NRG_DI double calculate_temperature(const MechCoef &mc, double T, double e_i, co
   return temp;
 }
 
+template <bool STREAM>
 __global__ void __launch_bounds__(256) closure_kernel(ClosureArgs a)
 {
   __shared__ MechCoef mc;
@@ -767,9 +782,9 @@ __global__ void __launch_bounds__(256) closure_kernel(ClosureArgs a)
       }
 #pragma unroll
       for (int s = 0; s < S; ++s) y[s] = dmax(y[s], 0.0) / sum;
-      a.E_f[off] = Ef;
+      put<STREAM>(&a.E_f[off], Ef);
 #pragma unroll
-      for (int s = 0; s < S; ++s) a.Y[s][off] = y[s];
+      for (int s = 0; s < S; ++s) put<STREAM>(&a.Y[s][off], y[s]);
     } else {
 #pragma unroll
       for (int s = 0; s < S; ++s) y[s] = a.Y[s][off];
@@ -788,8 +803,8 @@ __global__ void __launch_bounds__(256) closure_kernel(ClosureArgs a)
     for (int s = 0; s < S; ++s) X[s] = (y[s] / mc.W[s]) * wmix;
     e_i = e_i * wmix;
     const double Tn = calculate_temperature(mc, a.T[off], e_i, X);
-    a.T[off] = Tn;
-    if (a.p) a.p[off] = ((Tn * rho) * R_GAS_J) / wmix;
+    put<STREAM>(&a.T[off], Tn);
+    if (a.p) put<STREAM>(&a.p[off], ((Tn * rho) * R_GAS_J) / wmix);
   });
 }
 
@@ -886,7 +901,7 @@ constexpr int TABLE_LDS_BYTES = 32768;        // a table up to this size is stag
 // A grid of as many blocks as fit on the CUs strides over the cells, so the
 // table is staged into LDS once per block (not once per 256 cells) and the
 // integrated-cell count takes one global atomic per block.
-template <bool TAB_LDS>
+template <bool TAB_LDS, bool STREAM>
 __global__ void __launch_bounds__(TABLE_THREADS) table_kernel(TableArgs a)
 {
   extern __shared__ double tab_lds[];         // T_t[rows], dC_t[S][rows] when TAB_LDS
@@ -908,47 +923,48 @@ __global__ void __launch_bounds__(TABLE_THREADS) table_kernel(TableArgs a)
   // first inner cell's slice to the last inner cell) and skip ghost cells:
   // with ghost layers a row of inner cells starts off a cache line, and
   // walking inner cells would make every wave touch one line more per field.
-  for (long long off = a.g.pad0 + (long long)blockIdx.x * TABLE_THREADS + threadIdx.x;
-       off < a.g.pad1; off += stride) {
+  const double rdt = recip(a.dt);
+  for (long long off = a.g.pad0 + (long long)blockIdx.x * TABLE_THREADS + threadIdx.x; off < a.g.pad1; off += stride) {
     if (!inner_at(a.g, off)) continue;
     const double T = a.T[off];
     const int8_t bcv = a.bc ? a.bc[off] : (int8_t)0;
-    if (!(T >= a.t_gate && bcv == 0)) {
+    const bool run = T >= a.t_gate && bcv == 0;
+    double c[S], ef = 0.0;
 #pragma unroll
-      for (int s = 0; s < S; ++s) a.Yp[s][off] = 0.0;
-      a.Efp[off] = 0.0;
-      if (a.status) a.status[off] = NRG_CELL_GATED;
-      continue;
+    for (int s = 0; s < S; ++s) c[s] = 0.0;
+    if (run) {
+      ++cnt;
+      double cin[S];
+#pragma unroll
+      for (int s = 0; s < S; ++s) c[s] = cin[s] = a.Y[s][off];
+      const int i = table_interval(Tt, a.rows, a.ascending, T);
+      if (i >= 0) {
+        const double t0 = Tt[i], t1 = Tt[i + 1], up = t1 - t0, dn = t0 - t1, rup = recip(up);
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+          c[s] = div_by(dC[s * a.rows + i + 1] * (T - t0), up, rup) +
+                 div_by(dC[s * a.rows + i] * (T - t1), dn, -rup);
+      }
+      if (T < Tt[0]) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) c[s] = 0.0;
+      }
+      if (T > Tt[a.rows - 1]) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) c[s] = dC[s * a.rows + a.rows - 1];
+      }
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        put<STREAM>(&a.Yp2[s][off], c[s] - cin[s]);
+        ef = ef - div_by(href[s] * c[s], a.dt, rdt);
+        c[s] = div_by(c[s] * W[s], a.dt, rdt);
+      }
     }
-    ++cnt;
-    double cin[S], c[S];
+    // what gated cells have too, for the whole slice at once
 #pragma unroll
-    for (int s = 0; s < S; ++s) c[s] = cin[s] = a.Y[s][off];
-    const int i = table_interval(Tt, a.rows, a.ascending, T);
-    if (i >= 0) {
-      const double t0 = Tt[i], t1 = Tt[i + 1];
-#pragma unroll
-      for (int s = 0; s < S; ++s)
-        c[s] = (dC[s * a.rows + i + 1] * (T - t0)) / (t1 - t0) +
-               (dC[s * a.rows + i] * (T - t1)) / (t0 - t1);
-    }
-    if (T < Tt[0]) {
-#pragma unroll
-      for (int s = 0; s < S; ++s) c[s] = 0.0;
-    }
-    if (T > Tt[a.rows - 1]) {
-#pragma unroll
-      for (int s = 0; s < S; ++s) c[s] = dC[s * a.rows + a.rows - 1];
-    }
-    double ef = 0.0;
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-      a.Yp[s][off] = (c[s] * W[s]) / a.dt;
-      a.Yp2[s][off] = c[s] - cin[s];
-      ef = ef - (href[s] * c[s]) / a.dt;
-    }
-    a.Efp[off] = ef;
-    if (a.status) a.status[off] = NRG_CELL_OK;
+    for (int s = 0; s < S; ++s) put<STREAM>(&a.Yp[s][off], c[s]);
+    put<STREAM>(&a.Efp[off], ef);
+    if (a.status) put<STREAM>(&a.status[off], run ? NRG_CELL_OK : NRG_CELL_GATED);
   }
   if (cnt) atomicAdd(&n_integ, cnt);
   __syncthreads();
@@ -973,6 +989,7 @@ struct LowMachEosArgs {
   double *p, *cp, *gamma, *h_s, *v_s, *e_i, *E_f;   // optional
 };
 
+template <bool STREAM>
 __global__ void __launch_bounds__(LM_THREADS) low_mach_eos_kernel(LowMachEosArgs a)
 {
   __shared__ MechCoef mc;
@@ -986,42 +1003,42 @@ __global__ void __launch_bounds__(LM_THREADS) low_mach_eos_kernel(LowMachEosArgs
       avg = avg + X[s] / mc.W[s];
     }
     const double W = 1.0 / avg;
-    a.mmm[off] = W;
+    put<STREAM>(&a.mmm[off], W);
 #pragma unroll
     for (int s = 0; s < S; ++s) X[s] = (X[s] * W) / mc.W[s];
     double ps;
     if (a.predictor) {
       const double p0 = a.p_stat[off];
-      a.p_stat_old[off] = p0;
+      put<STREAM>(&a.p_stat_old[off], p0);
       ps = p0 + a.dp[off] * a.dt;
     } else {
       ps = 0.5 * ((a.p_stat[off] + a.p_stat_old[off]) + a.dp[off] * a.dt);
     }
-    a.p_stat[off] = ps;
+    put<STREAM>(&a.p_stat[off], ps);
     const double rho = a.rho[off];
     const double T = ((ps / rho) / R_GAS_J) * W;
-    a.T[off] = T;
+    put<STREAM>(&a.T[off], T);
     double cp = 0.0;
 #pragma unroll
     for (int s = 0; s < S; ++s) cp = cp + cp_molar(mc, T, s) * X[s];
     const double g = cp / (cp - R_GAS_J);
-    if (a.gamma) a.gamma[off] = g;
+    if (a.gamma) put<STREAM>(&a.gamma[off], g);
     if (a.h_s) {
       double hT = 0.0, h0 = 0.0;
 #pragma unroll
       for (int s = 0; s < S; ++s) hT = hT + h_molar(mc, T, s) * X[s];
 #pragma unroll
       for (int s = 0; s < S; ++s) h0 = h0 + mc.h_ref[s] * X[s];
-      a.h_s[off] = (hT - h0) / W;
+      put<STREAM>(&a.h_s[off], (hT - h0) / W);
     }
-    if (a.cp) a.cp[off] = cp;
-    if (a.p) a.p[off] = ps;
-    if (a.v_s) a.v_s[off] = sqrt((g * ps) / rho);
+    if (a.cp) put<STREAM>(&a.cp[off], cp);
+    if (a.p) put<STREAM>(&a.p[off], ps);
+    if (a.v_s) put<STREAM>(&a.v_s[off], sqrt((g * ps) / rho));
     const double ei = (ps / rho) / (g - 1.0);
-    if (a.e_i) a.e_i[off] = ei;
+    if (a.e_i) put<STREAM>(&a.e_i[off], ei);
     if (a.E_f && a.ndim > 0) {
       const double vd = a.v[a.ndim - 1][off];
-      a.E_f[off] = ei + 0.5 * (vd * vd);
+      put<STREAM>(&a.E_f[off], ei + 0.5 * (vd * vd));
     }
   });
 }
@@ -1036,6 +1053,7 @@ struct LowMachSpeciesArgs {
   double *rho_out, *Y_out[S];
 };
 
+template <bool STREAM>
 __global__ void __launch_bounds__(LM_THREADS) low_mach_species_kernel(LowMachSpeciesArgs a)
 {
   at_inner_cell(a.g, [&](long long off) {
@@ -1063,9 +1081,9 @@ __global__ void __launch_bounds__(LM_THREADS) low_mach_species_kernel(LowMachSpe
       sum = sum + r[s];
     }
     if (sum > DBL_MIN) {
-      a.rho_out[off] = sum;
+      put<STREAM>(&a.rho_out[off], sum);
 #pragma unroll
-      for (int s = 0; s < S; ++s) a.Y_out[s][off] = r[s] / sum;
+      for (int s = 0; s < S; ++s) put<STREAM>(&a.Y_out[s][off], r[s] / sum);
     }
   });
 }
@@ -1078,26 +1096,40 @@ struct LowMachDivArgs {
   double *div;
 };
 
+// (The fields' loads are issued before the mechanism is staged, so that a block
+// waits for memory once: 2.0M cells 110 -> 98 us.)
+template <bool STREAM>
 __global__ void __launch_bounds__(LM_THREADS) low_mach_div_kernel(LowMachDivArgs a)
 {
   __shared__ MechCoef mc;
-  stage_mech(mc, a.mech);
-  at_inner_cell(a.g, [&](long long off) {
-    if (a.bc && a.bc[off] != 0) return;
-    const double W = a.mmm[off], rho = a.rho[off], T = a.T[off];
-    double d = 0.0;
+  const long long off = a.g.pad0 + (long long)blockIdx.x * LM_THREADS + threadIdx.x;
+  const bool in = off < a.g.pad1 && inner_at(a.g, off);
+  int8_t bc = 0;
+  double W = 1.0, rho = 1.0, T = 1.0, d = 0.0, Y[S] = {}, Yc[S] = {};
+  if (in) {
+    if (a.bc) bc = a.bc[off];
+    W = a.mmm[off];
+    rho = a.rho[off];
+    T = a.T[off];
     d = d + a.Efc[off];
-    double cp = 0.0;
 #pragma unroll
-    for (int s = 0; s < S; ++s) cp = cp + cp_molar(mc, T, s) * ((a.Y[s][off] * W) / mc.W[s]);
-    d = d / (((rho * cp) * T) / W);
+    for (int s = 0; s < S; ++s) Y[s] = a.Y[s][off];
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-      const double hs = (h_molar(mc, T, s) - mc.h_ref[s]) / mc.W[s];
-      d = d + (((W / mc.W[s]) / rho) - hs / (((rho * cp) * T) / W)) * a.Yc[s][off];
-    }
-    a.div[off] = d;
-  });
+    for (int s = 0; s < S; ++s) Yc[s] = a.Yc[s][off];
+  }
+  stage_mech(mc, a.mech);
+  if (!in || bc != 0) return;
+  double cp = 0.0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) cp = cp + cp_molar(mc, T, s) * ((Y[s] * W) / mc.W[s]);
+  const double heat = ((rho * cp) * T) / W;
+  d = d / heat;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const double hs = (h_molar(mc, T, s) - mc.h_ref[s]) / mc.W[s];
+    d = d + (((W / mc.W[s]) / rho) - hs / heat) * Yc[s];
+  }
+  put<STREAM>(&a.div[off], d);
 }
 
 // ---------------------------------------------------------------------------
@@ -2276,9 +2308,22 @@ static int noalloc_setup(int dev)
 // Blocks of 256 threads covering the aligned walk, one offset per thread.
 static long long walk_blocks(const GridIdx &g) { return std::max<long long>(1, (g.pad1 - g.pad0 + 255) / 256); }
 
+// Whether a pass over `fields` FP64 fields stores past the caches: where it touches
+// more than the 256 MB memory-side cache keeps for whoever reads its outputs next.
+// Calls, plain / past the caches: table step (29 fields) 427,050 cells 76 / 79 us, 1.0M
+// 98 / 103, 2.0M 178 / 145, 4.1M 302 / 278; closure (37) 427,050 64.7 / 65.9, 1.0M 94 /
+// 94, 2.0M 136 / 134; the low-Mach passes (23 to 29, three in turn) 427,050 133 /
+// 133, 1.0M 218 / 198, 2.0M 356 / 316.  (Loads that pass the caches lose: the table
+// step's kernel 119 us, 140 with both.)
+static bool streams(const GridIdx &g, int fields, long long mib)
+{
+  return (g.pad1 - g.pad0) * 8 * fields > (mib << 20);
+}
+
 // Blocks for a kernel that strides over the aligned walk itself: its resident
-// blocks per CU times the CUs (a block more than fits would run as a tail
-// after the others), and no more blocks than the walk has 256-cell slices.
+// blocks per CU times the CUs at most (a block more than fits would run as a
+// tail after the others), and as many fewer as leave every block the same number
+// of the walk's 256-cell slices (table step of 427,050 cells 78 -> 75 us).
 template <class K>
 static long long resident_blocks(const nrg_chem_handle *h, K kernel, size_t dyn_lds, const GridIdx &g)
 {
@@ -2286,7 +2331,9 @@ static long long resident_blocks(const nrg_chem_handle *h, K kernel, size_t dyn_
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, dyn_lds) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
-  return std::min<long long>(walk_blocks(g), (long long)per_cu * h->num_cu);
+  const long long nb = walk_blocks(g), resident = (long long)per_cu * h->num_cu;
+  const long long rounds = (nb + resident - 1) / resident;
+  return (nb + rounds - 1) / rounds;
 }
 
 // ---- entry points of this topology (forwarded from nrg_api.cpp) ----------
@@ -2436,7 +2483,7 @@ static void enqueue_order(nrg_chem_t *h, StepArgs &a, bool use_hist, const int32
   b.in_list = in_list;
   b.npos = n;
   // runs as long as still give every CU four blocks (84,000 listed cells: 55 + 50 us
-  // with 32 cells a thread, and an offsets kernel of 8, 9 + 9 with one)
+  // with 32 cells a thread and an offsets kernel of 8, 9 + 9 with one)
   b.run = (int)std::min<long long>(BIN_RUN_MAX, std::max<long long>(1, n / (4ll * h->num_cu * BIN_THREADS)));
   const unsigned nb = (unsigned)((n + b.run * BIN_THREADS - 1) / (b.run * BIN_THREADS));
   hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(2 * NBIN), 0, h->stream, h->bins, 2 * NBIN);
@@ -2884,7 +2931,8 @@ static int closure_impl(nrg_chem_t *h, const nrg_grid *grid, double dt, int appl
   HIP_TRY(hipSetDevice(h->device));
   if (a.g.ninner > 0) {
     const long long nb = walk_blocks(a.g);
-    hipLaunchKernelGGL(closure_kernel, dim3((unsigned)nb), dim3(256), 0, h->stream, a);
+    const auto kernel = streams(a.g, 4 * S + 1, 320) ? closure_kernel<true> : closure_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(256), 0, h->stream, a);
     HIP_TRY(hipGetLastError());
   }
   HIP_TRY(hipStreamSynchronize(h->stream));
@@ -2997,13 +3045,12 @@ int nrg_chem_table_step_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, cons
   HIP_TRY(hipEventRecord(h->ev0, h->stream));
   if (a.g.ninner > 0) {
     const size_t tab_bytes = sizeof(double) * (size_t)(S + 1) * (size_t)a.rows;
-    if (tab_bytes <= (size_t)TABLE_LDS_BYTES)
-      hipLaunchKernelGGL(table_kernel<true>, dim3((unsigned)resident_blocks(h, table_kernel<true>, tab_bytes, a.g)),
-                         dim3(TABLE_THREADS), tab_bytes, h->stream, a);
-    else
-      hipLaunchKernelGGL(table_kernel<false>, dim3((unsigned)resident_blocks(h, table_kernel<false>, 0, a.g)),
-                         dim3(TABLE_THREADS), 0, h->stream, a);
-    HIP_TRY(hipGetLastError());
+    const bool lds = tab_bytes <= (size_t)TABLE_LDS_BYTES, st = streams(a.g, 3 * S + 2, 320);
+    const auto kernel = lds ? (st ? table_kernel<true, true> : table_kernel<true, false>)
+                            : (st ? table_kernel<false, true> : table_kernel<false, false>);
+    const size_t dyn = lds ? tab_bytes : 0;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)resident_blocks(h, kernel, dyn, a.g)), dim3(TABLE_THREADS), dyn,
+                       h->stream, a);
   }
   HIP_TRY(hipEventRecord(h->ev1, h->stream));
   HIP_TRY(hipMemcpyAsync(acc, h->dev_acc, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
@@ -3060,7 +3107,8 @@ int nrg_low_mach_state_equation_dev(nrg_chem_t *h, const nrg_grid *grid, double 
   a.E_f = E_f;
   HIP_TRY(hipSetDevice(h->device));
   if (a.g.ninner > 0) {
-    hipLaunchKernelGGL(low_mach_eos_kernel, dim3((unsigned)walk_blocks(a.g)), dim3(LM_THREADS), 0,
+    const auto kernel = streams(a.g, S + 16, 128) ? low_mach_eos_kernel<true> : low_mach_eos_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)walk_blocks(a.g)), dim3(LM_THREADS), 0,
                        h->stream, a);
     HIP_TRY(hipGetLastError());
   }
@@ -3101,7 +3149,8 @@ int nrg_low_mach_species_dev(nrg_chem_t *h, const nrg_grid *grid, double time_st
   a.rho_out = rho_out;
   HIP_TRY(hipSetDevice(h->device));
   if (a.g.ninner > 0) {
-    hipLaunchKernelGGL(low_mach_species_kernel, dim3((unsigned)walk_blocks(a.g)), dim3(LM_THREADS), 0,
+    const auto kernel = streams(a.g, 3 * S + 2, 128) ? low_mach_species_kernel<true> : low_mach_species_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)walk_blocks(a.g)), dim3(LM_THREADS), 0,
                        h->stream, a);
     HIP_TRY(hipGetLastError());
   }
@@ -3135,7 +3184,8 @@ int nrg_low_mach_chem_divergence_dev(nrg_chem_t *h, const nrg_grid *grid, const 
   a.div = div_v;
   HIP_TRY(hipSetDevice(h->device));
   if (a.g.ninner > 0) {
-    hipLaunchKernelGGL(low_mach_div_kernel, dim3((unsigned)walk_blocks(a.g)), dim3(LM_THREADS), 0,
+    const auto kernel = streams(a.g, 2 * S + 5, 128) ? low_mach_div_kernel<true> : low_mach_div_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)walk_blocks(a.g)), dim3(LM_THREADS), 0,
                        h->stream, a);
     HIP_TRY(hipGetLastError());
   }
