@@ -148,7 +148,7 @@ struct StepArgs {
   double *rates_out;                    // same buffer, written by rates_kernel
   long long base, nchunk;               // this launch covers queue positions [base, base+nchunk)
   const int32_t *list;                  // NULL: position t is inner cell t; else inner cell list[t]
-  int32_t *hist;                        // optional: NSTEP of each inner cell (0 if gated), for ordering
+  int32_t *hist;                        // optional: each inner cell's work (hist_code), for ordering
   int cpw;                              // cells a wave of the integrator holds at a time
 };
 
@@ -220,6 +220,11 @@ NRG_DI void stage_bdf(BdfCoef &dst, const MechCoef *src, double sqrtn)
   __syncthreads();
 }
 
+// What a step records of a cell for the next one's order: its steps and, above
+// them, its right-hand sides (0 if gated).
+constexpr int HIST_FE_SHIFT = 16, HIST_STEPS = (1 << HIST_FE_SHIFT) - 1;
+NRG_DI int32_t hist_code(int nstep, int nfe) { return min(nstep, HIST_STEPS) | (min(nfe, 0x7fff) << HIST_FE_SHIFT); }
+
 // accumulator slots
 enum { ACC_INTEG = 0, ACC_NSTEP, ACC_NFE, ACC_NJE, ACC_NCORR, ACC_NATT, ACC_NSTEP_MAX, ACC_NFE_MAX,
        ACC_STATUS0,     // ACC_STATUS0 + NRG_CELL_* (8 slots)
@@ -232,7 +237,8 @@ enum { ACC_INTEG = 0, ACC_NSTEP, ACC_NFE, ACC_NJE, ACC_NCORR, ACC_NATT, ACC_NSTE
 #if NRG_PART < 2
 __global__ void reset_kernel(unsigned long long *acc, int n)
 {
-  if ((int)threadIdx.x < n) acc[threadIdx.x] = 0ull;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) acc[i] = 0ull;
 }
 #endif
 
@@ -384,7 +390,7 @@ NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, const Cell &c, con
     a.Efp[off] = ef;
     if (a.status) a.status[off] = status;
     if (a.nstep) a.nstep[q] = c.nstep;
-    if (a.hist) a.hist[q] = c.nstep;
+    if (a.hist) a.hist[q] = hist_code(c.nstep, c.work);   // lane 0's counter: NFE
     atomicAdd(&tally[ACC_STATUS0 + status], 1ull);
   }
   if (a.nstep && ln.sub == WORK_NFE) a.nfe[q] = c.work;
@@ -592,7 +598,7 @@ NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, long long q, long 
     a.nfe[q] = c.nfe;
     a.nje[q] = c.nje;
   }
-  if (a.hist) a.hist[q] = c.nstep;
+  if (a.hist) a.hist[q] = hist_code(c.nstep, c.nfe);
   if (status != NRG_CELL_OK) atomicAdd(&tally[ACC_STATUS0 + status], 1ull);
   tl.integrated += 1;
   tl.nstep += c.nstep;
@@ -1138,8 +1144,15 @@ __global__ void __launch_bounds__(LM_THREADS) low_mach_div_kernel(LowMachDivArgs
 // global atomic per bin and block); within a bin, the cells of a run come in
 // roughly increasing index order.
 // ---------------------------------------------------------------------------
-constexpr int NBIN = 64;
-static_assert(NBIN == WAVE, "a bin to a lane");
+// Bins by steps, and of each by right-hand sides (modulo): a wave's lanes wait for
+// each other wherever their paths through the integrator part, and cells that
+// took as many right-hand sides in as many steps mostly took the same path (14 of
+// 64 lanes were busy per instruction on 256^3 hot kernels by steps alone).  One cell
+// per lane, by steps / 16 / 64 bins of each: 2.1M cells with hot kernels 4.85 / 3.73 /
+// 3.69 ms, 1M flame cells 14.6 / 12.2 / 11.9, 1M igniting 17.3 / 15.7 / 14.9.  (By a hash
+// of the path instead: 3.73, 11.4, 16.0.)  Placing 16.7M cells costs 0.34 ms, 0.10 before.
+constexpr int NBIN_STEP = 64, NBIN_FE = 64;
+constexpr int NBIN = NBIN_STEP * NBIN_FE;
 constexpr int BIN_THREADS = 256;
 constexpr int BIN_RUN_MAX = 32;       // cells a thread takes, at most
 
@@ -1148,7 +1161,7 @@ struct BinArgs {
   const double *T;
   const int8_t *bc;
   double t_gate;
-  const int32_t *hist;              // NSTEP of the previous call, or NULL (use T)
+  const int32_t *hist;              // hist_code of the previous call, or NULL (use T)
   unsigned long long *count;        // [NBIN]
   unsigned long long *cursor;       // [NBIN] cells of each bin placed
   const int32_t *in_list;           // cells to order (NULL: all inner cells 0..npos-1)
@@ -1165,18 +1178,18 @@ NRG_DI int cost_bin(const BinArgs &a, long long q)
   const double T = a.T[off];
   if (!(T >= a.t_gate && b == 0)) return 0;
   if (a.hist) {
-    const int n = max(a.hist[q], 0);
+    const int code = a.hist[q], n = code & HIST_STEPS, fe = code >> HIST_FE_SHIFT;
     const int k = n <= 31 ? n : 31 + (n - 28) / 4;     // unit bins to 31 steps, then 4-step bins
-    return 1 + min(NBIN - 2, k);
+    return (1 + min(NBIN_STEP - 2, k)) * NBIN_FE + fe % NBIN_FE;
   }
   const double x = (T - a.t_gate) * (1.0 / 50.0);                     // first call: 50 K bins
-  return 1 + (x < (double)(NBIN - 2) ? (int)x : NBIN - 2);
+  return (1 + (x < (double)(NBIN_STEP - 2) ? (int)x : NBIN_STEP - 2)) * NBIN_FE;
 }
 
 // Histogram of the block's run into LDS.
 NRG_DI void bin_histogram(const BinArgs &a, unsigned int *h)
 {
-  if (threadIdx.x < NBIN) h[threadIdx.x] = 0u;
+  for (int b = threadIdx.x; b < NBIN; b += BIN_THREADS) h[b] = 0u;
   __syncthreads();
   const long long p0 = (long long)blockIdx.x * a.run * BIN_THREADS + threadIdx.x;
   for (int k = 0; k < a.run; ++k) {
@@ -1190,7 +1203,8 @@ __global__ void __launch_bounds__(BIN_THREADS) bin_count_kernel(BinArgs a)
 {
   __shared__ unsigned int h[NBIN];
   bin_histogram(a, h);
-  if (threadIdx.x < NBIN && h[threadIdx.x]) atomicAdd(&a.count[threadIdx.x], (unsigned long long)h[threadIdx.x]);
+  for (int b = threadIdx.x; b < NBIN; b += BIN_THREADS)
+    if (h[b]) atomicAdd(&a.count[b], (unsigned long long)h[b]);
 }
 
 // Each block claims its bins' slots with one atomic per bin, behind the cells of
@@ -1199,17 +1213,27 @@ __global__ void __launch_bounds__(BIN_THREADS) bin_count_kernel(BinArgs a)
 __global__ void __launch_bounds__(BIN_THREADS) bin_scatter_kernel(BinArgs a)
 {
   __shared__ unsigned int h[NBIN];
-  __shared__ unsigned long long base[NBIN];
+  __shared__ unsigned long long base[NBIN], sums[BIN_THREADS / WAVE];
   bin_histogram(a, h);
-  if (threadIdx.x < NBIN) {
-    unsigned long long after = a.count[threadIdx.x];   // ... of this bin and the more expensive ones
-    for (int d = 1; d < NBIN; d <<= 1) {
-      const unsigned long long v = __shfl_down(after, d, WAVE);
-      after += (int)threadIdx.x + d < NBIN ? v : 0ull;
-    }
-    base[threadIdx.x] = after - a.count[threadIdx.x] +
-                        (h[threadIdx.x] ? atomicAdd(&a.cursor[threadIdx.x], (unsigned long long)h[threadIdx.x]) : 0ull);
-    h[threadIdx.x] = 0u;
+  // cells of the more expensive bins: each thread's bins, then the threads after it
+  constexpr int PER = NBIN / BIN_THREADS;
+  static_assert(NBIN % BIN_THREADS == 0, "bins to a thread");
+  const int b0 = threadIdx.x * PER, lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  unsigned long long mine = 0;
+  for (int b = b0; b < b0 + PER; ++b) mine += a.count[b];
+  unsigned long long after = mine;
+  for (int d = 1; d < WAVE; d <<= 1) {
+    const unsigned long long v = __shfl_down(after, d, WAVE);
+    after += lane + d < WAVE ? v : 0ull;
+  }
+  if (lane == 0) sums[w] = after;
+  __syncthreads();
+  for (int k = w + 1; k < BIN_THREADS / WAVE; ++k) after += sums[k];
+  after -= mine;
+  for (int b = b0 + PER - 1; b >= b0; --b) {
+    base[b] = after + (h[b] ? atomicAdd(&a.cursor[b], (unsigned long long)h[b]) : 0ull);
+    after += a.count[b];
+    h[b] = 0u;
   }
   __syncthreads();
   const long long p0 = (long long)blockIdx.x * a.run * BIN_THREADS + threadIdx.x;
@@ -2486,7 +2510,7 @@ static void enqueue_order(nrg_chem_t *h, StepArgs &a, bool use_hist, const int32
   // with 32 cells a thread and an offsets kernel of 8, 9 + 9 with one)
   b.run = (int)std::min<long long>(BIN_RUN_MAX, std::max<long long>(1, n / (4ll * h->num_cu * BIN_THREADS)));
   const unsigned nb = (unsigned)((n + b.run * BIN_THREADS - 1) / (b.run * BIN_THREADS));
-  hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(2 * NBIN), 0, h->stream, h->bins, 2 * NBIN);
+  hipLaunchKernelGGL(reset_kernel, dim3(2 * NBIN / 256), dim3(256), 0, h->stream, h->bins, 2 * NBIN);
   hipLaunchKernelGGL(bin_count_kernel, dim3(nb), dim3(BIN_THREADS), 0, h->stream, b);
   hipLaunchKernelGGL(bin_scatter_kernel, dim3(nb), dim3(BIN_THREADS), 0, h->stream, b);
 }
@@ -2518,15 +2542,14 @@ static int prepare_rates(nrg_chem_t *h, long long npos)
 // instead of one to a lane group: from there they fill the chip often enough
 // (65,536 once) that a lane's shorter way through a step counts more than the
 // group's shorter way through a cell.  Kernel ms, group against lane, KEROMNES:
-//   finite differences: 262,144 flame cells 4.62 / 4.49, 589,824 9.9 / 8.7,
-//   1M 17.4 / 14.6; igniting 262,144 5.2 / 4.6 in 100 ns and 11.8 / 13.3 in 1 us,
-//   545,400 in 1 us 23 / 25; with most cells cold (hot kernels) 884,736 2.6 / 3.6,
-//   1.4M 3.4 / 3.6, 2.1M 5.5 / 4.9.
+//   finite differences: 262,144 flame cells 4.1 / 3.7, 589,824 8.8 / 7.2, 1M 15.3 /
+//   11.9; igniting 262,144 4.7 / 4.1 in 100 ns and 11.8 / 12.9 in 1 us, 545,400 in 1 us
+//   23.0 / 24.1; with most cells cold (hot kernels) 884,736 2.5 / 3.5, 1.4M 3.4 / 3.5,
+//   2.1M 5.5 / 3.7.
 //   analytic Jacobian (few right-hand sides, so the vector work that a group
-//   shares counts less): 65,536 flame cells 0.91 / 1.11, 262,144 2.55 / 1.96;
-//   igniting 131,072 1.52 / 1.49, 196,608 2.14 / 1.80.  The learned step's
-//   fallback list holds no idle cells, which moves the line: 83,905 of 2.4M
-//   cells 1.67 / 1.51.
+//   shares counts less): 131,044 flame cells 1.33 / 1.09, 262,144 2.4 / 1.7; igniting
+//   131,072 1.41 / 1.52, 196,608 2.03 / 1.61.  The learned step's fallback list holds
+//   no idle cells, which moves the line: 83,905 of 2.4M cells 1.67 / 1.51.
 // With nine or ten species a group has 16 lanes, and a lane's state spills:
 //   TEREZA flame cells 1M 33.0 / 31.1, 2.4M 72 / 64; hot kernels 2.1M 10.6 /
 //   15.1, 7.1M 42 / 30; analytic igniting 131,072 3.1 / 2.0.
