@@ -2077,6 +2077,10 @@ struct StepKey {
   int jacobian;                // NRG_JAC_*: which integrator kernel the graph launches
 };
 
+// Pinned memory for the host-pointer entry points' fields, at most (137,000 cells of
+// KEROMNES).
+constexpr size_t STAGE_PINNED_MAX = 32u << 20;
+
 struct nrg_chem_handle {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -2090,13 +2094,14 @@ struct nrg_chem_handle {
   int jac_pct = 50;
   int persistent_blocks = 0;               // resident one-wave blocks of the integrator
   int lane_blocks = 0;                     // and of its one-cell-per-lane form
-  // staging buffers for the host-pointer entry point
-  std::vector<void *> stage;
+  // staging for the host-pointer entry point: device, and pinned host memory for small fields
+  void *stage = nullptr, *pinned = nullptr;
+  size_t stage_bytes = 0;
+  unsigned long long *acc_host = nullptr;  // pinned: counters on their way back
   // cell records of one chunk: REC_PAIRS pairs of doubles per position
   double *rates = nullptr;
   long long rates_cells = 0;
   long long chunk_max = 1ll << 23;
-  size_t stage_cells = 0;
   // learned step: features, network outputs, fallback list, counters
   hipEvent_t ev2 = nullptr, ev3 = nullptr;
   nrg::bf16 *sur_X = nullptr;
@@ -2329,6 +2334,16 @@ static int noalloc_setup(int dev)
 #endif
 }
 
+// The first n counters, once the stream is done (through pinned memory: a copy
+// into a stack variable adds ~10 us to a call).
+static hipError_t read_counters(nrg_chem_handle *h, unsigned long long *out, const unsigned long long *dev, int n)
+{
+  hipError_t e = hipMemcpyAsync(h->acc_host, dev, n * sizeof(*out), hipMemcpyDeviceToHost, h->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  if (e == hipSuccess) std::memcpy(out, h->acc_host, n * sizeof(*out));
+  return e;
+}
+
 // Blocks of 256 threads covering the aligned walk, one offset per thread.
 static long long walk_blocks(const GridIdx &g) { return std::max<long long>(1, (g.pad1 - g.pad0 + 255) / 256); }
 
@@ -2416,6 +2431,8 @@ int nrg_chem_create(const nrg_chem_mech *mech, const nrg_chem_opts *opts, nrg_ch
     return fail(set_error(NRG_CHEM_E_HIP, "hipMalloc mech"));
   if (hipMalloc(&h->dev_acc, ACC_SLOTS * sizeof(unsigned long long)) != hipSuccess)
     return fail(set_error(NRG_CHEM_E_HIP, "hipMalloc acc"));
+  if (hipHostMalloc(&h->acc_host, 16 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
+    return fail(set_error(NRG_CHEM_E_HIP, "hipHostMalloc acc"));
   {
     hipDeviceProp_t prop;
     int per_cu = 0;
@@ -2444,8 +2461,9 @@ void nrg_chem_destroy(nrg_chem_t *h)
   // teardown has no caller to report to: failures here are ignored
   (void)hipSetDevice(h->device);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  for (void *p : h->stage)
-    if (p) (void)hipFree(p);
+  if (h->stage) (void)hipFree(h->stage);
+  if (h->pinned) (void)hipHostFree(h->pinned);
+  if (h->acc_host) (void)hipHostFree(h->acc_host);
   if (h->dev_mech) (void)hipFree(h->dev_mech);
   if (h->dev_acc) (void)hipFree(h->dev_acc);
   if (h->rates) (void)hipFree(h->rates);
@@ -2756,8 +2774,7 @@ static int step_dev_impl(nrg_chem_t *h, const nrg_grid *grid, double dt, const d
       h->hist_grid = a.g;
     }
     HIP_TRY(hipEventRecord(h->ev1, h->stream));
-    HIP_TRY(hipMemcpyAsync(acc, h->dev_acc, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    HIP_TRY(read_counters(h, acc, h->dev_acc, 16));
     HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   }
   if (stats) fill_stats(acc, a.g.ninner, ms, stats);
@@ -2824,8 +2841,7 @@ int nrg_chem_step_dev_noalloc(nrg_chem_t *h, const nrg_grid *grid, double dt, co
   if (a.g.ninner > 0) enqueue_chunks(h, a, a.g.ninner, NRG_NOALLOC_CHUNK_CELLS, rates, acc_dev, false);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(h->ev1, h->stream));
-  HIP_TRY(hipMemcpyAsync(acc, acc_dev, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(hipStreamSynchronize(h->stream));
+  HIP_TRY(read_counters(h, acc, acc_dev, 16));
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   if (stats) fill_stats(acc, a.g.ninner, ms, stats);
   return integrator_status(acc);
@@ -2845,58 +2861,74 @@ static int step_host(nrg_chem_t *h, bool table, const nrg_grid *grid, double dt,
   const long long n = field_cells(grid);
   if (n <= 0) return set_error(NRG_CHEM_E_ARG, "empty field");
   HIP_TRY(hipSetDevice(h->device));
-  // staging layout: T, rho, E_f_prod, Y[S], Y_prod[S], Y_prod2[S] (doubles), bc (int8), status (int32)
-  const int nd = 3 + 3 * S;
-  if (h->stage_cells < (size_t)n) {
-    h->stage_cells = 0;
-    for (void *&q : h->stage)
-      if (q) {
-        void *old = q;
-        q = nullptr;   // never freed twice, even when this free fails
-        HIP_TRY(hipFree(old));
-      }
-    h->stage.assign(nd + 2, nullptr);
-    for (int i = 0; i < nd; ++i) HIP_TRY(hipMalloc(&h->stage[i], n * sizeof(double)));
-    HIP_TRY(hipMalloc(&h->stage[nd], n * sizeof(int8_t)));
-    HIP_TRY(hipMalloc(&h->stage[nd + 1], n * sizeof(int32_t)));
-    h->stage_cells = n;
+  for (int q = 0; q < S; ++q)
+    if (!Y[q] || !Y_prod[q] || !Y_prod2[q]) return set_error(NRG_CHEM_E_ARG, "species %d field is NULL", q + 1);
+  // staging layout: T, rho, Y[S], bc (padded to doubles); then what comes back:
+  // Y_prod[S], Y_prod2[S], E_f_prod, status
+  auto room = [&](size_t size) { return ((size_t)n * size + 255) / 256 * 256; };
+  const size_t in_bytes = (2 + S) * room(8) + room(1), out_bytes = (2 * S + 1) * room(8) + room(4);
+  if (h->stage_bytes < in_bytes + out_bytes) {
+    void *old = h->stage;
+    h->stage = nullptr;   // never freed twice, even when this free fails
+    h->stage_bytes = 0;
+    if (old) HIP_TRY(hipFree(old));
+    HIP_TRY(hipMalloc(&h->stage, in_bytes + out_bytes));
+    h->stage_bytes = in_bytes + out_bytes;
   }
-  auto D = [&](int i) { return (double *)h->stage[i]; };
-  const size_t bytes = n * sizeof(double);
+  // Small fields go through pinned memory, all in one copy each way: a copy from
+  // pageable memory returns only when it is done (~10 us each, 51 of them).  Calls of
+  // flame cells: 60 cells 980 -> 600 us, 9100 1580 -> 1100, 30,000 2080 -> 1640, 80,000
+  // 3860 -> 3740, 136,000 the same: from there the copies of single fields overlap.
+  const bool pin = in_bytes + out_bytes <= STAGE_PINNED_MAX;
+  if (pin && !h->pinned) HIP_TRY(hipHostMalloc(&h->pinned, STAGE_PINNED_MAX, hipHostMallocDefault));
+  char *dev = (char *)h->stage, *host = pin ? (char *)h->pinned : nullptr;
   hipStream_t s = h->stream;
-  HIP_TRY(hipMemcpyAsync(D(0), T, bytes, hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(D(1), rho, bytes, hipMemcpyHostToDevice, s));
+  size_t at = 0;
+  int rc = NRG_CHEM_OK;
+  auto up = [&](const void *src, size_t size) {   // the next field's device address
+    char *d = dev + at;
+    if (src && pin)
+      std::memcpy(host + at, src, n * size);
+    else if (src && rc == NRG_CHEM_OK && hipMemcpyAsync(d, src, n * size, hipMemcpyHostToDevice, s) != hipSuccess)
+      rc = set_error(NRG_CHEM_E_HIP, "copy of a field to the device");
+    at += room(size);
+    return src ? d : nullptr;
+  };
   const double *Yd[S];
   double *Ypd[S], *Yp2d[S];
-  for (int q = 0; q < S; ++q) {
-    if (!Y[q] || !Y_prod[q] || !Y_prod2[q]) return set_error(NRG_CHEM_E_ARG, "species %d field is NULL", q + 1);
-    HIP_TRY(hipMemcpyAsync(D(3 + q), Y[q], bytes, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(D(3 + 2 * S + q), Y_prod2[q], bytes, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(D(3 + S + q), Y_prod[q], bytes, hipMemcpyHostToDevice, s));
-    Yd[q] = D(3 + q);
-    Ypd[q] = D(3 + S + q);
-    Yp2d[q] = D(3 + 2 * S + q);
-  }
-  HIP_TRY(hipMemcpyAsync(D(2), E_f_prod, bytes, hipMemcpyHostToDevice, s));
-  int8_t *bcd = nullptr;
-  if (bc) {
-    bcd = (int8_t *)h->stage[nd];
-    HIP_TRY(hipMemcpyAsync(bcd, bc, n, hipMemcpyHostToDevice, s));
-  }
-  int32_t *std_ = cell_status ? (int32_t *)h->stage[nd + 1] : nullptr;
-  if (std_) HIP_TRY(hipMemcpyAsync(std_, cell_status, n * sizeof(int32_t), hipMemcpyHostToDevice, s));
-  int rc = table ? nrg_chem_table_step_dev(h, grid, dt, D(0), nullptr, D(1), Yd, bcd, Ypd, Yp2d, D(2),
-                                           std_, stats)
-                 : step_dev_impl(h, grid, dt, D(0), D(1), Yd, bcd, Ypd, Yp2d, D(2), std_, stats, nullptr,
-                                 nullptr, nullptr);
+  const double *Td = (const double *)up(T, 8), *rhod = (const double *)up(rho, 8);
+  for (int q = 0; q < S; ++q) Yd[q] = (const double *)up(Y[q], 8);
+  const int8_t *bcd = (const int8_t *)up(bc, 1);
+  for (int q = 0; q < S; ++q) Ypd[q] = (double *)up(Y_prod[q], 8);
+  for (int q = 0; q < S; ++q) Yp2d[q] = (double *)up(Y_prod2[q], 8);
+  double *Efd = (double *)up(E_f_prod, 8);
+  int32_t *std_ = (int32_t *)up(cell_status, 4);
+  if (rc != NRG_CHEM_OK) return rc;
+  if (pin) HIP_TRY(hipMemcpyAsync(dev, host, at, hipMemcpyHostToDevice, s));
+  rc = table ? nrg_chem_table_step_dev(h, grid, dt, Td, nullptr, rhod, Yd, bcd, Ypd, Yp2d, Efd, std_, stats)
+             : step_dev_impl(h, grid, dt, Td, rhod, Yd, bcd, Ypd, Yp2d, Efd, std_, stats, nullptr, nullptr,
+                             nullptr);
   if (rc != NRG_CHEM_OK && rc != NRG_CHEM_E_STEP_ZERO && rc != NRG_CHEM_E_REPEATED_FAIL) return rc;
-  for (int q = 0; q < S; ++q) {
-    HIP_TRY(hipMemcpyAsync(Y_prod[q], Ypd[q], bytes, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(Y_prod2[q], Yp2d[q], bytes, hipMemcpyDeviceToHost, s));
+  if (pin) {
+    HIP_TRY(hipMemcpyAsync(host + in_bytes, dev + in_bytes, out_bytes, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
   }
-  HIP_TRY(hipMemcpyAsync(E_f_prod, D(2), bytes, hipMemcpyDeviceToHost, s));
-  if (std_) HIP_TRY(hipMemcpyAsync(cell_status, std_, n * sizeof(int32_t), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
+  bool copied = true;
+  auto down = [&](void *dst, const void *src, size_t size) {
+    if (!dst) return;
+    if (pin)
+      std::memcpy(dst, host + ((const char *)src - dev), n * size);
+    else
+      copied = copied && hipMemcpyAsync(dst, src, n * size, hipMemcpyDeviceToHost, s) == hipSuccess;
+  };
+  for (int q = 0; q < S; ++q) {
+    down(Y_prod[q], Ypd[q], 8);
+    down(Y_prod2[q], Yp2d[q], 8);
+  }
+  down(E_f_prod, Efd, 8);
+  down(cell_status, std_, 4);
+  if (!copied) return set_error(NRG_CHEM_E_HIP, "copy of a field to the host");
+  if (!pin) HIP_TRY(hipStreamSynchronize(s));
   return rc;
 }
 
@@ -3076,8 +3108,7 @@ int nrg_chem_table_step_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, cons
                        h->stream, a);
   }
   HIP_TRY(hipEventRecord(h->ev1, h->stream));
-  HIP_TRY(hipMemcpyAsync(acc, h->dev_acc, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(hipStreamSynchronize(h->stream));
+  HIP_TRY(read_counters(h, acc, h->dev_acc, 16));
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
   if (stats) fill_stats(acc, a.g.ninner, ms, stats);
   return NRG_CHEM_OK;
@@ -3459,8 +3490,7 @@ int nrg_chem_surrogate_step_dev(nrg_chem_t *h, nrg_mlp_t *mlp, const nrg_surroga
                          dim3((unsigned)std::min<long long>(h->recheck_blocks, (n + RCHECK_CELLS - 1) / RCHECK_CELLS)),
                          dim3(256), 0, h->stream, sa);
       HIP_TRY(hipGetLastError());
-      HIP_TRY(hipMemcpyAsync(sur, h->sur_acc, sizeof(sur), hipMemcpyDeviceToHost, h->stream));
-      HIP_TRY(hipStreamSynchronize(h->stream));
+      HIP_TRY(read_counters(h, sur, h->sur_acc, SUR_SLOTS));
       ncand = screen == NRG_SUR_SCREEN_RATES ? (long long)sur[SUR_CAND] : 0;
       if (ncand > n || (long long)sur[SUR_FALLBACK] > n || (long long)sur[SUR_RECHECK] > n)
         return set_error(NRG_CHEM_E_HIP, "screen counts exceed %lld cells", n);
@@ -3489,8 +3519,7 @@ int nrg_chem_surrogate_step_dev(nrg_chem_t *h, nrg_mlp_t *mlp, const nrg_surroga
       HIP_TRY(hipGetLastError());
     }
     HIP_TRY(hipEventRecord(h->ev2, h->stream));
-    HIP_TRY(hipMemcpyAsync(sur, h->sur_acc, sizeof(sur), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    HIP_TRY(read_counters(h, sur, h->sur_acc, SUR_SLOTS));
     HIP_TRY(hipEventElapsedTime(&ms_gate, h->ev3, h->ev2));
     HIP_TRY(hipEventRecord(h->ev3, h->stream));
     const long long nfb = (long long)sur[SUR_FALLBACK];
@@ -3513,8 +3542,7 @@ int nrg_chem_surrogate_step_dev(nrg_chem_t *h, nrg_mlp_t *mlp, const nrg_surroga
       if ((st = enqueue_integrator(h, a, nfb, true))) return st;
     }
     HIP_TRY(hipEventRecord(h->ev1, h->stream));
-    HIP_TRY(hipMemcpyAsync(acc, h->dev_acc, sizeof(acc), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
+    HIP_TRY(read_counters(h, acc, h->dev_acc, 16));
     HIP_TRY(hipEventElapsedTime(&ms_fb, h->ev3, h->ev1));
   }
   if (stats) {
