@@ -1146,8 +1146,8 @@ __global__ void __launch_bounds__(LM_THREADS) low_mach_div_kernel(LowMachDivArgs
 // ---------------------------------------------------------------------------
 // Bins by steps, and of each by right-hand sides (modulo): a wave's lanes wait for
 // each other wherever their paths through the integrator part, and cells that
-// took as many right-hand sides in as many steps mostly took the same path (14 of
-// 64 lanes were busy per instruction on 256^3 hot kernels by steps alone).  One cell
+// took as many right-hand sides in as many steps mostly took the same path (256^3
+// hot kernels: 65 % of the lanes busy per instruction by steps alone, 71 % so).  One cell
 // per lane, by steps / 16 / 64 bins of each: 2.1M cells with hot kernels 4.85 / 3.73 /
 // 3.69 ms, 1M flame cells 14.6 / 12.2 / 11.9, 1M igniting 17.3 / 15.7 / 14.9.  (By a hash
 // of the path instead: 3.73, 11.4, 16.0.)  Placing 16.7M cells costs 0.34 ms, 0.10 before.
