@@ -1,5 +1,5 @@
 // chem_device.h -- thermochemistry, rate constants and mass action of the
-// gfx950 chemistry step, one cell per lane (the integrator is bdf_group.h).
+// gfx950 chemistry step, one cell per lane (the integrators: bdf_group.h, bdf_lane.h).
 //
 // The mechanism's numeric coefficients are one LDS copy per block.  Every
 // register-array index is a compile-time constant after unrolling.  Arithmetic

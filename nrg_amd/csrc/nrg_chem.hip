@@ -2879,8 +2879,12 @@ static int step_host(nrg_chem_t *h, bool table, const nrg_grid *grid, double dt,
   // pageable memory returns only when it is done (~10 us each, 51 of them).  Calls of
   // flame cells: 60 cells 980 -> 600 us, 9100 1580 -> 1100, 30,000 2080 -> 1640, 80,000
   // 3860 -> 3740, 136,000 the same: from there the copies of single fields overlap.
-  const bool pin = in_bytes + out_bytes <= STAGE_PINNED_MAX;
-  if (pin && !h->pinned) HIP_TRY(hipHostMalloc(&h->pinned, STAGE_PINNED_MAX, hipHostMallocDefault));
+  bool pin = in_bytes + out_bytes <= STAGE_PINNED_MAX;
+  if (pin && !h->pinned && hipHostMalloc(&h->pinned, STAGE_PINNED_MAX, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();   // no pinned memory to be had: field by field
+    h->pinned = nullptr;
+    pin = false;
+  }
   char *dev = (char *)h->stage, *host = pin ? (char *)h->pinned : nullptr;
   hipStream_t s = h->stream;
   size_t at = 0;
