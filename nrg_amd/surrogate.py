@@ -84,7 +84,7 @@ class MLP:
         torch = _torch()
         x, t = x.contiguous(), t.contiguous()
         g = torch.empty(self.num_params, dtype=torch.float32, device=x.device)
-        loss = torch.zeros(1, dtype=torch.float32, device=x.device)
+        loss = torch.empty(1, dtype=torch.float32, device=x.device)   # written, not added to
         y = torch.empty((x.shape[0], self.n_out), dtype=torch.float32, device=x.device)
         torch.cuda.synchronize()
         check(self.lib, self.lib.nrg_mlp_grad_dev(self.h, x.shape[0], x.data_ptr(), t.data_ptr(),
