@@ -268,10 +268,14 @@ NRG_DI double row_pass(double v)
 
 // ---------------------------------------------------------------------------
 // FP64 division and square root without the scaling steps of the compiler's
-// expansions: the same instructions otherwise, hence the same bits wherever
-// those would not scale (|n|, |d|, |n/d| within 2^+-700; x = 0 or above
-// 2^-767), which holds for every operand here.  A quotient takes 9
-// instructions instead of 13, one by a divisor whose reciprocal is at hand 4.
+// expansions, the same instructions otherwise: the same bits where those would
+// not scale, and only there.  A numerator below 2^-969 has a remainder that FP64
+// does not hold (the last bit goes), and a quotient above 2^1023 gives NaN
+// instead of infinity.  Concentrations, densities, time steps and tables come
+// from the caller with any exponent, so these are used only where the operands
+// are known: in norm_usual and norms (the ratio of two components from 2^-900 up,
+// and sums of squares that are 0 or above 2^-67), in solve (which see) and for what
+// a norm is divided by.  Everything else divides.
 // ---------------------------------------------------------------------------
 // v_rcp_f64 and two Newton steps: the reciprocal a division starts from.
 NRG_DI double recip(double d)
@@ -283,14 +287,14 @@ NRG_DI double recip(double d)
   return __builtin_fma(r, e, r);
 }
 // n / d from r = recip(d): quotient, remainder, correction, and the fix-up of
-// zeros, infinities and NaN.
+// zeros, infinities and NaN.  The bits of n / d where n is 0, infinite, NaN or above
+// 2^-969, and |d| and |n / d| within 2^+-1000.
 NRG_DI double div_by(double n, double d, double r)
 {
   const double q = n * r;
   const double e = __builtin_fma(-d, q, n);
   return __builtin_amdgcn_div_fixup(__builtin_fma(e, r, q), d, n);
 }
-NRG_DI double quot(double n, double d) { return div_by(n, d, recip(d)); }
 // without the fix-up: n and d finite, d != 0 (else the result is not used)
 NRG_DI double quot_raw(double n, double d)
 {
@@ -339,23 +343,15 @@ enum PowUse : int { POW_FIRST = 0, POW_SELECT, POW_CONV, POW_ERR };
 // work counters, counter i in lane i of the group
 enum WorkLane : int { WORK_NFE = 0, WORK_NJE, WORK_NCORR, WORK_NATT };
 
-// Uniform constants of a call with the reciprocals they are divided by.
-struct GroupConst {
-  double sqrtn, rsqrtn, eps, reps;
-};
-NRG_DI double uniform(double v)
-{
-  const long long x = __double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)x);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(x >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
 NRG_DI double el_of(const BdfCoef &mc, int j, int nq) { return mc.el[nq - 1][j - 1]; }
+// What the error test compares, nrm / (TQ(2, nq) sqrt(N)), and the same over sqrt(N):
+// div_by gives a quotient's bits from 2^-969 up, and below that no decision hangs on
+// them (EPS is at least UROUND here, and the powers end at UROUND).
+NRG_DI double over_tq2(const BdfCoef &mc, double nrm, int nq) { return div_by(nrm, mc.den[1][nq - 1], mc.rden2[nq - 1]); }
 // v / (TQ(k, nq) sqrt(N))
 NRG_DI double over_tq(const BdfCoef &mc, double v, int k, int nq)
 {
-  return div_by(v, mc.den[k - 1][nq - 1], mc.rden[k - 1][nq - 1]);
+  return v / mc.den[k - 1][nq - 1];
 }
 
 // Net stoichiometric coefficient of species s in reaction r (right - left terms).
@@ -384,7 +380,7 @@ struct Cell {
   double yh[MAXORD + 1];         // yh[j] = YH(sub, j+1)
   double y, ywt, save1, save2, fac;
   double p[SA];                  // row `sub` of the factors: L left of the diagonal, U from it on
-  double pd, prd;                // U(sub, sub) and its reciprocal
+  double pd, prd;                // U(sub, sub) and its reciprocal (NaN where div_by cannot use it)
   int src;                       // component of a right-hand side that DGESL's interchanges bring here
   double t, h, rc, rmax, trend, told, d1, nrm;
   int nq, nwait, jtask, jstepl, nstep, work;
@@ -459,7 +455,7 @@ NRG_DI double max_before(const Lane &ln, double v)
 // larger one on unscaled.  HITEST keeps DDRIV3's N (all species).
 // -------------------------------------------------------------------------
 // All phases, one component after the other, over the N values in the group's
-// exchange space (a component at or above HITEST, or NaN; all species).
+// exchange space (where one is unusual, or of all species).
 template <int N>
 NRG_DI double norm_serial(const Lane &ln)
 {
@@ -511,6 +507,25 @@ NRG_DI double norm_serial(const Lane &ln)
   return (st == 4) ? sqrt(sum) : xmax * sqrt(sum);
 }
 
+// A component that takes all phases: at or above HITEST, NaN, or so small that the
+// quotients would have to be scaled, which zero is not.
+NRG_DI bool unusual(const BdfConst &k, double v) { return !(fabs(v) < NRM_HITEST) || (fabs(v) < k.tiny && v != 0.0); }
+// The same of NV vectors: every lane gets the norm of vector `mine`.
+template <int NV>
+NRG_DI double norms_serial(const Lane &ln, const double (&v)[NV], int mine)
+{
+  double out = 0.0;
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    *own(ln, CX) = v[j];
+    wave_sync();
+    const double nrm = norm_serial<SA>(ln);
+    out = j == mine ? nrm : out;
+    wave_sync();
+  }
+  return out;
+}
+
 // Norms of NV vectors: every lane gets that of vector `mine`, so that the sums
 // of two vectors run side by side.
 //
@@ -519,29 +534,15 @@ NRG_DI double norm_serial(const Lane &ln)
 // path.  Each lane knows the maximum of the tiny components before its own
 // from a scan, so its quotient is formed beside the others'; only the sum runs
 // in order, as sum = a + sum * b with (a, b) = (r^2, 1) below the running
-// maximum, (1, r^2) at a new one and (0, 1) elsewhere.  Components under
-// 2^-960 count as zeros: they can change a norm only where it is far below any
-// it is compared with.
+// maximum, (1, r^2) at a new one and (0, 1) elsewhere.
 template <int NV>
-NRG_DI double norms(const Lane &ln, const double (&v)[NV], int mine)
+NRG_DI double norms(const Lane &ln, const BdfConst &k, const double (&v)[NV], int mine)
 {
   bool over = false;
 #pragma unroll
-  for (int j = 0; j < NV; ++j)
-    over = over || !(fabs(v[j]) < NRM_HITEST);
+  for (int j = 0; j < NV; ++j) over = over || unusual(k, v[j]);
   wave_sync();
-  if (wave_any(over)) {
-    double out = 0.0;
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      *own(ln, CX) = v[j];
-      wave_sync();
-      const double nrm = norm_serial<SA>(ln);
-      out = j == mine ? nrm : out;
-      wave_sync();
-    }
-    return out;
-  }
+  if (__builtin_expect(wave_any(over), 0)) return norms_serial(ln, v, mine);
   double xmax = 0.0;
   bool none = false;
 #pragma unroll
@@ -550,7 +551,7 @@ NRG_DI double norms(const Lane &ln, const double (&v)[NV], int mine)
     const unsigned below = (big & (0u - big)) - 1u;  // the lanes ahead of the first large component
     const double av = fabs(v[j]);
     const bool ahead = ((below >> ln.sub) & 1u) != 0u;
-    const bool tin = ahead && av >= 0x1p-960;
+    const bool tin = ahead && v[j] != 0.0;
     const double p = tin ? av : 0.0;
     const double before = max_before(ln, p);
     const double all = bcast<G - 1>(fmax(before, p));
@@ -589,17 +590,13 @@ NRG_DI double ordered_sum(double a, double b1, double b2, std::integer_sequence<
   ((s = bcast<I>(I == 0 ? a : a + (s * b1) * b2)), ...);
   return s;
 }
-NRG_DI double norm(const Lane &ln, double v)
+NRG_DI double norm_usual(const Lane &ln, double v)
 {
   const double av = fabs(v);
-  if (wave_any(!(av < NRM_HITEST))) {
-    const double one[1] = {v};
-    return norms<1>(ln, one, 0);
-  }
   const unsigned big = bits(ln, av > NRM_CUTLO);
   const unsigned first = big & (0u - big), below = first - 1u;
   const bool ahead = ((below >> ln.sub) & 1u) != 0u;
-  const bool tin = ahead && av >= 0x1p-960;
+  const bool tin = ahead && v != 0.0;
   const bool here = ((first >> ln.sub) & 1u) != 0u;
   const double p = tin ? av : 0.0;
   const double before = max_before(ln, p);
@@ -612,6 +609,12 @@ NRG_DI double norm(const Lane &ln, double v)
   const double b2 = here ? xmax : 1.0;
   const double s = root(ordered_sum(a, b1, b2, std::make_integer_sequence<int, SA>{}));
   return big == 0u ? xmax * s : s;
+}
+NRG_DI double norm(const Lane &ln, const BdfConst &k, double v)
+{
+  if (__builtin_expect(!wave_any(unusual(k, v)), 1)) return norm_usual(ln, v);
+  const double one[1] = {v};
+  return norms_serial<1>(ln, one, 0);
 }
 
 // -------------------------------------------------------------------------
@@ -736,7 +739,7 @@ NRG_DI void gefa_step(const Lane &ln, double (&a)[SA], int &pos, bool &singular)
     singular = true;
   } else {
     // DSCAL and DAXPY, which returns at once for DA == 0 (slatec/daxpy.f90:68)
-    const double t = quot(-1.0, piv);
+    const double t = -1.0 / piv;
     a[K] = pos > K ? t * a[K] : a[K];
 #pragma unroll
     for (int i = K + 1; i < SA; ++i) {
@@ -783,7 +786,7 @@ NRG_DI void factor(const Lane &ln, Cell &c, const double (&a)[SA])
 #pragma unroll
   for (int k = 0; k < SA; ++k) c.p[k] = x[k];
   c.pd = x[holds(ln) ? ln.sub : 0];
-  c.prd = recip(c.pd);
+  c.prd = fabs(c.pd) >= 0x1p-20 && fabs(c.pd) <= 0x1p40 ? recip(c.pd) : __builtin_nan("");
   c.src = (int)__double_as_longlong(x[SA]);
   wave_sync();
   c.swapped = bits(ln, holds(ln) && c.src != ln.sub) != 0u;
@@ -798,19 +801,22 @@ NRG_DI void solve_fwd(const Lane &ln, const Cell &c, double &b)
 }
 // A component's sum is complete once the ones after it are through; the
 // quotient by its diagonal is formed wherever it is needed.
-template <int K>
+template <bool FAST>
+NRG_DI double over_diagonal(const Cell &c, double b) { return FAST ? div_by(b, c.pd, c.prd) : b / c.pd; }
+template <int K, bool FAST>
 NRG_DI void solve_back(const Lane &ln, const Cell &c, double &b)
 {
-  const double t = -bcast<K>(div_by(b, c.pd, c.prd));
+  const double t = -bcast<K>(over_diagonal<FAST>(c, b));
   if (ln.sub < K && t != 0.0) b = b + t * c.p[K];
 }
-template <int... K>
+template <bool FAST, int... K>
 NRG_DI void solve_steps(const Lane &ln, const Cell &c, double &b, std::integer_sequence<int, K...>)
 {
   (solve_fwd<K>(ln, c, b), ...);
-  (solve_back<SA - 1 - K>(ln, c, b), ...);
+  (solve_back<SA - 1 - K, FAST>(ln, c, b), ...);
 }
-NRG_DI double solve(const Lane &ln, const Cell &c, double b)
+// The component of b that DGESL's interchanges bring to this lane.
+NRG_DI double interchanged(const Lane &ln, const Cell &c, double b)
 {
   if (wave_any(c.swapped)) {
     wave_sync();
@@ -819,9 +825,19 @@ NRG_DI double solve(const Lane &ln, const Cell &c, double b)
     b = *slot(ln, CX + c.src);
     wave_sync();
   }
-  solve_steps(ln, c, b, std::make_integer_sequence<int, SA - 1>{});
+  return b;
+}
+// FAST: the quotients are div_by's (4 instructions of a serial chain instead of
+// 11).  Where one of them is not what a division gives, its lane's component is
+// unusual once it is weighted: NaN (a diagonal out of range, an overflow), or so
+// small (a numerator under 2^-969 by a diagonal from 2^-20 and a weight from 2^-40
+// up is under 2^-900).  cor then solves with divisions.
+template <bool FAST>
+NRG_DI double solve(const Lane &ln, const Cell &c, double b)
+{
+  solve_steps<FAST>(ln, c, b, std::make_integer_sequence<int, SA - 1>{});
   // a lane without a species keeps zeros
-  return holds(ln) ? div_by(b, c.pd, c.prd) : 0.0;
+  return holds(ln) ? over_diagonal<FAST>(c, b) : 0.0;
 }
 
 // DDPSC (slatec/ddpsc.f90:26-38) for a compile-time order.
@@ -864,9 +880,9 @@ NRG_DI void scl(Cell &c, double rh, const BdfConst &k)
 {
   const double ah = fabs(c.h);
   if (c.h < 1.0)
-    rh = quot(dmin(dmin(ah * rh, ah * c.rmax), k.hmax), ah);
+    rh = dmin(dmin(ah * rh, ah * c.rmax), k.hmax) / ah;
   else
-    rh = dmin(dmin(rh, c.rmax), quot(k.hmax, ah));
+    rh = dmin(dmin(rh, c.rmax), k.hmax / ah);
   double r1 = 1.0;
 #pragma unroll
   for (int j = 1; j <= MAXORD; ++j) {
@@ -881,19 +897,27 @@ NRG_DI void scl(Cell &c, double rh, const BdfConst &k)
 
 // DDCOR, MITER = 2, IMPL = 0, IERROR = 3 (slatec/ddcor.f90:51-54,98-108); the
 // norm before its division by sqrt(N).
-NRG_DI double cor(const Lane &ln, Cell &c)
+NRG_DI double cor(const Lane &ln, Cell &c, const BdfConst &k)
 {
-  const double x = solve(ln, c, ((c.h * c.save2) - c.yh[1]) - c.save1);
+  const double b = interchanged(ln, c, ((c.h * c.save2) - c.yh[1]) - c.save1);
+  double x = solve<true>(ln, c, b), v = x / weight(c), nrm;
+  if (__builtin_expect(!wave_any(unusual(k, v)), 1)) {
+    nrm = norm_usual(ln, v);
+  } else {
+    x = solve<false>(ln, c, b);
+    const double one[1] = {x / weight(c)};
+    nrm = norms_serial<1>(ln, one, 0);
+  }
   c.save1 = c.save1 + x;
   count(ln, c, WORK_NCORR);
-  return norm(ln, quot(x, weight(c)));
+  return nrm;
 }
 
 // DDNTP, K = 0 (slatec/ddntp.f90:25-32).
 NRG_DI void ntp(Cell &c, double tout)
 {
   c.y = yh_col(c, c.nq);
-  const double r = quot(tout - c.t, c.h);
+  const double r = (tout - c.t) / c.h;
 #pragma unroll
   for (int j = MAXORD; j >= 1; --j) c.y = (j <= c.nq) ? c.yh[j - 1] + r * c.y : c.y;
 }
@@ -946,8 +970,7 @@ NRG_DI void bdf_init(Cell &c, double tout, const BdfConst &k)
 // every transition taken in one pass goes forward.  Each stage's code exists
 // once, is skipped by the whole wave when no group sits at it, and a group may
 // pass several stages per call.
-NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, const GroupConst &gc,
-                    const BdfCoef &mc)
+NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, const BdfCoef &mc)
 {
   // what a stage hands to a later one of the same pass
   double ctest = 0.0, rh = 0.0;
@@ -957,9 +980,9 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
   // ---- rest of DDNTL after its f(y) (slatec/ddntl.f90:68,152-161)
   if (wave_any(c.pc == PC_NTL_F) && c.pc == PC_NTL_F) {
     count(ln, c, WORK_NFE);
-    c.save1 = quot(c.save2, dmax(1.0, c.ywt));
-    const double sum = div_by(norm(ln, c.save1), gc.sqrtn, gc.rsqrtn);
-    if (sum > quot(gc.eps, fabs(c.h))) c.h = copysign(quot(gc.eps, sum), c.h);
+    c.save1 = c.save2 / dmax(1.0, c.ywt);
+    const double sum = norm(ln, k, c.save1) / k.sqrtn;
+    if (sum > k.eps / fabs(c.h)) c.h = copysign(k.eps / sum, c.h);
     c.yh[1] = c.h * c.save2;
     c.fac = k.sqrt_uround;
     if (c.ntl_restart) c.rmax = 10.0;
@@ -996,12 +1019,12 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
   }
   // ---- corrector iteration, label 130 (slatec/ddstp.f90:152-205)
   if (wave_any(c.pc == PC_CORR) && c.pc == PC_CORR) {
-    c.nrm = cor(ln, c);
-    const double d = div_by(c.nrm, gc.sqrtn, gc.rsqrtn);
-    if (c.iter > 0) c.trend = dmax(0.9 * c.trend, quot(d, c.d1));
+    c.nrm = cor(ln, c, k);
+    const double d = div_by(c.nrm, k.sqrtn, mc.rsqrtn);
+    if (c.iter > 0) c.trend = dmax(0.9 * c.trend, d / c.d1);
     c.d1 = d;
     ctest = dmin(2.0 * c.trend, 1.0) * d;
-    if (ctest <= gc.eps) {
+    if (ctest <= k.eps) {
       c.pc = PC_ERRTEST;
     } else {
       c.iter++;
@@ -1032,8 +1055,8 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
     c.convrg = true;
     // the norm of the sum of the corrections: after one iteration it is the
     // corrector's own
-    if (wave_any(c.iter > 0) && c.iter > 0) c.nrm = norm(ln, quot(c.save1, weight(c)));
-    if (over_tq(mc, c.nrm, 2, c.nq) > gc.eps) {
+    if (wave_any(c.iter > 0) && c.iter > 0) c.nrm = norm(ln, k, c.save1 / weight(c));
+    if (over_tq2(mc, c.nrm, c.nq) > k.eps) {
       use = POW_ERR;                                   // (:238-289)
       c.pc = PC_RETRACT;
     } else {
@@ -1086,29 +1109,29 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
   // whatever its vector holds and then not used.
   if (wave_any(c.pc == PC_POW) && c.pc == PC_POW) {
     const int cand = ln.sub < 2 ? ln.sub : 2;
-    const double etest = over_tq(mc, c.nrm, 2, c.nq);
+    const double etest = over_tq2(mc, c.nrm, c.nq);
     const int kt = cand == 2 ? 2 : 0;
-    const double den = mc.den[kt][c.nq - 1], rden = mc.rden[kt][c.nq - 1];
+    const double den = mc.den[kt][c.nq - 1];
     py = mc.inv[c.nq + cand];
     double err = etest;
     const bool need = use == POW_SELECT || (use == POW_ERR && c.nq > 1);
     if (wave_any(need) && need) {
-      const double w = weight(c), rw = recip(w);
-      const double v[2] = {div_by(yh_col(c, c.nq), w, rw), div_by(c.save1 - c.yh[MAXORD], w, rw)};
-      const double nrm = norms<2>(ln, v, cand == 2 ? 1 : 0);
-      const double e = div_by(nrm, den, rden);
+      const double w = weight(c);
+      const double v[2] = {yh_col(c, c.nq) / w, (c.save1 - c.yh[MAXORD]) / w};
+      const double nrm = norms<2>(ln, k, v, cand == 2 ? 1 : 0);
+      const double e = nrm / den;
       err = cand == 1 ? etest : e;
     }
-    px = div_by(err, gc.eps, gc.reps);
+    px = err / k.eps;
     if (use == POW_CONV) {
-      px = c.iter == 0 ? 1.0 : quot(gc.eps, ctest);
+      px = c.iter == 0 ? 1.0 : k.eps / ctest;
       py = 0.2;
     }
     const double pw = pow(px, py);
     // 1 / max(floor, bias * power), biases 1.3, 1.2, 1.4
     const double bias = cand == 0 ? 1.3 : cand == 1 ? 1.2 : 1.4;
     const double floor_ = use == POW_ERR ? (cand == 0 ? 1.0 : 0.0) : k.uround;
-    const double rc_ = quot(1.0, dmax(floor_, bias * pw));
+    const double rc_ = 1.0 / dmax(floor_, bias * pw);
     const double ra = bcast<0>(rc_), rb = bcast<1>(rc_), ru = bcast<2>(rc_);
     const int nq0 = c.nq;
     c.pc = PC_SCALE;
@@ -1130,9 +1153,9 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
         rh = rh3;
         do_scale = !(rh <= 1.0);
         if (do_scale) {
-          const double l = el_of(mc, c.nq + 1, c.nq), den = (double)(c.nq + 1), rden = recip(den);
+          const double l = el_of(mc, c.nq + 1, c.nq), den = (double)(c.nq + 1);
           const int dst = c.nq + 1;
-          const double newc = div_by(c.save1 * l, den, rden);
+          const double newc = (c.save1 * l) / den;
 #pragma unroll
           for (int j = 2; j <= MAXORD; ++j) c.yh[j] = (dst == j) ? newc : c.yh[j];
           c.nq = c.nq + 1;
@@ -1155,7 +1178,7 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
         finish(c, OUT_STEP_ZERO);
       }
     }
-    if (c.nq != nq0) c.rc = quot(c.rc * el_of(mc, 1, c.nq), el_of(mc, 1, nq0));
+    if (c.nq != nq0) c.rc = (c.rc * el_of(mc, 1, c.nq)) / el_of(mc, 1, nq0);
     if (use == POW_SELECT || use == POW_ERR) c.nwait = c.nq + 2;
   }
   // ---- pending DDSCL, then the next attempt or DDRIV3's label 470
@@ -1182,7 +1205,7 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
     // and EPS < SUM * UROUND cannot hold for EPS >= 2 * UROUND; the norm is
     // formed only when it can decide.
     bool eps_fail = false;
-    if (gc.eps < 2.0 * k.uround) {
+    if (k.eps < 2.0 * k.uround) {
       // over all species, in their order; the inert ones keep their initial concentration
       wave_sync();
       if (holds(ln)) *own(ln, CZ) = c.y;
@@ -1196,9 +1219,9 @@ NRG_DI void advance(const Lane &ln, Cell &c, double tout, const BdfConst &k, con
         }
       }
       wave_sync();
-      double sum = norm_serial<S>(ln) / gc.sqrtn;
+      double sum = norm_serial<S>(ln) / k.sqrtn;
       sum = dmax(1.0, sum);
-      eps_fail = gc.eps < sum * k.uround;
+      eps_fail = k.eps < sum * k.uround;
     }
     if (eps_fail) {
       c.y = c.yh[0];
@@ -1271,7 +1294,7 @@ NRG_DI void jac_fd(const Lane &ln, Cell &c, const BdfConst &k, const BdfCoef &mc
 #pragma unroll
   for (int q = 0; q < SA; ++q) z[q] = (q == ln.sub) ? yp : *slot(ln, CZ + q);
   rhs_lane(ln, z, f1);
-  const double scale_ = quot((-l0) * c.h, dy);
+  const double scale_ = ((-l0) * c.h) / dy;
   double diff = 0.0, s2m = 0.0, s1m = 0.0;
 #pragma unroll
   for (int i = 0; i < SA; ++i) {

@@ -18,11 +18,10 @@
 // What bounds it: FP64 VALU issue and its latency (the state takes the whole
 // register file: one wave per SIMD), and lanes that wait while others of their
 // wave pass a stage.  Cells of equal cost, which stiffness order brings
-// together, keep that share small; 65,536 cells fill the chip once.  With the
-// divisions of bdf_group.h (9 or 4 instructions instead of 13) and one path
-// through the norm instead of the walk through its phases, 1M flame cells went
-// from 16.5 to 14.6 ms, 2.1M cells with hot kernels from 5.4 to 4.9 and 1M
-// igniting ones from 19.6 to 17.3.
+// together, keep that share small; 65,536 cells fill the chip once.  The norm has
+// one path for ordinary vectors instead of the walk through its phases.  Kernel
+// time in stiffness order with a history: 1M flame cells 12.0 ms, 2.1M cells with
+// hot kernels 3.8, 1M igniting ones 15.1.
 //
 // Reference: computing_module/src/current_build/chemical_kinetics_solver.f90
 // (RHS :495-540, cell step :228-346) and SLATEC SDRIVE in
@@ -171,8 +170,9 @@ NRG_DI double dnrm2_phases_seq(const double *x, std::integer_sequence<int, I...>
   return dnrm2_phases_vals(x[I]...);
 }
 
-// (Components under 2^-960 count as zeros: they can change a norm only where it
-// is far below any it is compared with.)
+// (Components under 2^-960 count as zeros: beside a larger maximum than 2^-900
+// their squares are less than half an ulp of the sum, which is 1 at least, and
+// vectors that end below that take all phases.)
 template <int n>
 NRG_DI double dnrm2_core(const double *x)
 {
@@ -197,6 +197,12 @@ NRG_DI double dnrm2_core(const double *x)
       }
     }
     sum = scaled ? sum : sum + v * v;
+  }
+  if (scaled && xmax < 0x1p-900) {
+    bool zero = true;
+#pragma unroll
+    for (int i = 0; i < n; ++i) zero = zero && x[i] == 0.0;
+    if (!zero) return dnrm2_phases_seq(x, std::make_integer_sequence<int, n>{});
   }
   const double s = root(sum);
   return scaled ? xmax * s : s;
@@ -312,7 +318,7 @@ NRG_DI void gefa_col(double (&a)[SA][SA], int (&ipvt)[SA], int &info)
     a[K][K] = piv;
   }
   // DSCAL of the column below the pivot (skipped for a zero pivot)
-  const double t = quot(-1.0, a[K][K]);
+  const double t = -1.0 / a[K][K];
   if (wave_any(zero)) {
 #pragma unroll
     for (int i = K + 1; i < SA; ++i) a[K][i] = zero ? a[K][i] : t * a[K][i];
@@ -367,7 +373,7 @@ NRG_DI void gesl_fwd(const double (&a)[SA][SA], const int (&ipvt)[SA], double (&
 template <int K>
 NRG_DI void gesl_back(const double (&a)[SA][SA], double (&b)[SA])
 {
-  b[K] = quot(b[K], a[K][K]);
+  b[K] = b[K] / a[K][K];
   const double t = -b[K];
   daxpy_head<K>(t == 0.0, t, a[K], b);
 }
@@ -466,9 +472,9 @@ NRG_DI void scl(Cell &c, double rh, const BdfConst &k)
 {
   const double ah = fabs(c.h);
   if (c.h < 1.0)
-    rh = quot(dmin(dmin(ah * rh, ah * c.rmax), k.hmax), ah);
+    rh = dmin(dmin(ah * rh, ah * c.rmax), k.hmax) / ah;
   else
-    rh = dmin(dmin(rh, c.rmax), quot(k.hmax, ah));
+    rh = dmin(dmin(rh, c.rmax), k.hmax / ah);
   double r1 = 1.0;
 #pragma unroll
   for (int j = 1; j <= MAXORD; ++j) {
@@ -482,7 +488,7 @@ NRG_DI void scl(Cell &c, double rh, const BdfConst &k)
 }
 
 // DDCOR, MITER = 2, IMPL = 0, IERROR = 3 (slatec/ddcor.f90:51-54,98-108).
-NRG_DI double cor(Cell &c, const GroupConst &gc)
+NRG_DI double cor(Cell &c, const BdfConst &k)
 {
 #pragma unroll
   for (int i = 0; i < SA; ++i) c.save2[i] = ((c.h * c.save2[i]) - c.yh[1][i]) - c.save1[i];
@@ -490,10 +496,10 @@ NRG_DI double cor(Cell &c, const GroupConst &gc)
 #pragma unroll
   for (int i = 0; i < SA; ++i) {
     c.save1[i] = c.save1[i] + c.save2[i];
-    c.save2[i] = quot(c.save2[i], dmax(fabs(c.y[i]), c.ywt[i]));
+    c.save2[i] = c.save2[i] / dmax(fabs(c.y[i]), c.ywt[i]);
   }
   c.ncorr++;
-  return div_by(dnrm2(c.save2), gc.sqrtn, gc.rsqrtn);
+  return dnrm2(c.save2) / k.sqrtn;
 }
 
 // DDNTP, K = 0 (slatec/ddntp.f90:25-32).
@@ -503,7 +509,7 @@ NRG_DI void ntp(Cell &c, double tout)
   yh_col(c, c.nq, col);
 #pragma unroll
   for (int i = 0; i < SA; ++i) c.y[i] = col[i];
-  const double r = quot(tout - c.t, c.h);
+  const double r = (tout - c.t) / c.h;
 #pragma unroll
   for (int j = MAXORD; j >= 1; --j) {
     const bool on = (j <= c.nq);
@@ -585,15 +591,15 @@ NRG_DI bool at(const Cell &c, int pc) { return c.req == REQ_NONE && c.pc == pc; 
 //   4 error test, accept, step/order choice (label 170)
 //   5 corrector failure (label 160)   6 DDRIV3 label 260   7 attempt (label 100)
 // Each stage's code exists once; a lane may pass several stages per call.
-NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &gc, const BdfCoef &mc)
+NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const BdfCoef &mc)
 {
   // ---- 1: rest of DDNTL after its f(y) (slatec/ddntl.f90:68,152-161)
   if (wave_any(at(c, PC_NTL_F)) && at(c, PC_NTL_F)) {
     c.nfe++;
 #pragma unroll
-    for (int i = 0; i < SA; ++i) c.save1[i] = quot(c.save2[i], dmax(1.0, c.ywt[i]));
-    const double sum = div_by(dnrm2(c.save1), gc.sqrtn, gc.rsqrtn);
-    if (sum > quot(gc.eps, fabs(c.h))) c.h = copysign(quot(gc.eps, sum), c.h);
+    for (int i = 0; i < SA; ++i) c.save1[i] = c.save2[i] / dmax(1.0, c.ywt[i]);
+    const double sum = dnrm2(c.save1) / k.sqrtn;
+    if (sum > k.eps / fabs(c.h)) c.h = copysign(k.eps / sum, c.h);
 #pragma unroll
     for (int i = 0; i < SA; ++i) c.yh[1][i] = c.h * c.save2[i];
 #pragma unroll
@@ -636,8 +642,8 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
   }
   // ---- 3: corrector iteration, label 130 (slatec/ddstp.f90:152-205)
   if (wave_any(at(c, PC_CORR)) && at(c, PC_CORR)) {
-    const double d = cor(c, gc);
-    if (c.iter > 0) c.trend = dmax(0.9 * c.trend, quot(d, c.d1));
+    const double d = cor(c, k);
+    if (c.iter > 0) c.trend = dmax(0.9 * c.trend, d / c.d1);
     c.d1 = d;
     c.ctest = dmin(2.0 * c.trend, 1.0) * d;
     if (c.ctest <= k.eps) {
@@ -670,7 +676,7 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
   if (n4 > 0 && n4 * 100 >= k.gather_pct * nact && here4) {
     c.convrg = true;
 #pragma unroll
-    for (int i = 0; i < SA; ++i) c.save2[i] = quot(c.save1[i], dmax(fabs(c.y[i]), c.ywt[i]));
+    for (int i = 0; i < SA; ++i) c.save2[i] = c.save1[i] / dmax(fabs(c.y[i]), c.ywt[i]);
     const double etest = over_tq(mc, dnrm2(c.save2), 2, c.nq);
     c.etest = etest;
     if (etest > k.eps) {
@@ -693,7 +699,7 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
       c.after_accept = true;
       // step-size and order selection (slatec/ddstp.f90:360-432)
       if (c.jtask == 0 || c.jtask == 2) {
-        const double rh = quot(1.0, dmax(k.uround, 1.2 * nl_pow(div_by(etest, gc.eps, gc.reps), mc.inv[c.nq + 1])));
+        const double rh = 1.0 / dmax(k.uround, 1.2 * nl_pow(etest / k.eps, mc.inv[c.nq + 1]));
         c.rh = rh;
         c.do_scale = rh > 1.0;
       } else if (c.nwait > 1) {
@@ -711,18 +717,18 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
         yh_col(c, c.nq, dn);
 #pragma unroll
         for (int i = 0; i < SA; ++i) {
-          const double w = dmax(fabs(c.y[i]), c.ywt[i]), rw = recip(w);
-          dn[i] = div_by(dn[i], w, rw);
-          up[i] = div_by(c.save1[i] - c.yh[MAXORD][i], w, rw);
+          const double w = dmax(fabs(c.y[i]), c.ywt[i]);
+          dn[i] = dn[i] / w;
+          up[i] = (c.save1[i] - c.yh[MAXORD][i]) / w;
         }
         const Norm2 nr = dnrm2_pair(dn, up);
         const double erdn = over_tq(mc, nr.a, 1, c.nq);
         const double erup = over_tq(mc, nr.b, 3, c.nq);
-        const Pow3 pw = nl_pow3(div_by(erdn, gc.eps, gc.reps), mc.inv[c.nq], div_by(etest, gc.eps, gc.reps),
-                                mc.inv[c.nq + 1], div_by(erup, gc.eps, gc.reps), mc.inv[c.nq + 2]);
-        const double rh1 = (c.nq != 1) ? quot(1.0, dmax(k.uround, 1.3 * pw.a)) : 0.0;
-        const double rh2 = quot(1.0, dmax(k.uround, 1.2 * pw.b));
-        const double rh3 = (c.nq != k.maxord) ? quot(1.0, dmax(k.uround, 1.4 * pw.c)) : 0.0;
+        const Pow3 pw = nl_pow3(erdn / k.eps, mc.inv[c.nq], etest / k.eps,
+                                mc.inv[c.nq + 1], erup / k.eps, mc.inv[c.nq + 2]);
+        const double rh1 = (c.nq != 1) ? 1.0 / dmax(k.uround, 1.3 * pw.a) : 0.0;
+        const double rh2 = 1.0 / dmax(k.uround, 1.2 * pw.b);
+        const double rh3 = (c.nq != k.maxord) ? 1.0 / dmax(k.uround, 1.4 * pw.c) : 0.0;
         double rh;
         bool change = true;
         if (rh1 > rh2 && rh1 >= rh3) {
@@ -731,7 +737,7 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
             change = false;
           } else {
             c.nq = c.nq - 1;
-            c.rc = quot(c.rc * el_of(mc, 1, c.nq), el_of(mc, 1, c.nq + 1));
+            c.rc = (c.rc * el_of(mc, 1, c.nq)) / el_of(mc, 1, c.nq + 1);
           }
         } else if (rh2 >= rh1 && rh2 >= rh3) {
           rh = rh2;
@@ -742,18 +748,18 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
             change = false;
           } else {
             const double e = el_of(mc, c.nq + 1, c.nq);
-            const double den = (double)(c.nq + 1), rden = recip(den);
+            const double den = (double)(c.nq + 1);
             const int dst = c.nq + 1;
             double newc[SA];
 #pragma unroll
-            for (int i = 0; i < SA; ++i) newc[i] = div_by(c.save1[i] * e, den, rden);
+            for (int i = 0; i < SA; ++i) newc[i] = (c.save1[i] * e) / den;
 #pragma unroll
             for (int j = 2; j <= MAXORD; ++j) {
 #pragma unroll
               for (int i = 0; i < SA; ++i) c.yh[j][i] = (dst == j) ? newc[i] : c.yh[j][i];
             }
             c.nq = c.nq + 1;
-            c.rc = quot(c.rc * el_of(mc, 1, c.nq), el_of(mc, 1, c.nq - 1));
+            c.rc = (c.rc * el_of(mc, 1, c.nq)) / el_of(mc, 1, c.nq - 1);
           }
         }
         c.rh = rh;
@@ -778,7 +784,7 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
     if (!c.fail_err) {                                 // label 160
       c.nwait = c.nq + 2;
       if (c.jtask != 0 && c.jtask != 2) c.rmax = 2.0;
-      const double rh = (c.iter == 0) ? 0.3 : 0.9 * nl_pow(quot(gc.eps, c.ctest), 0.2);
+      const double rh = (c.iter == 0) ? 0.3 : 0.9 * nl_pow(k.eps / c.ctest, 0.2);
       if (rh * c.h == 0.0) {
         copy_yh0_to_y(c);
         finish(c, OUT_STEP_ZERO);
@@ -791,18 +797,18 @@ NRG_DI void advance(Cell &c, double tout, const BdfConst &k, const GroupConst &g
       c.nfail++;
       if (c.nfail < 3 || c.nq == 1) {
         if (c.jtask != 0 && c.jtask != 2) c.rmax = 2.0;
-        const double rh2 = quot(1.0, 1.2 * nl_pow(div_by(c.etest, gc.eps, gc.reps), mc.inv[c.nq + 1]));
+        const double rh2 = 1.0 / (1.2 * nl_pow(c.etest / k.eps, mc.inv[c.nq + 1]));
         double rh = rh2;
         if (c.nq > 1) {
           double col[SA];
           yh_col(c, c.nq, col);
 #pragma unroll
-          for (int i = 0; i < SA; ++i) c.save2[i] = quot(col[i], dmax(fabs(c.y[i]), c.ywt[i]));
+          for (int i = 0; i < SA; ++i) c.save2[i] = col[i] / dmax(fabs(c.y[i]), c.ywt[i]);
           const double erdn = over_tq(mc, dnrm2(c.save2), 1, c.nq);
-          const double rh1 = quot(1.0, dmax(1.0, 1.3 * nl_pow(div_by(erdn, gc.eps, gc.reps), mc.inv[c.nq])));
+          const double rh1 = 1.0 / dmax(1.0, 1.3 * nl_pow(erdn / k.eps, mc.inv[c.nq]));
           if (rh2 < rh1) {
             c.nq = c.nq - 1;
-            c.rc = quot(c.rc * el_of(mc, 1, c.nq), el_of(mc, 1, c.nq + 1));
+            c.rc = (c.rc * el_of(mc, 1, c.nq)) / el_of(mc, 1, c.nq + 1);
             rh = rh1;
           }
         }
@@ -948,7 +954,7 @@ NRG_DI void jac_batch(Cell &c, bool mine, const BdfConst &k, const BdfCoef &mc, 
       rhs(kl, c.y, f1);
 #pragma unroll
       for (int q = 0; q < SA; ++q) c.y[q] = (q == j) ? yj : c.y[q];
-      const double factor = quot((-l0) * c.h, dy);
+      const double factor = ((-l0) * c.h) / dy;
       double col[SA];
 #pragma unroll
       for (int i = 0; i < SA; ++i) col[i] = (f1[i] - c.save2[i]) * factor;

@@ -59,7 +59,7 @@ struct MechCoef {
 struct BdfCoef {
   double el[MAXORD][MAXORD + 1];
   double den[3][MAXORD];         // den[k-1][nq-1] = TQ(k, nq) * sqrt(N)
-  double rden[3][MAXORD];        // what a division by it starts from
+  double rsqrtn, rden2[MAXORD];  // what div_by takes of sqrt(N) and of den[1]
   double inv[8];                 // 1 / n
   double W[S];
   double h_ref[S];
@@ -68,6 +68,7 @@ struct BdfCoef {
 // Integrator constants of one call (reference literals + D1MACH-derived values).
 struct BdfConst {
   double eps, ewt, hmax, uround, sqrtn, sqrt_uround;
+  double tiny;                   // weighted components below it take DNRM2's phases one by one
   double br, bl, bp, facmin;     // u**.875, u**.75, u**-.15, u**.78 (slatec/ddpst.f90:54-57)
   double t_gate;
   int mxstep, maxord;

@@ -210,8 +210,9 @@ NRG_DI void stage_bdf(BdfCoef &dst, const MechCoef *src, double sqrtn)
   for (int i = threadIdx.x; i < 3 * MAXORD; i += blockDim.x) {
     const double d = src->tq[i % MAXORD][i / MAXORD] * sqrtn;
     (&dst.den[0][0])[i] = d;
-    (&dst.rden[0][0])[i] = recip(d);
+    if (i / MAXORD == 1) dst.rden2[i % MAXORD] = recip(d);
   }
+  if (threadIdx.x == 0) dst.rsqrtn = recip(sqrtn);
   if (threadIdx.x < 8) dst.inv[threadIdx.x] = 1.0 / (double)(int)threadIdx.x;
   for (int i = threadIdx.x; i < S; i += blockDim.x) {
     dst.W[i] = src->W[i];
@@ -362,7 +363,6 @@ NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, const Cell &c, con
   wave_sync();
   const long long q = __double_as_longlong(*slot(ln, CCELL));
   const long long off = __double_as_longlong(*slot(ln, CCELL + 1));
-  const double rdt = recip(a.dt);
 #pragma unroll
   for (int s0 = 0; s0 < S; s0 += G) {
     const int s = s0 + ln.sub;
@@ -371,9 +371,9 @@ NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, const Cell &c, con
       const double cin = *slot(ln, 2 * REC_C + s);
       const double ys = inert_species(s) ? cin : *slot(ln, CZ + active_slot(s));
       const double dc = ys - cin;
-      a.Yp[s][off] = div_by(dc * mc.W[s], a.dt, rdt);
+      a.Yp[s][off] = (dc * mc.W[s]) / a.dt;
       a.Yp2[s][off] = dc;
-      *slot(ln, CX + s) = div_by(mc.h_ref[s] * dc, a.dt, rdt);
+      *slot(ln, CX + s) = (mc.h_ref[s] * dc) / a.dt;
     }
   }
   wave_sync();
@@ -459,7 +459,6 @@ extern template __global__ void chem_bdf_kernel<true>(StepArgs);
   const int lane = threadIdx.x;
   if (lane < ACC_QUEUE0) tally[lane] = 0ull;
   stage_bdf(mc, a.mech, a.k.sqrtn);
-  const GroupConst gc = {a.k.sqrtn, uniform(recip(a.k.sqrtn)), a.k.eps, uniform(recip(a.k.eps))};
   Lane ln;
   group_init(ln, (lds_double *)cells, (lds_word *)table, ANALYTIC ? (lds_word *)jtable : nullptr, lane);
   Cell c;
@@ -502,7 +501,7 @@ extern template __global__ void chem_bdf_kernel<true>(StepArgs);
         jac_fd(ln, c, a.k, mc);
       c.pc &= 15;
     }
-    if (c.pc < PC_WAIT_F) advance(ln, c, a.dt, a.k, gc, mc);
+    if (c.pc < PC_WAIT_F) advance(ln, c, a.dt, a.k, mc);
     if ((c.pc & PC_DONE) && c.pc != PC_IDLE) {
       finish_cell(a, mc, c, ln, tally);
       c.pc = PC_IDLE;
@@ -575,16 +574,15 @@ struct LaneTally {
 NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, long long q, long long off,
                         const lane::Cell &c, const double *kl, LaneTally &tl, unsigned long long *tally)
 {
-  const double rdt = recip(a.dt);
   double ef = 0.0;
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     const double cin = lane::rec_c(kl, s);   // the initial concentration as rates_kernel recorded it
     const double ys = (kSp.act[s] >= 0) ? c.y[kSp.act[s]] : c.yi[kSp.islot[s]];
     const double dc = ys - cin;
-    a.Yp[s][off] = div_by(dc * mc.W[s], a.dt, rdt);
+    a.Yp[s][off] = (dc * mc.W[s]) / a.dt;
     a.Yp2[s][off] = dc;
-    ef = ef - div_by(mc.h_ref[s] * dc, a.dt, rdt);
+    ef = ef - (mc.h_ref[s] * dc) / a.dt;
   }
   a.Efp[off] = ef;
   const int status = (c.outcome == lane::OUT_OK) ? NRG_CELL_OK
@@ -633,7 +631,6 @@ extern template __global__ void chem_bdf_lane_kernel<true>(StepArgs);
   const int lane = threadIdx.x;
   if (lane < ACC_QUEUE0) tally[lane] = 0ull;
   stage_bdf(mc, a.mech, a.k.sqrtn);
-  const GroupConst gc = {a.k.sqrtn, uniform(recip(a.k.sqrtn)), a.k.eps, uniform(recip(a.k.eps))};
   const double *kl = recl + 2 * lane;
   lds_double *recl_lds = (lds_double *)recl;   // the array's LDS address (direct loads' M0)
   lane::Cell c;
@@ -680,7 +677,7 @@ extern template __global__ void chem_bdf_lane_kernel<true>(StepArgs);
       lane::rhs(kl, c.y, c.save2);
     if (have && (c.req == lane::REQ_NONE || (run_jac ? wantj : wantf))) {
       c.req = lane::REQ_NONE;
-      lane::advance(c, a.dt, a.k, gc, mc);
+      lane::advance(c, a.dt, a.k, mc);
     }
     if (have && c.req == lane::REQ_DONE) {
       finish_cell(a, mc, q, off, c, kl, tl, tally);
@@ -929,7 +926,6 @@ __global__ void __launch_bounds__(TABLE_THREADS) table_kernel(TableArgs a)
   // first inner cell's slice to the last inner cell) and skip ghost cells:
   // with ghost layers a row of inner cells starts off a cache line, and
   // walking inner cells would make every wave touch one line more per field.
-  const double rdt = recip(a.dt);
   for (long long off = a.g.pad0 + (long long)blockIdx.x * TABLE_THREADS + threadIdx.x; off < a.g.pad1; off += stride) {
     if (!inner_at(a.g, off)) continue;
     const double T = a.T[off];
@@ -945,11 +941,11 @@ __global__ void __launch_bounds__(TABLE_THREADS) table_kernel(TableArgs a)
       for (int s = 0; s < S; ++s) c[s] = cin[s] = a.Y[s][off];
       const int i = table_interval(Tt, a.rows, a.ascending, T);
       if (i >= 0) {
-        const double t0 = Tt[i], t1 = Tt[i + 1], up = t1 - t0, dn = t0 - t1, rup = recip(up);
+        const double t0 = Tt[i], t1 = Tt[i + 1], up = t1 - t0, dn = t0 - t1;
 #pragma unroll
         for (int s = 0; s < S; ++s)
-          c[s] = div_by(dC[s * a.rows + i + 1] * (T - t0), up, rup) +
-                 div_by(dC[s * a.rows + i] * (T - t1), dn, -rup);
+          c[s] = (dC[s * a.rows + i + 1] * (T - t0)) / up +
+                 (dC[s * a.rows + i] * (T - t1)) / dn;
       }
       if (T < Tt[0]) {
 #pragma unroll
@@ -962,8 +958,8 @@ __global__ void __launch_bounds__(TABLE_THREADS) table_kernel(TableArgs a)
 #pragma unroll
       for (int s = 0; s < S; ++s) {
         put<STREAM>(&a.Yp2[s][off], c[s] - cin[s]);
-        ef = ef - div_by(href[s] * c[s], a.dt, rdt);
-        c[s] = div_by(c[s] * W[s], a.dt, rdt);
+        ef = ef - (href[s] * c[s]) / a.dt;
+        c[s] = (c[s] * W[s]) / a.dt;
       }
     }
     // what gated cells have too, for the whole slice at once
@@ -2237,6 +2233,8 @@ BdfConst make_const(const nrg_chem_opts &o)
   k.hmax = o.hmax;
   k.uround = 2.220446049250313080847e-16;        // epsilon(1d0)
   k.sqrtn = std::sqrt((double)S);
+  // with weights under 2^-40 every component (solve, bdf_group.h)
+  k.tiny = o.ewt >= 0x1p-40 ? 0x1p-900 : INFINITY;
   k.sqrt_uround = std::sqrt(k.uround);
   k.br = std::pow(k.uround, 0.875);
   k.bl = std::pow(k.uround, 0.75);
