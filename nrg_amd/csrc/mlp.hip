@@ -758,6 +758,42 @@ int mlp_infer_bf16(nrg_mlp_t *h, long long n, const bf16 *X, float *Y, hipStream
   return launch_infer(h, n, X, nullptr, Y, stream);
 }
 
+namespace {
+
+// The kernels write rows while other blocks still read theirs, so an input that an
+// output overlaps is read from a copy (a caller may let the outputs take the
+// inputs' place).
+class Apart {
+ public:
+  explicit Apart(hipStream_t s) : stream(s) {}
+  ~Apart() { free_all({copies[0], copies[1], copies[2]}); }   // (waits for the kernels that read them)
+  void output(const float *p, long long n)
+  {
+    if (p) outs[n_outs++] = {p, p + n};
+  }
+  int input(const float *&p, long long n)
+  {
+    bool over = false;
+    for (int i = 0; i < n_outs; ++i) over = over || (p < outs[i].end && outs[i].begin < p + n);
+    if (!p || !over) return NRG_CHEM_OK;
+    void *&c = copies[n_copies++];
+    HIP_TRY(hipMalloc(&c, n * sizeof(float)));
+    HIP_TRY(hipMemcpyAsync(c, p, n * sizeof(float), hipMemcpyDeviceToDevice, stream));
+    p = (const float *)c;
+    return NRG_CHEM_OK;
+  }
+
+ private:
+  hipStream_t stream;
+  struct Range {
+    const float *begin, *end;
+  } outs[3];
+  void *copies[3] = {nullptr, nullptr, nullptr};
+  int n_outs = 0, n_copies = 0;
+};
+
+}  // namespace
+
 hipStream_t mlp_stream(nrg_mlp_t *h) { return h->stream; }
 int mlp_n_out(const nrg_mlp_t *h) { return h->n_out; }
 int mlp_n_in(const nrg_mlp_t *h) { return h->n_in; }
@@ -879,7 +915,10 @@ int nrg_mlp_forward_dev(nrg_mlp_t *h, int64_t n, const float *x, float *y)
   if (!h || (n > 0 && (!x || !y)) || n < 0) return set_error(NRG_CHEM_E_ARG, "bad argument");
   if (n == 0) return NRG_CHEM_OK;
   HIP_TRY(hipSetDevice(h->device));
-  const int rc = launch_infer(h, n, nullptr, x, y, h->stream);
+  Apart apart(h->stream);
+  apart.output(y, n * h->n_out);
+  int rc = apart.input(x, n * h->n_in);
+  if (!rc) rc = launch_infer(h, n, nullptr, x, y, h->stream);
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(h->stream));
   return NRG_CHEM_OK;
@@ -890,7 +929,14 @@ int nrg_mlp_grad_dev(nrg_mlp_t *h, int64_t n, const float *x, const float *t, co
 {
   if (!h || n <= 0 || !x || !t || !grad) return set_error(NRG_CHEM_E_ARG, "bad argument");
   HIP_TRY(hipSetDevice(h->device));
-  int rc = loss_and_grad(h, n, x, t, w, loss, y_out, grad);
+  Apart apart(h->stream);
+  apart.output(grad, h->n_packed);
+  apart.output(loss, 1);
+  apart.output(y_out, n * h->n_out);
+  int rc = apart.input(x, n * h->n_in);
+  if (!rc) rc = apart.input(t, n * h->n_out);
+  if (!rc) rc = apart.input(w, h->n_out);
+  if (!rc) rc = loss_and_grad(h, n, x, t, w, loss, y_out, grad);
   if (rc) return rc;
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(h->stream));
