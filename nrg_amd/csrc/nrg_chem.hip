@@ -3108,6 +3108,7 @@ int nrg_chem_table_step_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, cons
     const size_t dyn = lds ? tab_bytes : 0;
     hipLaunchKernelGGL(kernel, dim3((unsigned)resident_blocks(h, kernel, dyn, a.g)), dim3(TABLE_THREADS), dyn,
                        h->stream, a);
+    HIP_TRY(hipGetLastError());
   }
   HIP_TRY(hipEventRecord(h->ev1, h->stream));
   HIP_TRY(read_counters(h, acc, h->dev_acc, 16));

@@ -1,0 +1,82 @@
+"""What the entry points do when the runtime refuses a launch: an error from the
+call whose launch was refused.  On the CPU, in a process of its own, against a
+runtime without a device (fake_hip.c) that can be told to refuse."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+ROCM = "/opt/rocm/include"
+
+CHILD = r"""
+import ctypes as C, json, os, sys
+sys.modules['torch'] = None   # not needed here, and it brings a runtime of its own
+import numpy as np
+from nrg_amd import capi, mechanism
+lib = capi.load_library()
+fake = C.CDLL(sys.argv[2])
+fake.fake_hip_host_bytes.restype = C.c_size_t
+mech = mechanism.load_mechanism()
+S, n, dt = mech.species_number, int(sys.argv[3]), 1e-7
+m = capi.MechStruct(mech)
+h = C.c_void_p()
+out = {"create": lib.nrg_chem_create(m.ref(), None, C.byref(h))}
+if out["create"] == 0:
+    g = capi.flat_grid(n)
+    keep = []
+    def f(v=1.0):
+        keep.append(np.full(n, v))
+        return keep[-1].ctypes.data
+    def fs(v=0.1):
+        return capi.ptr_array([f(v) for _ in range(S)])
+    st = capi.NrgChemStats()
+    T_t, dC = np.array([300.0, 900.0, 2500.0]), np.zeros((S, 3))
+    lib.nrg_chem_set_table(h, 3, T_t.ctypes.data, dC.ctypes.data)
+    calls = {
+        "table": lambda: lib.nrg_chem_table_step_dev(h, C.byref(g), dt, f(900.0), None, f(), fs(), None, fs(), fs(), f(), None, C.byref(st)),
+        "step": lambda: lib.nrg_chem_step_dev(h, C.byref(g), dt, f(900.0), None, f(), fs(), None, fs(), fs(), f(), None, C.byref(st)),
+        "host_step": lambda: lib.nrg_chem_step(h, C.byref(g), dt, f(900.0), None, f(), fs(), None, fs(), fs(), f(), None, C.byref(st)),
+        "noalloc": lambda: lib.nrg_chem_step_dev_noalloc(h, C.byref(g), dt, f(900.0), None, f(), fs(), None, fs(), fs(), f(), None, C.byref(st)),
+        "closure": lambda: lib.nrg_chem_closure_dev(h, C.byref(g), dt, f(), None, 0, f(), fs(), None, f(), fs(), f(900.0), None),
+        "energy": lambda: lib.nrg_energy_from_temperature_dev(h, C.byref(g), f(900.0), fs(), None, 0, f()),
+    }
+    for name in sys.argv[1].split(","):
+        out[name] = calls[name]()
+    out["host_bytes"] = fake.fake_hip_host_bytes()
+    lib.nrg_chem_destroy(h)
+    out["host_bytes_left"] = fake.fake_hip_host_bytes()
+print(json.dumps(out))
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None or not os.path.exists(os.path.join(ROCM, "hip", "hip_runtime_api.h")):
+        pytest.skip("no C compiler or no HIP headers")
+    so = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    subprocess.run([cc, "-shared", "-fPIC", "-O1", "-I" + ROCM, os.path.join(HERE, "fake_hip.c"), "-o", so], check=True)
+    return so
+
+
+def _run(fake, calls, n=60, **env):
+    import json
+    e = dict(os.environ, PYTHONPATH=ROOT, **env)
+    e["LD_PRELOAD"] = " ".join(x for x in (fake, e.get("LD_PRELOAD", "")) if x)
+    r = subprocess.run([sys.executable, "-c", CHILD, calls, fake, str(n)], env=e, cwd=ROOT, timeout=120,
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.strip().splitlines()[-1])
+
+
+@pytest.mark.parametrize("call,kernel", [("table", "table_kernel"), ("step", "rates_kernel"), ("step", "chem_bdf"),
+                                         ("noalloc", "chem_bdf"), ("closure", "closure_kernel"),
+                                         ("energy", "energy_kernel")])
+def test_refused_launch_is_an_error(fake, call, kernel):
+    from nrg_amd import capi
+    assert _run(fake, call)[call] == capi.NRG_CHEM_OK
+    assert _run(fake, call, FAKE_HIP_REFUSE_LAUNCH=kernel)[call] == capi.NRG_CHEM_E_HIP
