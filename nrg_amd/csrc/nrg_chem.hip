@@ -2074,7 +2074,7 @@ struct StepKey {
 };
 
 // Pinned memory for the host-pointer entry points' fields, at most (137,000 cells of
-// KEROMNES).
+// KEROMNES); a handle holds what its largest call up to that has needed.
 constexpr size_t STAGE_PINNED_MAX = 32u << 20;
 
 struct nrg_chem_handle {
@@ -2092,8 +2092,8 @@ struct nrg_chem_handle {
   int lane_blocks = 0;                     // and of its one-cell-per-lane form
   // staging for the host-pointer entry point: device, and pinned host memory for small fields
   void *stage = nullptr, *pinned = nullptr;
-  size_t stage_bytes = 0;
-  unsigned long long *acc_host = nullptr;  // pinned: counters on their way back
+  size_t stage_bytes = 0, pinned_bytes = 0;
+  unsigned long long *acc_host = nullptr;  // pinned: counters on their way back (or NULL)
   // cell records of one chunk: REC_PAIRS pairs of doubles per position
   double *rates = nullptr;
   long long rates_cells = 0;
@@ -2332,13 +2332,14 @@ static int noalloc_setup(int dev)
 #endif
 }
 
-// The first n counters, once the stream is done (through pinned memory: a copy
-// into a stack variable adds ~10 us to a call).
+// The first n counters, once the stream is done (through pinned memory where there
+// is some: a copy into a stack variable adds ~10 us to a call).
 static hipError_t read_counters(nrg_chem_handle *h, unsigned long long *out, const unsigned long long *dev, int n)
 {
-  hipError_t e = hipMemcpyAsync(h->acc_host, dev, n * sizeof(*out), hipMemcpyDeviceToHost, h->stream);
+  unsigned long long *to = h->acc_host ? h->acc_host : out;
+  hipError_t e = hipMemcpyAsync(to, dev, n * sizeof(*out), hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  if (e == hipSuccess) std::memcpy(out, h->acc_host, n * sizeof(*out));
+  if (e == hipSuccess && to != out) std::memcpy(out, to, n * sizeof(*out));
   return e;
 }
 
@@ -2429,8 +2430,10 @@ int nrg_chem_create(const nrg_chem_mech *mech, const nrg_chem_opts *opts, nrg_ch
     return fail(set_error(NRG_CHEM_E_HIP, "hipMalloc mech"));
   if (hipMalloc(&h->dev_acc, ACC_SLOTS * sizeof(unsigned long long)) != hipSuccess)
     return fail(set_error(NRG_CHEM_E_HIP, "hipMalloc acc"));
-  if (hipHostMalloc(&h->acc_host, 16 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess)
-    return fail(set_error(NRG_CHEM_E_HIP, "hipHostMalloc acc"));
+  if (hipHostMalloc(&h->acc_host, 16 * sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();   // no pinned memory to be had: the counters come without it
+    h->acc_host = nullptr;
+  }
   {
     hipDeviceProp_t prop;
     int per_cu = 0;
@@ -2878,10 +2881,18 @@ static int step_host(nrg_chem_t *h, bool table, const nrg_grid *grid, double dt,
   // flame cells: 60 cells 980 -> 600 us, 9100 1580 -> 1100, 30,000 2080 -> 1640, 80,000
   // 3860 -> 3740, 136,000 the same: from there the copies of single fields overlap.
   bool pin = in_bytes + out_bytes <= STAGE_PINNED_MAX;
-  if (pin && !h->pinned && hipHostMalloc(&h->pinned, STAGE_PINNED_MAX, hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();   // no pinned memory to be had: field by field
+  if (pin && h->pinned_bytes < in_bytes + out_bytes) {
+    void *old = h->pinned;
     h->pinned = nullptr;
-    pin = false;
+    h->pinned_bytes = 0;
+    if (old) HIP_TRY(hipHostFree(old));
+    if (hipHostMalloc(&h->pinned, in_bytes + out_bytes, hipHostMallocDefault) == hipSuccess) {
+      h->pinned_bytes = in_bytes + out_bytes;
+    } else {
+      (void)hipGetLastError();   // no pinned memory to be had: field by field
+      h->pinned = nullptr;
+      pin = false;
+    }
   }
   char *dev = (char *)h->stage, *host = pin ? (char *)h->pinned : nullptr;
   hipStream_t s = h->stream;

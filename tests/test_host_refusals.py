@@ -1,6 +1,7 @@
-"""What the entry points do when the runtime refuses a launch: an error from the
-call whose launch was refused.  On the CPU, in a process of its own, against a
-runtime without a device (fake_hip.c) that can be told to refuse."""
+"""What the entry points do when the runtime refuses a launch or pinned memory: an
+error from the call whose launch was refused, and the way around pinned memory.
+On the CPU, in a process of its own, against a runtime without a device
+(fake_hip.c) that can be told to refuse."""
 import os
 import shutil
 import subprocess
@@ -80,3 +81,18 @@ def test_refused_launch_is_an_error(fake, call, kernel):
     from nrg_amd import capi
     assert _run(fake, call)[call] == capi.NRG_CHEM_OK
     assert _run(fake, call, FAKE_HIP_REFUSE_LAUNCH=kernel)[call] == capi.NRG_CHEM_E_HIP
+
+
+def test_without_pinned_memory(fake):
+    from nrg_amd import capi
+    got = _run(fake, "step,noalloc,table,host_step", FAKE_HIP_REFUSE_PINNED="1")
+    for k in ("create", "step", "noalloc", "table", "host_step"):
+        assert got[k] == capi.NRG_CHEM_OK, k
+
+
+@pytest.mark.parametrize("n,most", [(60, 256 << 10), (30000, 16 << 20)])
+def test_pinned_memory_is_what_the_call_needs(fake, n, most):
+    got = _run(fake, "host_step", n=n)
+    assert got["host_step"] == 0
+    assert 0 < got["host_bytes"] <= most
+    assert got["host_bytes_left"] == 0
