@@ -54,15 +54,13 @@ constexpr int imax(int a, int b) { return a > b ? a : b; }
 // A cell's slice of LDS, in doubles:
 //   [0, 2 REC_PAIRS)   the cell record (chem_device.h)
 //   CZERO, CZERO+1     0.0 (an absent term)
-//   CCELL, CCELL+1     the cell's inner index and its offset in the fields
 //   CONE               1.0 (the factor of an absent operand)
 //   CZ .. CZ+SA        y of the right-hand side being formed, by active slot
 //   CX ..              exchange space: rates of the reactions (fwd, rev, fwd),
 //                      rows of the iteration matrix, norm terms
 // ---------------------------------------------------------------------------
 constexpr int CZERO = 2 * REC_PAIRS;
-constexpr int CCELL = CZERO + 2;
-constexpr int CONE = CCELL + 2;
+constexpr int CONE = CZERO + 2;
 constexpr int CZ = CONE + 1;
 constexpr int CX = (CZ + SA + 1) & ~1;
 constexpr int LDP = (SA + 1) | 1;           // row pitch of a matrix in the exchange space (a spare column at least)

@@ -200,20 +200,20 @@ constexpr bool uses_m(int r)
          topo::rtype[r] == 6 || topo::rtype[r] == 7;
 }
 
-// Cell record: what rates_kernel hands the integrator for one queue position
+// Cell record: what rates_kernel hands the integrator for integrated cell
 // t of a chunk of nrec positions, as pairs of doubles (16 bytes: one lane's
 // share of a direct HBM -> LDS load, global_load_lds_dwordx4).
 //   pairs [0, R)             (k_f(r), k_r(r))
 //   pairs [REC_M, REC_C)     [M] slots 2j, 2j+1
-//   pairs [REC_C, REC_PAIRS) C_s (mol/m^3) at slot s, then the gate flag at
-//                            slot S (1: integrate, 0: gated)
-// In HBM pair p of position t sits at rec[2 (p nrec + t)] (pair-major: the
+//   pairs [REC_C, REC_PAIRS) C_s (mol/m^3) at slot s, then the cell's inner index
+//                            (its bits) at slot S
+// In HBM pair p of record t sits at rec[2 (p nrec + t)] (pair-major: the
 // rate kernel's waves write 1 KiB runs); the integrator keeps a cell's copy in
 // LDS, pair p at doubles 2p, 2p+1 of the cell's slice.
 constexpr int REC_M = R;
 constexpr int REC_C = REC_M + (NM + 1) / 2;
 constexpr int REC_PAIRS = REC_C + (S + 2) / 2;
-constexpr int REC_FLAG = S;
+constexpr int REC_CELL = S;
 // Offset (doubles) of slot j of the pairs starting at pair p0, position 0.
 NRG_DI long long rec_slot(int p0, int j, long long nrec)
 {

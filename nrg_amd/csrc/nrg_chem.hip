@@ -150,7 +150,20 @@ struct StepArgs {
   const int32_t *list;                  // NULL: position t is inner cell t; else inner cell list[t]
   int32_t *hist;                        // optional: each inner cell's work (hist_code), for ordering
   int cpw;                              // cells a wave of the integrator holds at a time
+  // How many of the launch's positions are integrated: in stiffness order, whose
+  // gated cells come last, from the npos positions and the gated ones among them;
+  // else rates_kernel counts them in *live and gives them the records [0, *live).
+  const unsigned long long *gated;
+  unsigned long long *live;
+  long long npos;
 };
+
+NRG_DI long long live_records(const StepArgs &a)
+{
+  if (!a.gated) return (long long)*a.live;
+  const long long n = a.npos - (long long)*a.gated - a.base;
+  return n < 0 ? 0 : n < a.nchunk ? n : a.nchunk;
+}
 
 // Inner cell (inner-loop order) at position base + t of the launch's queue.
 // The 64-bit form alone: the integrator kernel's one call (at a refill) keeps
@@ -231,7 +244,8 @@ enum { ACC_INTEG = 0, ACC_NSTEP, ACC_NFE, ACC_NJE, ACC_NCORR, ACC_NATT, ACC_NSTE
        ACC_STATUS0,     // ACC_STATUS0 + NRG_CELL_* (8 slots)
        ACC_QUEUE0 = 16, // one queue head per chunk
        MAX_CHUNKS = 48,
-       ACC_SLOTS = ACC_QUEUE0 + MAX_CHUNKS };
+       ACC_LIVE0 = ACC_QUEUE0 + MAX_CHUNKS,   // and one count of integrated cells
+       ACC_SLOTS = ACC_LIVE0 + MAX_CHUNKS };
 
 // Zero the work accumulators and the queue head (a kernel, so the launch
 // sequence can be captured in a graph without memset nodes).
@@ -244,10 +258,9 @@ __global__ void reset_kernel(unsigned long long *acc, int n)
 #endif
 
 // Load one cell and set it up (chemical_kinetics_solver.f90:228-265): the
-// group's lanes copy the cell record of position t (rates_kernel) from HBM to
-// the cell's slice of LDS, all loads in one round trip.  Returns false for a
-// gated cell, whose outputs are written here (:341-346).
-NRG_DI bool start_cell(const StepArgs &a, long long t, Cell &c, const Lane &ln)
+// group's lanes copy cell record t (rates_kernel) from HBM to the cell's slice of
+// LDS, all loads in one round trip.
+NRG_DI void start_cell(const StepArgs &a, long long t, Cell &c, const Lane &ln)
 {
   const double *src = a.rates + 2 * t;
   constexpr int K = (REC_PAIRS + G - 1) / G;
@@ -258,8 +271,6 @@ NRG_DI bool start_cell(const StepArgs &a, long long t, Cell &c, const Lane &ln)
     if ((k + 1) * G <= REC_PAIRS || p < REC_PAIRS)
       v[k] = *reinterpret_cast<const double2 *>(src + 2 * (long long)p * a.nchunk);
   }
-  const long long q = cell_of(a, t);
-  const long long off = cell_offset(a.g, q);
   wave_sync();
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -269,35 +280,14 @@ NRG_DI bool start_cell(const StepArgs &a, long long t, Cell &c, const Lane &ln)
       *slot(ln, 2 * p + 1) = v[k].y;
     }
   }
-  if (ln.sub == 0) {
-    *slot(ln, CCELL) = __longlong_as_double(q);
-    *slot(ln, CCELL + 1) = __longlong_as_double(off);
-  }
   wave_sync();
-  if (*slot(ln, 2 * REC_C + REC_FLAG) == 0.0) {
-#pragma unroll
-    for (int s0 = 0; s0 < S; s0 += G)
-      if (s0 + ln.sub < S) a.Yp[s0 + ln.sub][off] = 0.0;
-    if (ln.sub == 0) {
-      a.Efp[off] = 0.0;
-      if (a.status) a.status[off] = NRG_CELL_GATED;
-      if (a.nstep) {
-        a.nstep[q] = 0;
-        a.nfe[q] = 0;
-        a.nje[q] = 0;
-      }
-      if (a.hist) a.hist[q] = 0;
-    }
-    return false;
-  }
   c.y = holds(ln) ? *slot(ln, 2 * REC_C + slot_species(ln.sub)) : 0.0;
   bdf_init(c, a.dt, a.k);
-  return true;
 }
 
 #if NRG_PART < 2
-// Cell records of the chunk's positions: the gate (:224-227), and for every
-// integrated cell its concentrations (:228-233), rate constants and [M]
+// Cell records of the chunk's positions: the gate (:224-227) and the outputs of the
+// cells it closes (:341-346), and for every integrated cell its concentrations (:228-233), rate constants and [M]
 // (:235-252, 360-493), kept apart from the integrator so its ~80
 // transcendentals run coherently.  A block covers
 // RATES_CELLS cells RATES_GROUPS times: the waves of group g compute
@@ -314,17 +304,50 @@ __global__ void __launch_bounds__(256) rates_kernel(StepArgs a)
   stage_mech(mc, a.mech);
   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / RATES_CELLS);   // wave-uniform
   const long long t = (long long)blockIdx.x * RATES_CELLS + (threadIdx.x % RATES_CELLS);
-  if (t >= a.nchunk) return;
-  const long long q = cell_of(a, t);
-  const long long off = cell_offset(a.g, q);
-  const double T = a.T[off];
-  const int8_t bcv = a.bc ? a.bc[off] : (int8_t)0;
-  double *out = a.rates_out + 2 * t;
-  if (!(T >= a.k.t_gate && bcv == 0)) {
-    if (grp == 0)   // the gate flag's pair
-      *reinterpret_cast<double2 *>(out + rec_slot(REC_C, REC_FLAG & ~1, a.nchunk)) = make_double2(0.0, 0.0);
+  const bool in = t < a.nchunk;
+  long long q = 0, off = 0, record = t;
+  double T = 0.0;
+  bool live = false;
+  if (in) {
+    q = cell_of(a, t);
+    off = cell_offset(a.g, q);
+    T = a.T[off];
+    live = T >= a.k.t_gate && (!a.bc || a.bc[off] == 0);
+  }
+  if (!a.gated) {
+    // the block's integrated cells take the next records (one atomic a block)
+    constexpr int WAVES = RATES_CELLS / WAVE;
+    __shared__ unsigned long long first;
+    __shared__ int count[WAVES];
+    const unsigned long long mask = __ballot(live ? 1 : 0);
+    const int w = threadIdx.x % RATES_CELLS / WAVE;
+    if (grp == 0 && threadIdx.x % WAVE == 0) count[w] = __popcll(mask);
+    __syncthreads();
+    int before = __popcll(mask & ((1ull << (threadIdx.x % WAVE)) - 1ull)), all = 0;
+    for (int i = 0; i < WAVES; ++i) {
+      before += i < w ? count[i] : 0;
+      all += count[i];
+    }
+    if (threadIdx.x == 0 && all) first = atomicAdd(a.live, (unsigned long long)all);
+    __syncthreads();
+    record = (long long)first + before;
+  }
+  if (!live) {
+    if (in && grp == 0) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) a.Yp[s][off] = 0.0;
+      a.Efp[off] = 0.0;
+      if (a.status) a.status[off] = NRG_CELL_GATED;
+      if (a.nstep) {
+        a.nstep[q] = 0;
+        a.nfe[q] = 0;
+        a.nje[q] = 0;
+      }
+      if (a.hist) a.hist[q] = 0;
+    }
     return;
   }
+  double *out = a.rates_out + 2 * record;
   const double rho = a.rho[off];
   double C[S];
 #pragma unroll
@@ -339,13 +362,13 @@ __global__ void __launch_bounds__(256) rates_kernel(StepArgs a)
     rate_constants<InlineMath, 2 * R / G, 3 * R / G>(mc, T, C, out, a.nchunk);
   else
     rate_constants<InlineMath, 3 * R / G, R>(mc, T, C, out, a.nchunk);
-  // the concentrations and the gate flag, written last (stored ahead of the
+  // the concentrations and the cell's index, written last (stored ahead of the
   // rate constants, they doubled the kernel's registers: occupancy 4 -> 2)
   if (grp == 0) {
 #pragma unroll
-    for (int j = 0; j <= REC_FLAG; j += 2) {
-      const double lo = j < S ? C[j] : 1.0;
-      const double hi = j + 1 < S ? C[j + 1] : (j + 1 == REC_FLAG ? 1.0 : 0.0);
+    for (int j = 0; j <= REC_CELL; j += 2) {
+      const double lo = j < S ? C[j] : __longlong_as_double(q);
+      const double hi = j + 1 < S ? C[j + 1] : (j + 1 == REC_CELL ? __longlong_as_double(q) : 0.0);
       *reinterpret_cast<double2 *>(out + rec_slot(REC_C, j, a.nchunk)) = make_double2(lo, hi);
     }
   }
@@ -361,8 +384,8 @@ NRG_DI void finish_cell(const StepArgs &a, const BdfCoef &mc, const Cell &c, con
   wave_sync();
   if (holds(ln)) *own(ln, CZ) = c.y;
   wave_sync();
-  const long long q = __double_as_longlong(*slot(ln, CCELL));
-  const long long off = __double_as_longlong(*slot(ln, CCELL + 1));
+  const long long q = __double_as_longlong(*slot(ln, 2 * REC_C + REC_CELL));
+  const long long off = cell_offset(a.g, q);
 #pragma unroll
   for (int s0 = 0; s0 < S; s0 += G) {
     const int s = s0 + ln.sub;
@@ -464,6 +487,8 @@ extern template __global__ void chem_bdf_kernel<true>(StepArgs);
   Cell c;
   c.pc = PC_IDLE;
   const int grp = lane / G;
+  const long long limit = live_records(a);
+  if (blockIdx.x == 0 && lane == 0) tally[ACC_STATUS0 + NRG_CELL_GATED] = (unsigned long long)(a.nchunk - limit);
   bool exhausted = grp >= a.cpw;
   for (;;) {
     bool need = c.pc >= PC_DONE && !exhausted;
@@ -478,10 +503,10 @@ extern template __global__ void chem_bdf_kernel<true>(StepArgs);
       if (need) {
         const long long t =
             (long long)(base + (unsigned long long)(__popcll(mask & ((1ull << ln.gshift) - 1ull)) / G));
-        if (t >= a.nchunk)
+        if (t >= limit)
           exhausted = true;
-        else if (!start_cell(a, t, c, ln) && ln.sub == 0)
-          atomicAdd(&tally[ACC_STATUS0 + NRG_CELL_GATED], 1ull);
+        else
+          start_cell(a, t, c, ln);
       }
       need = need && c.pc >= PC_DONE && !exhausted;
     }
@@ -521,11 +546,10 @@ constexpr int LANE_WAVES_PER_CU = 4;   // one to a SIMD: it takes the whole regi
 typedef __attribute__((address_space(3))) void lds_void;
 
 // Load one cell and set it up (chemical_kinetics_solver.f90:228-265).  The
-// cell record of position t (rates_kernel) goes from HBM straight into the
-// lane's LDS slots (recl: the block's record array, kl: this lane's view of
-// it): one round trip, no registers in between.  Returns false for a gated
-// cell, whose outputs are written here (:341-346).
-NRG_DI bool start_cell(const StepArgs &a, long long t, long long q, long long &off, lane::Cell &c,
+// cell record t (rates_kernel) goes from HBM straight into the lane's LDS slots
+// (recl: the block's record array, kl: this lane's view of it): one round trip, no
+// registers in between.
+NRG_DI void start_cell(const StepArgs &a, long long t, long long &q, long long &off, lane::Cell &c,
                        lds_double *recl, const double *kl)
 {
   const double *src = a.rates + 2 * t;
@@ -533,22 +557,10 @@ NRG_DI bool start_cell(const StepArgs &a, long long t, long long q, long long &o
   for (int p = 0; p < REC_PAIRS; ++p)
     __builtin_amdgcn_global_load_lds((const void *)(src + 2 * (long long)p * a.nchunk),
                                      (lds_void *)(recl + 2 * p * WAVE), 16, 0, 0);   // M0: LDS address
-  off = cell_offset_wide(a.g, q);
   // a direct load's data is in LDS once vmcnt has counted it
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if (lane::rec_c(kl, REC_FLAG) == 0.0) {
-#pragma unroll
-    for (int s = 0; s < S; ++s) a.Yp[s][off] = 0.0;
-    a.Efp[off] = 0.0;
-    if (a.status) a.status[off] = NRG_CELL_GATED;
-    if (a.nstep) {
-      a.nstep[q] = 0;
-      a.nfe[q] = 0;
-      a.nje[q] = 0;
-    }
-    if (a.hist) a.hist[q] = 0;
-    return false;
-  }
+  q = __double_as_longlong(lane::rec_c(kl, REC_CELL));
+  off = cell_offset_wide(a.g, q);
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     if (kSp.act[s] >= 0)
@@ -557,14 +569,13 @@ NRG_DI bool start_cell(const StepArgs &a, long long t, long long q, long long &o
       c.yi[kSp.islot[s]] = lane::rec_c(kl, s);
   }
   lane::bdf_init(c, a.dt, a.k);
-  return true;
 }
 
 // A lane's counts of its finished cells.  (In registers: cells of equal cost
 // finish together, and 64 atomics to one LDS word take as many turns; 2.1M
 // cells with hot kernels 5.44 ms so, 4.85 here.)
 struct LaneTally {
-  unsigned integrated = 0, gated = 0;
+  unsigned integrated = 0;
   unsigned long long nstep = 0, nfe = 0, nje = 0, ncorr = 0, natt = 0;
   int nstep_max = 0, nfe_max = 0;
 };
@@ -633,6 +644,8 @@ extern template __global__ void chem_bdf_lane_kernel<true>(StepArgs);
   stage_bdf(mc, a.mech, a.k.sqrtn);
   const double *kl = recl + 2 * lane;
   lds_double *recl_lds = (lds_double *)recl;   // the array's LDS address (direct loads' M0)
+  const long long limit = live_records(a);
+  if (blockIdx.x == 0 && lane == 0) tally[ACC_STATUS0 + NRG_CELL_GATED] = (unsigned long long)(a.nchunk - limit);
   lane::Cell c;
   c.req = lane::REQ_DONE;
   long long q = -1, off = 0;
@@ -651,12 +664,11 @@ extern template __global__ void chem_bdf_lane_kernel<true>(StepArgs);
       base = __shfl(base, leader, WAVE);
       if (need) {
         const long long t = (long long)(base + (unsigned long long)__popcll(mask & ((1ull << lane) - 1ull)));
-        if (t >= a.nchunk) {
+        if (t >= limit) {
           exhausted = true;
         } else {
-          q = cell_of(a, t);
-          have = start_cell(a, t, q, off, c, recl_lds, kl);
-          tl.gated += have ? 0 : 1;
+          start_cell(a, t, q, off, c, recl_lds, kl);
+          have = true;
         }
       }
       need = !have && !exhausted;
@@ -684,7 +696,6 @@ extern template __global__ void chem_bdf_lane_kernel<true>(StepArgs);
       have = false;
     }
   }
-  atomicAdd(&tally[ACC_STATUS0 + NRG_CELL_GATED], (unsigned long long)tl.gated);
   atomicAdd(&tally[ACC_INTEG], (unsigned long long)tl.integrated);
   atomicAdd(&tally[ACC_NSTEP], tl.nstep);
   atomicAdd(&tally[ACC_NFE], tl.nfe);
@@ -2044,12 +2055,12 @@ using namespace kern;
 
 // ===========================================================================
 // Scratch of nrg_chem_step_dev_noalloc: the work accumulators and queue heads
-// (ACC_SLOTS words, padded to 512 bytes), then the cell records of one chunk
+// (ACC_SLOTS words, padded to 1024 bytes), then the cell records of one chunk
 // of NRG_NOALLOC_CHUNK_CELLS cells.  One copy per device, held until the
 // process ends.  Host code reaches it only through the per-device address
 // hipGetSymbolAddress returned (g_noalloc_scratch), never through its name.
 // ===========================================================================
-constexpr size_t NOALLOC_ACC_BYTES = 512;
+constexpr size_t NOALLOC_ACC_BYTES = 1024;
 #if NRG_TOPO_PRIMARY
 static_assert(ACC_SLOTS * sizeof(unsigned long long) <= NOALLOC_ACC_BYTES, "accumulators");
 static_assert(NOALLOC_ACC_BYTES + (size_t)NRG_NOALLOC_CHUNK_CELLS * REC_PAIRS * 2 * sizeof(double) <=
@@ -2585,12 +2596,16 @@ static void enqueue_chunks(nrg_chem_t *h, StepArgs &a, long long npos, long long
                            double *rates, unsigned long long *acc, bool fallback)
 {
   const long long nchunks = npos > 0 ? (npos + chunk - 1) / chunk : 0;
+  const bool ordered = a.list && a.list == h->order_list;
+  a.npos = npos;
+  a.gated = ordered ? h->bins : nullptr;   // bin 0 (cost_bin)
   a.rates = rates;
   a.rates_out = rates;
   for (long long ci = 0; ci < nchunks; ++ci) {
     a.base = ci * chunk;
     a.nchunk = std::min<long long>(chunk, npos - a.base);
     a.queue = acc + ACC_QUEUE0 + ci;
+    a.live = acc + ACC_LIVE0 + ci;
     hipLaunchKernelGGL(rates_kernel, dim3((unsigned)((a.nchunk + RATES_CELLS - 1) / RATES_CELLS)),
                        dim3(256), 0, h->stream, a);
     // A wave holds fewer cells than it could where the grid gives the SIMDs less
@@ -2598,7 +2613,6 @@ static void enqueue_chunks(nrg_chem_t *h, StepArgs &a, long long npos, long long
     // stages (420 flame cells: one to a wave 0.60 ms, eight 0.75; 16,384: the same).
     a.cpw = (int)std::min<long long>(CPW, std::max<long long>(1, (a.nchunk + 4 * h->num_cu - 1) / (4 * h->num_cu)));
     const bool analytic = h->opts.jacobian == NRG_JAC_ANALYTIC;
-    const bool ordered = a.list && a.list == h->order_list;
     const long long need = (a.nchunk + a.cpw - 1) / a.cpw;
     const dim3 grid((unsigned)std::min<long long>(need, h->persistent_blocks));
     if constexpr (LANE_KERNEL)
