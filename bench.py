@@ -242,9 +242,12 @@ def main():
                    (1 << (args.chunk_log2 or 23)))
     nchunks = -(-ncells // chunk_cells)
     tr = profiled_traffic(ncells)
-    # large launches in stiffness order give a cell a lane, the others a group of lanes
+    # in stiffness order a cell goes to a lane where a launch's right-hand sides are those
+    # of a chip full of its longest cell (and many to a step), else to a group of lanes
+    full = stats.nfe_sum / max(1, stats.nfe_max) * min(1.0, chunk_cells / ncells)
     integrator = ("chem_bdf_lane_kernel" if effective_setup(args, tuning)["order"] == "stiffness"
-                  and min(ncells, chunk_cells) >= LANE_CELLS else "chem_bdf_kernel")
+                  and full >= 256 * torch.cuda.get_device_properties(dev).multi_processor_count
+                  and stats.nfe_sum >= 2.5 * stats.nstep_sum else "chem_bdf_kernel")
     roofline = {
         "kernel": "rates_kernel + %s (one chemistry step)" % integrator,
         "bound": "fp64_valu",
@@ -430,7 +433,6 @@ SQ_PROFILE = os.path.join(ROOT, "profiles", "chem_step_256cube_sq_counters.txt")
 RESOURCE_USAGE = {"chem_bdf_kernel": os.path.join(ROOT, "nrg_amd", "csrc", "resource_usage.txt"),
                   "chem_bdf_lane_kernel": os.path.join(ROOT, "nrg_amd", "csrc",
                                                        "resource_usage_lane_keromnes.txt")}
-LANE_CELLS = 5 << 17             # cells of a launch from which the one-cell-per-lane integrator runs
 
 
 def profiled_lanes(kernel="chem_bdf_kernel"):

@@ -82,7 +82,7 @@ enum {
 /*
  * Launch form of the per-cell integrator.  Both forms run the same resident
  * grid over the work queue (same arithmetic, same results, same time): a cell to
- * a group of lanes, or, in large grids in stiffness order, a cell to a lane.
+ * a group of lanes or, where the previous call's counts say that it pays, to a lane.
  */
 enum {
   NRG_FORM_PLAIN = 0,
@@ -146,9 +146,10 @@ typedef struct nrg_chem_opts {
                                   are stepping is there (100: the wave's cells take their
                                   steps' error tests together; 0: no waiting).  Same results. */
   int32_t refill_min_idle;     /* a wave hands new cells to its idle lanes once this many of its
-                                  64 lanes are idle, or all are (1..64; 0 = default: 63 in
-                                  stiffness order, where a wave's cells cost alike and start
-                                  together, 32 in natural order).  Same results.              */
+                                  64 lanes are idle, or all are (1..64; 0 = default: 63 where
+                                  a wave's cells cost alike and start together, in stiffness
+                                  order and where the previous call's did, else 32).  Same
+                                  results.                                                    */
 } nrg_chem_opts;
 
 /*
@@ -293,8 +294,8 @@ int nrg_energy_from_temperature_dev(nrg_chem_t *h, const nrg_grid *grid,
                                     const double *const *v, int32_t ndim, double *E_f);
 
 /*
- * Autotuner of the batched form.  A cell is one lane and a workgroup one
- * wave (64 cells), so what is tuned is how the queue feeds the waves: cell
+ * Autotuner of the batched form.  A workgroup is one wave, whose lanes or lane
+ * groups hold the cells, so what is tuned is how the queue feeds the waves: cell
  * order, the error-test gathering, the batched-Jacobian threshold,
  * the refill threshold, resident waves per CU and the queue chunk size.  Starting from the handle's current set-up it tries
  * one change at a time (greedy), each as a full chemistry step on the given

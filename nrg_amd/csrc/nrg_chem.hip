@@ -2081,7 +2081,17 @@ struct StepKey {
   int use_hist, form;
   long long chunk_max;
   long long persistent_blocks; // the integrator's grid (the autotuner may change it alone)
-  int jacobian;                // NRG_JAC_*: which integrator kernel the graph launches
+  int jacobian;                // NRG_JAC_* and which chunks go one cell to a lane: the
+  unsigned long long lanes;    // integrator kernels the graph launches
+};
+
+// What a handle's previous call on a grid counted, and what it led to (plan).
+struct Seen {
+  bool valid = false, alike = false;
+  GridIdx g{};
+  long long cells = 0, nfe_max = 0;
+  double nfe = 0.0, nstep = 0.0;
+  unsigned long long lanes = 0;
 };
 
 // Pinned memory for the host-pointer entry points' fields, at most (137,000 cells of
@@ -2099,6 +2109,7 @@ struct nrg_chem_handle {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   int form = NRG_FORM_PLAIN;
   int jac_pct = 50;
+  bool refill_auto = true;                 // the caller has set no refill threshold
   int persistent_blocks = 0;               // resident one-wave blocks of the integrator
   int lane_blocks = 0;                     // and of its one-cell-per-lane form
   // staging for the host-pointer entry point: device, and pinned host memory for small fields
@@ -2126,6 +2137,7 @@ struct nrg_chem_handle {
   int32_t *hist = nullptr;
   unsigned long long *bins = nullptr;      // count[NBIN], cursor[NBIN]
   long long order_cells = 0;
+  Seen seen_step, seen_fallback;           // steps, and fallbacks of the learned step
   bool hist_valid = false;
   GridIdx hist_grid{};
   // table-approximated mode: T_t[rows], then dC_t[S][rows]
@@ -2425,6 +2437,7 @@ int nrg_chem_create(const nrg_chem_mech *mech, const nrg_chem_opts *opts, nrg_ch
   h->opts = o;
   h->device = o.device;
   h->k = make_const(o);
+  h->refill_auto = o.refill_min_idle == 0;
   h->form = o.form;
   h->order = o.cell_order;
   h->use_graph = o.use_graph != 0;
@@ -2491,11 +2504,6 @@ void nrg_chem_destroy(nrg_chem_t *h)
 }
 
 void *nrg_chem_stream(nrg_chem_t *h) { return h ? (void *)h->stream : nullptr; }
-
-static bool same_grid(const GridIdx &x, const GridIdx &y)
-{
-  return std::memcmp(&x, &y, sizeof(GridIdx)) == 0;
-}
 
 // Build the stiffness-ordered cell list of this call into h->order_list and
 // point a.list / a.hist at it (device work only, so it can be captured).
@@ -2568,32 +2576,97 @@ static int prepare_rates(nrg_chem_t *h, long long npos)
   return NRG_CHEM_OK;
 }
 
-// Cells of a launch in stiffness order from which they go one to a lane
-// instead of one to a lane group: from there they fill the chip often enough
-// (65,536 once) that a lane's shorter way through a step counts more than the
-// group's shorter way through a cell.  Kernel ms, group against lane, KEROMNES:
-//   finite differences: 262,144 flame cells 4.1 / 3.7, 589,824 8.8 / 7.2, 1M 15.3 /
-//   11.9; igniting 262,144 4.7 / 4.1 in 100 ns and 11.8 / 12.9 in 1 us, 545,400 in 1 us
-//   23.0 / 24.1; with most cells cold (hot kernels) 884,736 2.5 / 3.5, 1.4M 3.4 / 3.5,
-//   2.1M 5.5 / 3.7.
-//   analytic Jacobian (few right-hand sides, so the vector work that a group
-//   shares counts less): 131,044 flame cells 1.33 / 1.09, 262,144 2.4 / 1.7; igniting
-//   131,072 1.41 / 1.52, 196,608 2.03 / 1.61.  The learned step's fallback list holds
-//   no idle cells, which moves the line: 83,905 of 2.4M cells 1.67 / 1.51.
-// With nine or ten species a group has 16 lanes, and a lane's state spills:
-//   TEREZA flame cells 1M 33.0 / 31.1, 2.4M 72 / 64; hot kernels 2.1M 10.6 /
-//   15.1, 7.1M 42 / 30; analytic igniting 131,072 3.1 / 2.0.
-// In natural order a group is ahead at every size (1M flame cells: 23.5 ms, a
-// lane 39).
-static long long lane_cells(bool analytic, bool fallback)
+static bool same_grid(const GridIdx &x, const GridIdx &y)
 {
-  return analytic ? (fallback ? 1 : 3) << 16 : SA <= 8 ? 5 << 17 : 1 << 22;
+  return std::memcmp(&x, &y, sizeof(GridIdx)) == 0;
+}
+
+// A lane or a lane group to a cell?  A lane's way through a right-hand side and an
+// iteration matrix costs the chip less (0.6 to 0.8 of a group's time where the chip is
+// full of cells that cost alike), but it is three times as long, and a wave waits
+// for the longest of its 64 cells.  So it depends on what a launch holds, which the
+// counters of the handle's previous call on the grid tell: right-hand sides in
+// all over those of the longest cell are the cells' worth of work (`full`), and that
+// over the cells is how alike they are (`alike`: 0.7 a flame, 0.04 a grid of cold gas
+// with hot kernels).  Below, time of a lane over that of a group, KEROMNES unless
+// said otherwise; 65,536 lanes fill the chip.
+//  Stiffness order with a history (a wave's cells cost alike):
+//   finite differences, `full` in thousands: hot kernels 13: 2.35, 36: 1.31, 82: 0.67;
+//    flame 64: 1.09, 112: 0.92, 434: 0.80; igniting 18: 2.1, 35: 1.5, 70: 0.88, 279: 0.82;
+//    one composition at 900 K 23: 1.5, 46: 0.97, 91: 0.85.  In 1 us, where a cell takes
+//    many steps to a Jacobian (2.2 right-hand sides a step; 2.6 and up elsewhere), 92:
+//    1.09, 192: 1.04: what a lane does better is right-hand sides.  With 16 lanes to a
+//    group a lane's state spills (TEREZA flame 90: 1.01, 155: 0.96, igniting 139: 1.03).
+//   analytic Jacobian: hot kernels 13: 1.7, 36: 0.79; flame 26: 1.23, 57: 0.82, 392: 0.67;
+//    igniting 18: 1.7, 38: 1.06, 75: 0.74; 1100 K 35: 1.24, 71: 0.69; a learned step's
+//    fallback list 24: 1.3, 44: 0.9, 89: 0.79.
+//   (Under 0.5 of the lanes the longest cell decides; where there are three times as
+//   many cells as lanes, the others run beside it.)
+//  Without a history there is nothing to tell, and stiffness order has only 50 K
+//   temperature bins: finite differences, hot kernels 1.4 to 1.8 (TEREZA 2.6 to 3.1),
+//   flame 0.9, one composition 0.8: a group loses less.  Analytic, hot kernels 1.0 to
+//   1.4, flame and igniting 0.77, one composition 0.63 (TEREZA 0.4): a lane does, from
+//   where it fills the chip a few times (natural order 1.0 to 1.26 and 0.62 to 0.95).
+//  Natural order, both with the refill that fits: `alike` 0.82: 0.8 to 0.9, 0.69: 0.85 to
+//   1.0, flame (0.67) 112: 1.2, 434: 1.06, 0.58: 1.1 to 0.9, igniting (0.27) 1.2, hot kernels
+//   1.4; analytic 0.61: 0.8 to 1.07, 0.54: 0.7 to 0.9, 0.29: 1.05 to 1.2 (TEREZA 0.9), hot kernels
+//   1.1 (TEREZA 1.03 at 39, 0.8 above).
+// The choice keeps to what it was until the numbers are a fifth past the line, so that
+// a captured graph does not change with every call.
+static bool alike(const Seen &s)
+{
+  return s.valid && s.nfe * (s.alike ? 2.5 : 2.0) >= (double)s.cells * s.nfe_max;
+}
+static bool lane_launch(const nrg_chem_t *h, const Seen &s, bool ordered, bool use_hist, bool fallback,
+                        long long npos, long long nchunk, bool before)
+{
+  if (!LANE_KERNEL) return false;
+  const bool analytic = h->opts.jacobian == NRG_JAC_ANALYTIC;
+  const double lanes = (double)WAVE * LANE_WAVES_PER_CU * h->num_cu, slack = before ? 0.8 : 1.0;
+  if (!s.valid || s.nfe_max <= 0 || (ordered && !use_hist))
+    return analytic && nchunk >= (fallback ? 1 : ordered ? 3 : 8) * lanes;
+  const double part = (double)nchunk / (fallback ? s.cells : npos);
+  const double full = part * s.nfe / s.nfe_max;
+  const double fills = analytic ? (!ordered ? 1.0 : part * s.cells >= 3 * lanes ? 0.4 : 0.5625)
+                                : (ordered && G == 8 ? 1.0 : 2.0);
+  if (full < slack * fills * lanes) return false;
+  if (ordered) return analytic || s.nfe >= slack * 2.5 * s.nstep || alike(s);
+  return alike(s) || (analytic && G == 16);
+}
+
+// The chunks of a call that go one cell to a lane (a bit each), and the refill threshold
+// of natural order where the caller has set none.
+static unsigned long long plan(nrg_chem_t *h, Seen &s, StepArgs &a, long long npos, long long chunk, bool ordered,
+                               bool use_hist, bool fallback)
+{
+  if (s.valid && !same_grid(s.g, a.g)) s = Seen();
+  unsigned long long lanes = 0;
+  for (long long ci = 0; ci * chunk < npos; ++ci)
+    if (lane_launch(h, s, ordered, use_hist, fallback, npos, std::min(chunk, npos - ci * chunk), s.lanes >> ci & 1))
+      lanes |= 1ull << ci;
+  s.lanes = lanes;
+  s.alike = alike(s);
+  if (h->refill_auto)
+    a.k.refill_idle = ordered || s.alike ? REFILL_IDLE_ORDERED : REFILL_IDLE_NATURAL;
+  return lanes;
+}
+
+// Keep what a call has counted for the next one's plan.
+static void note(Seen &s, const GridIdx &g, const unsigned long long (&acc)[16])
+{
+  s.valid = acc[ACC_INTEG] > 0;
+  s.g = g;
+  s.cells = (long long)acc[ACC_INTEG];
+  s.nfe = (double)acc[ACC_NFE];
+  s.nstep = (double)acc[ACC_NSTEP];
+  s.nfe_max = (long long)acc[ACC_NFE_MAX];
 }
 
 // Launch rates_kernel + the integrator kernel per chunk of `chunk` positions, with
-// the chunk's rate constants in `rates` and its queue head in acc[ACC_QUEUE0 + ci].
+// the chunk's rate constants in `rates` and its queue head in acc[ACC_QUEUE0 + ci];
+// chunk ci goes to the one-cell-per-lane integrator where bit ci of `lanes` is set.
 static void enqueue_chunks(nrg_chem_t *h, StepArgs &a, long long npos, long long chunk,
-                           double *rates, unsigned long long *acc, bool fallback)
+                           double *rates, unsigned long long *acc, unsigned long long lanes)
 {
   const long long nchunks = npos > 0 ? (npos + chunk - 1) / chunk : 0;
   const bool ordered = a.list && a.list == h->order_list;
@@ -2616,12 +2689,12 @@ static void enqueue_chunks(nrg_chem_t *h, StepArgs &a, long long npos, long long
     const long long need = (a.nchunk + a.cpw - 1) / a.cpw;
     const dim3 grid((unsigned)std::min<long long>(need, h->persistent_blocks));
     if constexpr (LANE_KERNEL)
-      if (ordered && a.nchunk >= lane_cells(analytic, fallback)) {
-        const dim3 lanes((unsigned)std::min<long long>((a.nchunk + WAVE - 1) / WAVE, h->lane_blocks));
+      if (lanes >> ci & 1) {
+        const dim3 blocks((unsigned)std::min<long long>((a.nchunk + WAVE - 1) / WAVE, h->lane_blocks));
         if (analytic)
-          hipLaunchKernelGGL(chem_bdf_lane_kernel<true>, lanes, dim3(WAVE), 0, h->stream, a);
+          hipLaunchKernelGGL(chem_bdf_lane_kernel<true>, blocks, dim3(WAVE), 0, h->stream, a);
         else
-          hipLaunchKernelGGL(chem_bdf_lane_kernel<false>, lanes, dim3(WAVE), 0, h->stream, a);
+          hipLaunchKernelGGL(chem_bdf_lane_kernel<false>, blocks, dim3(WAVE), 0, h->stream, a);
         continue;
       }
     if (analytic)
@@ -2631,11 +2704,11 @@ static void enqueue_chunks(nrg_chem_t *h, StepArgs &a, long long npos, long long
   }
 }
 
-static int enqueue_integrator(nrg_chem_t *h, StepArgs &a, long long npos, bool fallback = false)
+static int enqueue_integrator(nrg_chem_t *h, StepArgs &a, long long npos, unsigned long long lanes)
 {
   int st = prepare_rates(h, npos);
   if (st) return st;
-  enqueue_chunks(h, a, npos, chunk_for(h, npos), h->rates, h->dev_acc, fallback);
+  enqueue_chunks(h, a, npos, chunk_for(h, npos), h->rates, h->dev_acc, lanes);
   HIP_TRY(hipGetLastError());
   return NRG_CHEM_OK;
 }
@@ -2671,16 +2744,16 @@ static int integrator_status(const unsigned long long (&acc)[16])
 
 // The device work of one chemistry step: counters reset, optional ordering,
 // rate constants and integrator per chunk.  Launches only.
-static int enqueue_step(nrg_chem_t *h, StepArgs &a, bool use_hist)
+static int enqueue_step(nrg_chem_t *h, StepArgs &a, bool use_hist, unsigned long long lanes)
 {
   hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(ACC_SLOTS), 0, h->stream, h->dev_acc, ACC_SLOTS);
   if (a.list) enqueue_order(h, a, use_hist);
-  return enqueue_integrator(h, a, a.g.ninner);
+  return enqueue_integrator(h, a, a.g.ninner, lanes);
 }
 
 // Replay the captured step when the arguments equal the captured ones;
 // otherwise capture the step into a new graph first.
-static int launch_step_graph(nrg_chem_t *h, StepArgs &a, bool use_hist)
+static int launch_step_graph(nrg_chem_t *h, StepArgs &a, bool use_hist, unsigned long long lanes)
 {
   StepKey key;
   std::memset(&key, 0, sizeof(key));
@@ -2691,13 +2764,14 @@ static int launch_step_graph(nrg_chem_t *h, StepArgs &a, bool use_hist)
   key.chunk_max = h->chunk_max;
   key.persistent_blocks = h->persistent_blocks;
   key.jacobian = h->opts.jacobian;
+  key.lanes = lanes;
   if (!h->graph_exec || std::memcmp(&key, &h->graph_key, sizeof(key)) != 0) {
     if (h->graph_exec) HIP_TRY(hipGraphExecDestroy(h->graph_exec));
     h->graph_exec = nullptr;
     hipGraph_t graph = nullptr;
     HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     StepArgs c = a;
-    const int st = enqueue_step(h, c, use_hist);
+    const int st = enqueue_step(h, c, use_hist, lanes);
     const hipError_t e = hipStreamEndCapture(h->stream, &graph);
     if (st) {
       if (graph) (void)hipGraphDestroy(graph);
@@ -2778,11 +2852,13 @@ static int step_dev_impl(nrg_chem_t *h, const nrg_grid *grid, double dt, const d
       a.hist = h->hist;
     }
     if ((st = prepare_rates(h, a.g.ninner))) return st;
+    const unsigned long long lanes =
+        plan(h, h->seen_step, a, a.g.ninner, chunk_for(h, a.g.ninner), ordered, use_hist, false);
     HIP_TRY(hipEventRecord(h->ev0, h->stream));
     if (h->use_graph) {
-      if ((st = launch_step_graph(h, a, use_hist))) return st;
+      if ((st = launch_step_graph(h, a, use_hist, lanes))) return st;
     } else {
-      if ((st = enqueue_step(h, a, use_hist))) return st;
+      if ((st = enqueue_step(h, a, use_hist, lanes))) return st;
     }
     if (ordered) {
       h->hist_valid = true;
@@ -2791,6 +2867,7 @@ static int step_dev_impl(nrg_chem_t *h, const nrg_grid *grid, double dt, const d
     HIP_TRY(hipEventRecord(h->ev1, h->stream));
     HIP_TRY(read_counters(h, acc, h->dev_acc, 16));
     HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
+    note(h->seen_step, a.g, acc);
   }
   if (stats) fill_stats(acc, a.g.ninner, ms, stats);
   return integrator_status(acc);
@@ -2853,11 +2930,16 @@ int nrg_chem_step_dev_noalloc(nrg_chem_t *h, const nrg_grid *grid, double dt, co
   float ms = 0.f;
   HIP_TRY(hipEventRecord(h->ev0, h->stream));
   hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(ACC_SLOTS), 0, h->stream, acc_dev, ACC_SLOTS);
-  if (a.g.ninner > 0) enqueue_chunks(h, a, a.g.ninner, NRG_NOALLOC_CHUNK_CELLS, rates, acc_dev, false);
+  if (a.g.ninner > 0) {
+    const unsigned long long lanes =
+        plan(h, h->seen_step, a, a.g.ninner, NRG_NOALLOC_CHUNK_CELLS, false, false, false);
+    enqueue_chunks(h, a, a.g.ninner, NRG_NOALLOC_CHUNK_CELLS, rates, acc_dev, lanes);
+  }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(h->ev1, h->stream));
   HIP_TRY(read_counters(h, acc, acc_dev, 16));
   HIP_TRY(hipEventElapsedTime(&ms, h->ev0, h->ev1));
+  note(h->seen_step, a.g, acc);
   if (stats) fill_stats(acc, a.g.ninner, ms, stats);
   return integrator_status(acc);
 #endif
@@ -3296,6 +3378,7 @@ int nrg_chem_autotune_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, const 
   auto apply = [&](const Cfg &c) {
     h->k.gather_pct = c.gather;
     h->k.refill_idle = c.refill;
+    h->refill_auto = false;
     h->form = c.form;
     h->order = c.order;
     h->jac_pct = c.jac;
@@ -3336,8 +3419,9 @@ int nrg_chem_autotune_dev(nrg_chem_t *h, const nrg_grid *grid, double dt, const 
   if ((st = trial(best, best_ms))) return st;
   auto consider = [&](Cfg c) -> int {
     double ms = 0.0;
-    const int s = trial(c, ms);
-    if (s) return s;
+    int s = NRG_CHEM_OK;
+    if (c.order == NRG_ORDER_STIFFNESS && best.order != NRG_ORDER_STIFFNESS && (s = trial(c, ms))) return s;
+    if ((s = trial(c, ms))) return s;      // (in stiffness order, with a history)
     if (ms < best_ms) {
       best_ms = ms;
       best = c;
@@ -3558,20 +3642,25 @@ int nrg_chem_surrogate_step_dev(nrg_chem_t *h, nrg_mlp_t *mlp, const nrg_surroga
       // expensive first, by the step counts this handle recorded for them
       // (an FP64 step or an earlier fallback; temperature bins when it has
       // none for this grid), and record their step counts for the next call
-      if (h->order == NRG_ORDER_STIFFNESS) {
+      const bool ordered = h->order == NRG_ORDER_STIFFNESS;
+      bool use_hist = false;
+      if (ordered) {
         if ((st = prepare_order(h, n))) return st;
-        const bool use_hist = h->hist_valid && same_grid(h->hist_grid, a.g);
+        use_hist = h->hist_valid && same_grid(h->hist_grid, a.g);
         enqueue_order(h, a, use_hist, h->sur_list, nfb);
         a.list = h->order_list;
         a.hist = h->hist;
         h->hist_valid = true;
         h->hist_grid = a.g;
       }
-      if ((st = enqueue_integrator(h, a, nfb, true))) return st;
+      const unsigned long long lanes =
+          plan(h, h->seen_fallback, a, nfb, chunk_for(h, nfb), ordered, use_hist, true);
+      if ((st = enqueue_integrator(h, a, nfb, lanes))) return st;
     }
     HIP_TRY(hipEventRecord(h->ev1, h->stream));
     HIP_TRY(read_counters(h, acc, h->dev_acc, 16));
     HIP_TRY(hipEventElapsedTime(&ms_fb, h->ev3, h->ev1));
+    if (nfb > 0) note(h->seen_fallback, a.g, acc);
   }
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
