@@ -440,6 +440,7 @@ __global__ void __launch_bounds__(256) frag_kernel(FragArgs a)
 // which spill; at 128 99 and 104), but four at width 64 (50 us, 57 with two).
 constexpr int infer_waves(int nt) { return nt >= 4 ? 2 : 4; }
 constexpr int infer_tiles(int nt) { return nt >= 4 ? 4 : 2; }
+constexpr bool infer_ahead(int nt) { return nt >= 4; }
 
 template <int NT>
 __global__ void __launch_bounds__(NT * 64) __attribute__((amdgpu_waves_per_eu(infer_waves(NT), infer_waves(NT))))
@@ -447,7 +448,11 @@ mlp_infer_kernel(InferArgs a)
 {
   constexpr bool PERM = NT == 8;
   constexpr int KB = 2 * NT, LD = 32 * NT + 8, TILES = infer_tiles(NT);
+  constexpr bool AHEAD = infer_ahead(NT);
+  constexpr int XBUF = !AHEAD ? 0 : NT == 8 ? 2 : 1, XLD = MLP_IN_PAD + 8, XV = 32 * TILES * MLP_IN_PAD / (NT * WAVE);
+  static_assert(TILES <= NT, "a tile's output layer is one wave's work");
   __shared__ __align__(16) bf16 act[2][32 * TILES][LD];
+  __shared__ __align__(16) bf16 xin[XBUF ? XBUF : 1][XBUF ? 32 * TILES : 1][XLD];
   const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
   const int r32 = l & 31, hi = l >> 5;
   const long long T = (a.n + 31) / 32;
@@ -458,9 +463,14 @@ mlp_infer_kernel(InferArgs a)
     return reinterpret_cast<const bf16x8 *>(a.W[layer])[(PERM ? mt * kbs + kb : kb * nt + mt) * WAVE + l];
   };
   bf16x8 W[KB];
+  // this wave's weights of a layer (of the output layer: its one feature tile's)
   auto weights = [&](int layer) {
+    const bool out = layer == a.layers;
+    if (out && w >= TILES) return;
+    const bf16x8 *p = reinterpret_cast<const bf16x8 *>(a.W[layer]) + (out ? 0 : PERM ? w * KB : w) * WAVE + l;
+    const int step = out || PERM ? WAVE : NT * WAVE;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) W[kb] = weight(layer, w, NT, kb, KB);
+    for (int kb = 0; kb < KB; ++kb) W[kb] = p[kb * step];
   };
   auto biases = [&](int layer, int mt) {
     f32x16 b;
@@ -478,11 +488,35 @@ mlp_infer_kernel(InferArgs a)
       *reinterpret_cast<bf16x4 *>(d + (PERM ? 16 * (q / 2) + 8 * hi + 4 * (q % 2) : 8 * q + 4 * hi)) = v;
     }
   };
+  // the input: packed in memory, or converted on its way through LDS: into its own
+  // buffer while the group before is at work, or into the second one of activations
+  auto tile_of = [&](int g) { return t0 + (t1 - t0) * g / groups; };
+  const int xr = threadIdx.x / MLP_IN_PAD, xc = threadIdx.x % MLP_IN_PAD;
+  float xv[XV];
+  auto fetch = [&](int g) {
+    const long long row0 = 32 * tile_of(g) + xr;
+#pragma unroll
+    for (int k = 0; k < XV; ++k) {
+      const long long row = row0 + k * (NT * WAVE / MLP_IN_PAD), cell = row < a.n ? row : a.n - 1;
+      xv[k] = xc < a.n_in ? a.x[cell * a.n_in + xc] : 0.0f;
+    }
+  };
+  auto place = [&](int g) {
+#pragma unroll
+    for (int k = 0; k < XV; ++k) xin[g % (XBUF ? XBUF : 1)][xr + k * (NT * WAVE / MLP_IN_PAD)][xc] = (bf16)xv[k];
+  };
+  if (AHEAD && !a.X && groups > 0) {
+    fetch(0);
+    place(0);
+    lds_barrier();
+  }
+  int first = 0;                                 // buffer of the first layer's output
   for (int g = 0; g < groups; ++g) {
-    const long long tile = t0 + (t1 - t0) * g / groups;
-    const int nt = (int)(t0 + (t1 - t0) * (g + 1) / groups - tile);
-    // the input: packed in memory, or converted into the second buffer
-    if (!a.X) {
+    const long long tile = tile_of(g);
+    const int nt = (int)(tile_of(g + 1) - tile);
+    const bool more = AHEAD && !a.X && g + 1 < groups;
+    if (more) fetch(g + 1);
+    if (!AHEAD && !a.X) {
       for (int i = threadIdx.x; i < 32 * nt * MLP_IN_PAD; i += NT * WAVE) {
         const int row = i / MLP_IN_PAD, c = i % MLP_IN_PAD;
         const long long cell = 32 * tile + row < a.n ? 32 * tile + row : a.n - 1;
@@ -491,7 +525,7 @@ mlp_infer_kernel(InferArgs a)
     }
     f32x16 bias = biases(0, w);
     const bf16x8 W0[2] = {weight(0, w, NT, 0, 2), weight(0, w, NT, 1, 2)};
-    if (!a.X) lds_barrier();
+    if (!AHEAD && !a.X) lds_barrier();
     for (int t = 0; t < nt; ++t) {
       const long long cell = 32 * (tile + t) + r32 < a.n ? 32 * (tile + t) + r32 : a.n - 1;
       bf16x8 x[2];
@@ -499,19 +533,21 @@ mlp_infer_kernel(InferArgs a)
       for (int kb = 0; kb < 2; ++kb)
         if (a.X)
           x[kb] = *reinterpret_cast<const bf16x8 *>(a.X + cell * MLP_IN_PAD + 16 * kb + 8 * hi);
+        else if (AHEAD)
+          x[kb] = *reinterpret_cast<const bf16x8 *>(&xin[g % (XBUF ? XBUF : 1)][32 * t + r32][16 * kb + 8 * hi]);
         else
           x[kb] = *reinterpret_cast<const bf16x8 *>(&act[1][32 * t + r32][16 * kb + 8 * hi]);
       f32x16 acc = PERM ? bias : f32x16{};
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) acc = mfma(W0[kb], x[kb], acc);
-      if (t == nt - 1 && a.layers > 1) weights(1);
-      store(0, t, acc, bias);
+      if (t == nt - 1) weights(1);
+      store(first, t, acc, bias);
     }
     for (int layer = 1; layer < a.layers; ++layer) {
       bias = biases(layer, w);
       lds_barrier();
       auto product = [&](int t) {
-        const bf16 *in = &act[(layer - 1) & 1][32 * t + r32][8 * hi];
+        const bf16 *in = &act[(first + layer - 1) & 1][32 * t + r32][8 * hi];
         f32x16 acc = PERM ? bias : f32x16{};
         if (NT >= 4) {                           // all loads ahead
           bf16x8 f[KB];
@@ -531,29 +567,34 @@ mlp_infer_kernel(InferArgs a)
 #pragma unroll 1
       for (int t = 1; t < nt; ++t) {
         const f32x16 next = product(t);
-        store(layer & 1, t - 1, cur, bias);
+        store((first + layer) & 1, t - 1, cur, bias);
         cur = next;
       }
-      if (layer + 1 < a.layers) weights(layer + 1);
-      store(layer & 1, nt - 1, cur, bias);
+      weights(layer + 1);
+      store((first + layer) & 1, nt - 1, cur, bias);
+    }
+    bias = biases(a.layers, 0);
+    if (more) {
+      if (XBUF == 1 && a.layers == 1) lds_barrier();   // the first layer reads it to its end
+      place(g + 1);
     }
     lds_barrier();
-#pragma unroll 1
-    for (int t = w; t < nt; t += NT) {           // output layer: a tile to a wave
-      const bf16 *in = &act[(a.layers - 1) & 1][32 * t + r32][8 * hi];
-      bias = biases(a.layers, 0);
+    if (w < nt) {                                // output layer: a tile to a wave
+      const bf16 *in = &act[(first + a.layers - 1) & 1][32 * w + r32][8 * hi];
       f32x16 o = PERM ? bias : f32x16{};
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
-        o = mfma(weight(a.layers, 0, 1, kb, KB), *reinterpret_cast<const bf16x8 *>(in + 16 * kb), o);
-      const long long cell = 32 * (tile + t) + r32;
+        o = mfma(W[kb], *reinterpret_cast<const bf16x8 *>(in + 16 * kb), o);
+      const long long cell = 32 * (tile + w) + r32;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int f = acc_row(r, hi);
         if (cell < a.n && f < a.n_out) a.Y[cell * a.n_out + f] = PERM ? o[r] : o[r] + bias[r];
       }
     }
-    lds_barrier();                               // the next tiles take the activations' place
+    // the next tiles' activations: in the buffer that nobody reads now, or in this one's place
+    if (AHEAD) first = (first + a.layers) & 1;
+    else lds_barrier();
   }
 }
 
