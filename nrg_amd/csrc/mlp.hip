@@ -363,8 +363,8 @@ __global__ void to_bf16_kernel(const float *P, bf16 *Pbf, long long n)
 // All layers in one kernel, computed transposed, Z^T = W^T H^T: the weights are the
 // MFMA A operand (32 output features x 16 inputs) and the activations the B operand
 // (16 inputs x 32 cells).  A wave owns 32 features of every hidden layer; its
-// weights of a layer (up to 16 KB) come from L2 into registers and serve the two
-// 32-cell tiles that a block works on, whose activations pass through LDS.  A
+// weights of a layer (up to 16 KB) come from L2 into registers and serve the two or
+// four 32-cell tiles that a block works on, whose activations pass through LDS.  A
 // lane's accumulator holds, for its cell, features 32 w + 8 q + 4 hi + i (q, i =
 // 0..3, hi = lane/32): four stores of four.  Width 256 keeps a k-block's inputs in
 // the order (8 hi + 4 (q%2) + i of block q/2) that its K rows have in WswT, and the
@@ -375,9 +375,21 @@ __global__ void to_bf16_kernel(const float *P, bf16 *Pbf, long long n)
 // loads.  The blocks share the tiles evenly.  Before, a wave took its cells through
 // all features with the weights staged in LDS (at the narrower widths the
 // activations): few cells left most of the chip idle for a long chain, and 70,001
-// cells were a second, nearly empty round.  Call times, width 256 x 4: 256 cells 56
-// -> 29 us, 16,384 58 -> 35, 70,001 91 -> 61, 262,144 197 -> 187; 128 x 4: 4096 39 ->
-// 26, 262,144 130 -> 99; 64 x 3: 4096 31 -> 25, 262,144 72 -> 50.
+// cells were a second, nearly empty round.
+//
+// At widths 128 and 256 nothing of a group of tiles waits for memory: the group's
+// input is fetched while the one before goes through its layers and lies in its own
+// LDS, the output layer's weights and bias come with the last GELUs, and the waves
+// without an output tile go on with the next group, whose first layer writes the
+// buffer that the output layer does not read (one barrier a layer).  Without that the
+// ends of a group cost more than a layer: 256 x 1, 1,000,000 cells, 227 us with the
+// loads where they are used, 169 with a wave per 32 cells, 140 so.
+//
+// Call times in turn (a wave per 32 cells -> loads where they are used -> this), width
+// 256 x 4: 1000 cells 48 -> 22 -> 21 us, 16,384 49 -> 27 -> 26, 70,001 88 -> 62 -> 58,
+// 262,144 180 -> 172 -> 157, 4,000,000 2401 -> 2388 -> 2095; 256 x 2, 1,000,000: 313 ->
+// 340 -> 257; 128 x 1, 1,000,000: 144 -> 159 -> 93; 128 x 4, 262,144: 111 -> 89 -> 79;
+// 64 x 4, 262,144: 71 -> 50 -> 49.
 struct InferArgs {
   const bf16 *X;               // n x 32, or NULL:
   const float *x;              // n x n_in
@@ -436,8 +448,10 @@ __global__ void __launch_bounds__(256) frag_kernel(FragArgs a)
 
 // Resident waves per SIMD, and the 32-cell tiles a block takes through the layers
 // together: two waves with up to 256 registers (a tile's fragments and a layer's
-// weights in flight at once; 262,144 cells at width 256 186 us, 298 with four waves,
-// which spill; at 128 99 and 104), but four at width 64 (50 us, 57 with two).
+// weights in flight at once; before the inputs were fetched ahead 262,144 cells at
+// width 256 took 186 us, 298 with four waves, which spill; at 128 99 and 104), but four
+// at width 64 (50 us, 57 with two), where the blocks' LDS leaves no room for an input
+// buffer of their own and the SIMD's other waves cover the loads.
 constexpr int infer_waves(int nt) { return nt >= 4 ? 2 : 4; }
 constexpr int infer_tiles(int nt) { return nt >= 4 ? 4 : 2; }
 constexpr bool infer_ahead(int nt) { return nt >= 4; }
