@@ -2094,9 +2094,10 @@ struct Seen {
   unsigned long long lanes = 0;
 };
 
-// Pinned memory for the host-pointer entry points' fields, at most (137,000 cells of
-// KEROMNES); a handle holds what its largest call up to that has needed.
-constexpr size_t STAGE_PINNED_MAX = 32u << 20;
+// Pinned memory for the host-pointer entry points' fields, at most (102,000 cells of
+// KEROMNES); a handle holds what its largest call up to that has needed, and grows it
+// by half at least, as pinning takes ~0.3 ms a MiB.
+constexpr size_t STAGE_PINNED_MAX = 24u << 20;
 
 struct nrg_chem_handle {
   int device = 0;
@@ -2973,17 +2974,20 @@ static int step_host(nrg_chem_t *h, bool table, const nrg_grid *grid, double dt,
     h->stage_bytes = in_bytes + out_bytes;
   }
   // Small fields go through pinned memory, all in one copy each way: a copy from
-  // pageable memory returns only when it is done (~10 us each, 51 of them).  Calls of
-  // flame cells: 60 cells 980 -> 600 us, 9100 1580 -> 1100, 30,000 2080 -> 1640, 80,000
-  // 3860 -> 3740, 136,000 the same: from there the copies of single fields overlap.
+  // pageable memory returns only when it is done (~10 us each, 51 of them).  Field by
+  // field and in one copy, flame steps, table steps: 10,000 cells 1030 and 605 us, 650 and
+  // 220; 30,000 1400 and 1040, 850 and 495; 65,000 2190 and 1960, 1230 and 1030; 100,000
+  // 3000 and 2990, 1650 and 1650; 120,000 3430 and 3590, 1870 and 2020: by then the host's
+  // own copies are as long as the transfers, which single fields' copies run beside.
   bool pin = in_bytes + out_bytes <= STAGE_PINNED_MAX;
   if (pin && h->pinned_bytes < in_bytes + out_bytes) {
+    const size_t grown = std::max(in_bytes + out_bytes, std::min(h->pinned_bytes / 2 * 3, STAGE_PINNED_MAX));
     void *old = h->pinned;
     h->pinned = nullptr;
     h->pinned_bytes = 0;
     if (old) HIP_TRY(hipHostFree(old));
-    if (hipHostMalloc(&h->pinned, in_bytes + out_bytes, hipHostMallocDefault) == hipSuccess) {
-      h->pinned_bytes = in_bytes + out_bytes;
+    if (hipHostMalloc(&h->pinned, grown, hipHostMallocDefault) == hipSuccess) {
+      h->pinned_bytes = grown;
     } else {
       (void)hipGetLastError();   // no pinned memory to be had: field by field
       h->pinned = nullptr;

@@ -96,3 +96,10 @@ def test_pinned_memory_is_what_the_call_needs(fake, n, most):
     assert got["host_step"] == 0
     assert 0 < got["host_bytes"] <= most
     assert got["host_bytes_left"] == 0
+
+
+def test_large_fields_are_not_pinned(fake):
+    """120,000 cells: single fields' copies are the faster way there (the counters' 128 bytes stay)."""
+    got = _run(fake, "host_step", n=120000)
+    assert got["host_step"] == 0
+    assert got["host_bytes"] <= 4096
