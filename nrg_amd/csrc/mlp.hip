@@ -728,9 +728,10 @@ int loss_and_grad(nrg_mlp_t *h, long long n, const float *x, const float *t, con
   if (rc) return rc;
   if ((rc = refresh_frags(h, false))) return rc;
   // 16 rows to a block up to two blocks per CU, where a block's latency counts
-  // (256 x 4: 4096 rows 73 us, 77 with 32; 128 x 4: 8192 rows 64, 68); above, the
-  // MFMAs' second half is worth having (256 x 4: 16384 rows 134, 141; 65536 378, 412).
-  // (64 rows, two tiles sharing each weight fragment: within 2 % of 32.)
+  // (256 x 4: 4096 rows 50 us, 54 with 32; 128 x 4: 8192 rows 40, 44; 64 x 3: 4096 rows
+  // 28, 31); above, the MFMAs' second half is worth having (256 x 4: 16384 rows 102, 109
+  // with 16; 65536 340, 379; 128 x 4: 65536 157, 163; at 16384 the narrower widths are
+  // 3 to 4 us faster with 16).
   const int rows = n <= 32ll * h->num_cu ? 16 : 32;
   const long long row_blocks = (n + rows - 1) / rows;
   TrainArgs a{};
@@ -770,8 +771,8 @@ int loss_and_grad(nrg_mlp_t *h, long long n, const float *x, const float *t, con
   g.layers = h->layers + 1;
   g.kblocks = row_blocks * (rows / 16);
   // Ranges of the rows: at least 512 rows each, and no more than fill the chip,
-  // since every range adds its sums to G (256 x 4, 16384 rows: 32 ranges 134 us, 8
-  // of them 122).
+  // since every range adds its sums to G (256 x 4, 16384 rows: 103 us, 113 with all 32
+  // ranges; 65536: 340, 371).
   const long long ksplit = std::max<long long>(1, std::min<long long>(n / 512, 2 * h->num_cu / blocks));
   g.kper = (g.kblocks + ksplit - 1) / ksplit;
   g.loss_part = h->loss_part; g.n_part = row_blocks; g.loss = loss;

@@ -1157,7 +1157,7 @@ __global__ void __launch_bounds__(LM_THREADS) low_mach_div_kernel(LowMachDivArgs
 // hot kernels: 65 % of the lanes busy per instruction by steps alone, 71 % so).  One cell
 // per lane, by steps / 16 / 64 bins of each: 2.1M cells with hot kernels 4.85 / 3.73 /
 // 3.69 ms, 1M flame cells 14.6 / 12.2 / 11.9, 1M igniting 17.3 / 15.7 / 14.9.  (By a hash
-// of the path instead: 3.73, 11.4, 16.0.)  Placing 16.7M cells costs 0.34 ms, 0.10 before.
+// of the path instead: 3.73, 11.4, 16.0.)  Placing 16.7M cells costs 0.26 ms, 0.10 with 64 bins.
 constexpr int NBIN_STEP = 64, NBIN_FE = 64;
 constexpr int NBIN = NBIN_STEP * NBIN_FE;
 constexpr int BIN_THREADS = 256;
@@ -1216,7 +1216,9 @@ __global__ void __launch_bounds__(BIN_THREADS) bin_count_kernel(BinArgs a)
 
 // Each block claims its bins' slots with one atomic per bin, behind the cells of
 // the more expensive bins, then places its run's cells (same run as
-// bin_count_kernel, binned again).
+// bin_count_kernel, binned again).  A thread has 16 bins: one claim after the other, each
+// waited for, took 54 us of a list of 84,000 cells (12 now), 194 of 545,400 igniting
+// cells (33) and 326 of 16.7M with hot kernels (261).
 __global__ void __launch_bounds__(BIN_THREADS) bin_scatter_kernel(BinArgs a)
 {
   __shared__ unsigned int h[NBIN];
@@ -1226,8 +1228,18 @@ __global__ void __launch_bounds__(BIN_THREADS) bin_scatter_kernel(BinArgs a)
   constexpr int PER = NBIN / BIN_THREADS;
   static_assert(NBIN % BIN_THREADS == 0, "bins to a thread");
   const int b0 = threadIdx.x * PER, lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-  unsigned long long mine = 0;
-  for (int b = b0; b < b0 + PER; ++b) mine += a.count[b];
+  unsigned long long cells[PER], claim[PER], mine = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) cells[k] = a.count[b0 + k];
+  // the claims, all under way before the first is waited for (neighbouring threads take
+  // neighbouring bins: those that a run fills lie together)
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int b = k * BIN_THREADS + threadIdx.x;
+    claim[k] = h[b] ? atomicAdd(&a.cursor[b], (unsigned long long)h[b]) : 0ull;
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) mine += cells[k];
   unsigned long long after = mine;
   for (int d = 1; d < WAVE; d <<= 1) {
     const unsigned long long v = __shfl_down(after, d, WAVE);
@@ -1237,9 +1249,16 @@ __global__ void __launch_bounds__(BIN_THREADS) bin_scatter_kernel(BinArgs a)
   __syncthreads();
   for (int k = w + 1; k < BIN_THREADS / WAVE; ++k) after += sums[k];
   after -= mine;
-  for (int b = b0 + PER - 1; b >= b0; --b) {
-    base[b] = after + (h[b] ? atomicAdd(&a.cursor[b], (unsigned long long)h[b]) : 0ull);
-    after += a.count[b];
+#pragma unroll
+  for (int k = PER - 1; k >= 0; --k) {
+    base[b0 + k] = after;
+    after += cells[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int b = k * BIN_THREADS + threadIdx.x;
+    base[b] += claim[k];
     h[b] = 0u;
   }
   __syncthreads();
@@ -2545,8 +2564,8 @@ static void enqueue_order(nrg_chem_t *h, StepArgs &a, bool use_hist, const int32
   b.list = h->order_list;
   b.in_list = in_list;
   b.npos = n;
-  // runs as long as still give every CU four blocks (84,000 listed cells: 55 + 50 us
-  // with 32 cells a thread and an offsets kernel of 8, 9 + 9 with one)
+  // runs as long as still give every CU four blocks (84,000 listed cells: 9 + 12 us with
+  // one cell a thread; with 32, in an earlier form of both kernels, 55 + 50)
   b.run = (int)std::min<long long>(BIN_RUN_MAX, std::max<long long>(1, n / (4ll * h->num_cu * BIN_THREADS)));
   const unsigned nb = (unsigned)((n + b.run * BIN_THREADS - 1) / (b.run * BIN_THREADS));
   hipLaunchKernelGGL(reset_kernel, dim3(2 * NBIN / 256), dim3(256), 0, h->stream, h->bins, 2 * NBIN);
