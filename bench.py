@@ -18,7 +18,7 @@ legs run from the same initial state: the learned step and the method without
 the network (their FP64 fallback integrating at eps 1e-6 with the analytic
 Jacobian, on a handle of its own, and again at the reference's eps 1e-9 with
 the FD Jacobian), the table-approximated mode, the low-Mach coupling kernels,
-and the uneven-stiffness field (persistent queue vs one cell per lane at
+and the uneven-stiffness field (stiffness order in a graph vs natural order at
 three dt).
 """
 import argparse
@@ -52,7 +52,7 @@ def parse():
                     help="0: every core this process may run on, at most 16 (one GPU's share "
                          "of the host)")
     ap.add_argument("--form", choices=["plain", "persistent"], default="persistent",
-                    help="integrator launch form (same results)")
+                    help="accepted for the library's option; both forms run the same kernels")
     ap.add_argument("--jacobian", choices=["fd", "analytic"], default="fd",
                     help="fd: SLATEC finite differences (reference parity); analytic: fast mode")
     ap.add_argument("--order", choices=["natural", "stiffness"], default="stiffness",
@@ -67,7 +67,7 @@ def parse():
     ap.add_argument("--gather-pct", type=int, default=0,
                     help="error-test gathering threshold in percent of stepping lanes (same results)")
     ap.add_argument("--refill-idle", type=int, default=0,
-                    help="persistent form: idle lanes of 64 that trigger a refill (0: default 63; "
+                    help="idle lanes of 64 that trigger a refill (0: the library's choice; "
                          "same results)")
     ap.add_argument("--surrogate", default="auto",
                     help="trained surrogate (.npz) timed beside the FP64 integrator from the same "
@@ -100,8 +100,8 @@ def parse():
                     help="time the low-Mach coupling kernels on the FP64 run's outputs (0: skip)")
     ap.add_argument("--uneven", type=int, default=1,
                     help="time the uneven-stiffness 256^3 field (5%% of cells in the 1000-1300 K "
-                         "ignition window) at dt 1e-8, 1e-7, 1e-6 s: persistent graph queue vs "
-                         "one cell per lane (0: skip)")
+                         "ignition window) at dt 1e-8, 1e-7, 1e-6 s: stiffness order in a graph vs "
+                         "natural order (0: skip)")
     ap.add_argument("--table-line", type=int, default=512,
                     help="cells of the flame line the table is written from")
     ap.add_argument("--copy-calibration-mib", type=int, default=0,
@@ -114,12 +114,11 @@ def effective_setup(args, tuning):
     """Queue set-up the timed steps ran with: the autotuner's choice when it ran."""
     from nrg_amd import capi
     if tuning is None:
-        return {"form": args.form, "order": args.order, "jac_batch_pct": args.jac_pct or 50,
-                "errtest_gather_pct": args.gather_pct, "refill_min_idle": args.refill_idle or 63,
+        return {"order": args.order, "jac_batch_pct": args.jac_pct or 50,
+                "errtest_gather_pct": args.gather_pct, "refill_min_idle": args.refill_idle or (63 if args.order == "stiffness" else 32),
                 "chunk_log2": args.chunk_log2 or 23}
     b = tuning["best"]
-    return {"form": "persistent" if b["form"] == capi.NRG_FORM_PERSISTENT else "plain",
-            "order": "stiffness" if b["cell_order"] == capi.NRG_ORDER_STIFFNESS else "natural",
+    return {"order": "stiffness" if b["cell_order"] == capi.NRG_ORDER_STIFFNESS else "natural",
             "jac_batch_pct": b["jac_batch_pct"], "errtest_gather_pct": b["errtest_gather_pct"],
             "refill_min_idle": b["refill_min_idle"],
             "chunk_log2": int(b["chunk_cells"]).bit_length() - 1}
@@ -129,8 +128,8 @@ def main():
     args = parse()
     world = int(os.environ.get("WORLD_SIZE", "1"))
     if args.gpus != 1 or world != 1:
-        print("bench.py: this build measures one GPU only (the chemistry step is cell-local; "
-              "see DESIGN.md for how it shards); run with --gpus 1", file=sys.stderr)
+        print("bench.py: one GPU only (the chemistry step is cell-local and needs no collective); "
+              "run with --gpus 1", file=sys.stderr)
         sys.exit(2)
 
     import numpy as np
@@ -320,7 +319,7 @@ def main():
     # ---- table-approximated mode from the same initial state -----------------------------
     tab = table_leg(args, mech, dm, solver, fields0, Y0, T_ref, Y_ref, value, S) if args.table else None
 
-    # ---- uneven stiffness: persistent graph queue vs one cell per lane --------------------
+    # ---- uneven stiffness: stiffness order in a graph vs natural order ---------------------
     uneven = None
     if args.uneven:
         del fields0, Y0, T_ref, Y_ref
@@ -528,12 +527,12 @@ def audit_against(dm, T_ref, Y_ref, S, steps):
 
 # algorithmic bytes per inner cell of the low-Mach coupling kernels as bench.py
 # calls them (no markers set, three velocity components, all optional outputs):
-# EOS predictor reads rho, 9 Y, dp_stat_dt, p_stat, 3 v, marker (121 B) and writes
-# 11 fields (88 B); the species predictor with the chemistry source reads rho,
+# EOS predictor reads rho, 9 Y, dp_stat_dt, p_stat, the last v, marker (105 B) and
+# writes 11 fields (88 B); the species predictor with the chemistry source reads rho,
 # 9 Y, 9 Y_prod, marker (153 B) and writes rho_int, 9 Y_int (80 B); the reactive
 # divergence reads rho, T, 9 Y, W_mix, E_f_prod, 9 Y_prod, marker (177 B) and
 # writes div_v (8 B)
-LOW_MACH_BYTES = {"low_mach_eos_kernel": 121 + 88, "low_mach_species_kernel": 153 + 80,
+LOW_MACH_BYTES = {"low_mach_eos_kernel": 105 + 88, "low_mach_species_kernel": 153 + 80,
                   "low_mach_div_kernel": 177 + 8}
 
 
@@ -594,10 +593,11 @@ def low_mach_leg(args, dm, solver, S, reps=10):
 def uneven_leg(args, mech, tuning, dts=(1e-8, 1e-7, 1e-6), reps=2):
     """The uneven-stiffness workload: n^3 cells, 5 % of them fresh mixture in the
     1000-1300 K ignition window (tens to hundreds of steps each), the rest burnt
-    or cold (a few steps).  For each dt, the chemistry step (rates_kernel +
-    chem_bdf_kernel, device time from HIP events) in two set-ups from the
-    same state: stiffness order in a HIP graph with the main leg's autotuned queue
-    set-up (a cell to a lane), and natural order (a cell to a group of lanes).  Both give the same outputs bit for bit (checked here)."""
+    or cold (a few steps).  For each dt, the chemistry step (rates_kernel + the
+    integrator that the library takes, device time from HIP events) in two set-ups
+    from the same state: stiffness order in a HIP graph with the main leg's autotuned
+    queue set-up, and natural order.  Both give the same outputs bit for bit
+    (checked here)."""
     import numpy as np
     import torch
 

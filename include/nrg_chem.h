@@ -296,11 +296,11 @@ int nrg_energy_from_temperature_dev(nrg_chem_t *h, const nrg_grid *grid,
 /*
  * Autotuner of the batched form.  A workgroup is one wave, whose lanes or lane
  * groups hold the cells, so what is tuned is how the queue feeds the waves: cell
- * order, the error-test gathering, the batched-Jacobian threshold,
- * the refill threshold, resident waves per CU and the queue chunk size.  Starting from the handle's current set-up it tries
- * one change at a time (greedy), each as a full chemistry step on the given
- * fields timed with HIP events, keeps the fastest and leaves it in the
- * handle.  Every trial writes the step's outputs (identical for every set-up).
+ * order, the error-test gathering, the batched-Jacobian threshold, the refill
+ * threshold, resident waves per CU and the queue chunk size.  Starting from the
+ * handle's current set-up it tries one change at a time (greedy), each as a full
+ * chemistry step on the given fields timed with HIP events, keeps the fastest and
+ * leaves it in the handle.  Every trial writes the step's outputs (identical for every set-up).
  * Arguments as nrg_chem_step_dev; `out` receives the trials and the choice.
  */
 #define NRG_TUNE_MAX_TRIALS 24

@@ -19,11 +19,11 @@
 // igniting mixture: the scalar work of a step, its divisions, powers and
 // ordered sums, is done in all G lanes alike); a small grid is bound by the
 // way of one cell through its steps.  Against one cell per lane (bdf_lane.h),
-// kernel time in stiffness order: 65,536 KEROMNES flame cells 2.15 -> 1.50 ms,
-// 262,144 cells with hot kernels 2.58 -> 1.15, 84,000 igniting ones 3.66 ->
-// 2.10, 65,536 KONNOV flame cells (13 species) 83 -> 10.9; one cell per lane
-// stays ahead where it fills the chip several times over (1M flame cells: 14.6
-// ms, 17.4 here).
+// kernel time in stiffness order: 65,536 KEROMNES flame cells 2.03 -> 1.45 ms,
+// 262,144 cells with hot kernels 2.71 -> 1.15, 65,536 igniting ones 3.57 ->
+// 1.66, 65,536 KONNOV flame cells (13 species) 83 -> 10.9; one cell per lane
+// stays ahead where cells that cost alike fill the chip (1M flame cells: 11.9
+// ms, 14.8 here).
 //
 // Also measured: two species to a lane (4 lanes per cell, 233 registers, two
 // waves per SIMD): 26 % fewer VALU instructions, but latency-bound; 8 % faster

@@ -1,4 +1,5 @@
-// bdf_lane.h -- the integrator of large grids: one cell per lane.
+// bdf_lane.h -- one cell per lane: the integrator where cells that cost alike fill
+// the chip.
 //
 // A cell's Gear-BDF state (Nordsieck history, iteration matrix, work vectors)
 // lives in VGPRs/AGPRs; its 2R rate constants live in a per-lane LDS slot.
@@ -20,8 +21,8 @@
 // wave pass a stage.  Cells of equal cost, which stiffness order brings
 // together, keep that share small; 65,536 cells fill the chip once.  The norm has
 // one path for ordinary vectors instead of the walk through its phases.  Kernel
-// time in stiffness order with a history: 1M flame cells 12.0 ms, 2.1M cells with
-// hot kernels 3.8, 1M igniting ones 15.1.
+// time in stiffness order with a history: 1M flame cells 11.9 ms, 2.1M cells with
+// hot kernels 3.7, 1M igniting ones 15.0.
 //
 // Reference: computing_module/src/current_build/chemical_kinetics_solver.f90
 // (RHS :495-540, cell step :228-346) and SLATEC SDRIVE in

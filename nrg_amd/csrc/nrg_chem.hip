@@ -458,7 +458,8 @@ NRG_DI void flush_tally(unsigned long long *acc, const unsigned long long *tally
 // with 32, 26.0 with 8); in natural order a long cell would keep the others'
 // lanes idle (262,144 cells of an igniting mixture: 12.1 ms with 64, 9.0 with
 // 32, 8.0 with 8, but flame fronts and hot kernels want more: 22.0, 23.5, 24.2
-// and 6.7, 6.4, 9.1).
+// and 6.7, 6.4, 9.1), except where the last call has counted that the grid's cells
+// cost alike (plan): they are started together as well.
 constexpr int REFILL_IDLE_ORDERED = 63, REFILL_IDLE_NATURAL = 32;
 
 // Resident waves per SIMD the register budget is sized for (168 registers at
@@ -537,8 +538,8 @@ extern template __global__ void chem_bdf_kernel<true>(StepArgs);
 #endif
 
 // ---------------------------------------------------------------------------
-// The same step with one cell per lane (bdf_lane.h), for large grids of the
-// topologies whose state fits the register file.
+// The same step with one cell per lane (bdf_lane.h), where a launch's cells fill the
+// chip so (lane_launch), for the topologies whose state fits the register file.
 // ---------------------------------------------------------------------------
 constexpr bool LANE_KERNEL = SA <= 10;
 constexpr int LANE_WAVES_PER_CU = 4;   // one to a SIMD: it takes the whole register file
@@ -2573,9 +2574,7 @@ static void enqueue_order(nrg_chem_t *h, StepArgs &a, bool use_hist, const int32
   hipLaunchKernelGGL(bin_scatter_kernel, dim3(nb), dim3(BIN_THREADS), 0, h->stream, b);
 }
 
-// Enqueue rates_kernel + chem_bdf_kernel over npos queue positions (all inner
-// cells when a.list is NULL, else the cells a.list names), in chunks of at
-// most chunk_max positions, each with its own queue head.
+// Positions to a chunk: at most chunk_max, each chunk with its own queue head.
 static long long chunk_for(const nrg_chem_t *h, long long npos)
 {
   long long chunk = std::min<long long>(npos, h->chunk_max);
